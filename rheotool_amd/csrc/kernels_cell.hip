@@ -579,17 +579,26 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(3, 8))
     double q[19];
 #pragma unroll
     for (int i = 0; i < 19; ++i) q[i] = qs[i][threadIdx.x];
-    write_partials<19>(q, a.partials);
+    __syncthreads();
+    write_partials<19>(q, a.partials, blk_of_launch(&qs[0][0]));
 }
 
-__global__ void __launch_bounds__(BLK) k_fin_assemble(AssembleArgs a, int G) {
-    double sums[19];
-    sum_partials<19>(a.partials, G, sums);
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < 6; ++c)
-            if (a.valid[c] > 0) finish_initial(a.cs[c], a.ctl, sums[c], sums[6 + c], sums[12 + c]);
-        *a.nnzOut = sums[18];
+__global__ void __launch_bounds__(FBLK) k_fin_assemble(AssembleArgs a, int G) {
+    __shared__ double lds[FIN_LDS];
+    const int c = threadIdx.x;
+    bool on = false;
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+        if (i == c) on = a.valid[i] > 0;
+    CompState cs;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<19>(a.partials, G, lds, sums);
+    if (on) {
+        finish_initial(cs, a.ctl, sums[c], sums[6 + c], sums[12 + c]);
+        a.cs[c] = cs;
     }
+    if (c == 6) *a.nnzOut = sums[18];
 }
 
 // ----------------------------------------------------------- calcEig + tau
@@ -1401,7 +1410,7 @@ void launch_assemble(Ctx* ctx, const AssembleArgs& a, int grid) {
         ProfScope ps(ctx, a.mixed ? "k_assemble<f32>" : "k_assemble<f64>", by);
         g = a.mixed ? launch_assemble_kind<float>(ctx, a, grid) : launch_assemble_kind<double>(ctx, a, grid);
     }
-    hipLaunchKernelGGL(k_fin_assemble, dim3(1), dim3(BLK), 0, ctx->stream, a, g);
+    hipLaunchKernelGGL(k_fin_assemble, dim3(1), dim3(FBLK), 0, ctx->stream, a, g);
     RT_HIP(hipGetLastError());
 }
 void launch_eig_tau(Ctx* ctx, int32_t N, const ModelParams& prm, const double* theta,

@@ -80,7 +80,7 @@ __device__ __forceinline__ bool inner_running(const KryArgs<T>& a) {
 }
 
 template <class T, int MODE>
-__device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& k_) {
     constexpr int NQ = 18;
     bool on[6];
     bool any = false;
@@ -100,13 +100,13 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, int gG, int
     // (the first colour's residual is zero once it has been eliminated)
     const int64_t nRows = (int64_t)a.N - a.rowBegin;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = a.rowBegin > 0 ? tile_of_g(it, nRows, 0, gG, gB) : tile_of_g(it, a.N, a.nRed, gG, gB);
+        const int64_t tl = a.rowBegin > 0 ? tile_of_g(it, nRows, 0, k_.G, k_.b) : tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
         const int64_t t0 = tl * BLK;
-        const int32_t r = (int32_t)(a.rowBegin + t0 + threadIdx.x);
+        const int32_t r = (int32_t)(a.rowBegin + t0 + k_.tid);
         if (r >= a.N) continue;
         const double d = a.diag[r];
         double y[6], xv[6];
@@ -155,59 +155,64 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, int gG, int
         st6(a.r + (int64_t)NCMP * r, rt);
         st6(a.r0 + (int64_t)NCMP * r, rt);
     }
-    write_partials<NQ>(q, a.partials, gB);
+    write_partials<NQ>(q, a.partials, k_);
 }
 
 template <class T, int MODE>
 __global__ void __launch_bounds__(BLK) k_residual(KryArgs<T> a) {
-    k_residual_body<T, MODE>(a, gridDim.x, blockIdx.x);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_residual_body<T, MODE>(a, blk_of_launch(red));
 }
 
+// The finalize bodies: every thread of the workgroup sums the partials, then
+// lane c of the first wavefront updates component c's record.  (Thread 0
+// updating the six records one after another, with a memory round trip for
+// each, was most of these kernels' time.)
 template <class T, int MODE>
-__device__ __forceinline__ void k_fin_residual_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_fin_residual_body(const KryArgs<T>& a, double* lds) {
     constexpr int NQ = 18;
-    bool on[6];
-    bool any = false;
+    bool on = false, any = false;
+    const int c = threadIdx.x;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.valid[c] > 0 && (MODE == 0 || a.cs[c].needRefine);
-        any |= on[c];
+    for (int i = 0; i < 6; ++i) {
+        const bool o = a.valid[i] > 0 && (MODE == 0 || a.cs[i].needRefine);
+        any |= o;
+        if (i == c) on = o;
     }
     if (!any || (MODE == 1 && inner_running(a))) return;
-    double sums[NQ];
-    sum_partials<NQ>(a.partials, a.G, sums);
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
-            CompState& cs = a.cs[c];
-            if (MODE == 0) {
-                finish_initial(cs, a.ctl, sums[c], sums[6 + c], sums[12 + c]);
-            } else {
-                cs.needRefine = 0;
-                cs.foldE = 0;
-                cs.nRefine += 1;
-                cs.finalRes = sums[c] / cs.normFactor;
-                if (conv_outer(cs, a.ctl, cs.finalRes) && cs.iter >= a.ctl.minIter) {
-                    cs.converged = 1;
-                    cs.active = 0;
-                } else if (cs.nRefine >= a.ctl.maxRefine || cs.iter >= a.ctl.maxIter) {
-                    cs.active = 0;
-                } else {
-                    start_inner(cs, a.ctl, a.ctl.bicg ? sums[12 + c] : sums[6 + c]);
-                }
-            }
+    CompState cs;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<NQ>(a.partials, a.G, lds, sums);
+    if (!on) return;
+    if (MODE == 0) {
+        finish_initial(cs, a.ctl, sums[c], sums[6 + c], sums[12 + c]);
+    } else {
+        cs.needRefine = 0;
+        cs.foldE = 0;
+        cs.nRefine += 1;
+        cs.finalRes = sums[c] / cs.normFactor;
+        if (conv_outer(cs, a.ctl, cs.finalRes) && cs.iter >= a.ctl.minIter) {
+            cs.converged = 1;
+            cs.active = 0;
+        } else if (cs.nRefine >= a.ctl.maxRefine || cs.iter >= a.ctl.maxIter) {
+            cs.active = 0;
+        } else {
+            start_inner(cs, a.ctl, a.ctl.bicg ? sums[12 + c] : sums[6 + c]);
         }
     }
+    a.cs[c] = cs;
 }
 
 template <class T, int MODE>
-__global__ void __launch_bounds__(BLK) k_fin_residual(KryArgs<T> a) {
-    k_fin_residual_body<T, MODE>(a, gridDim.x, blockIdx.x);
+__global__ void __launch_bounds__(FBLK) k_fin_residual(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_residual_body<T, MODE>(a, lds);
 }
 
 // ---- p = r  |  p = r + beta (p - omega v) ---------------------------------
 template <class T>
-__device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     bool first[6];
     T beta[6], omega[6];
@@ -226,14 +231,14 @@ __device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, int gG, int gB
     if (!update) {
         // every active component starts an inner solve: p = r.  The other
         // components' p is dead until their own restart sets it.
-        for (int64_t i = (int64_t)gB * BLK + threadIdx.x; i < N; i += (int64_t)gG * BLK) {
+        for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
             T rr[6];
             ld6(a.r + NCMP * i, rr);
             st6(a.p + NCMP * i, rr);
         }
         return;
     }
-    for (int64_t i = (int64_t)gB * BLK + threadIdx.x; i < N; i += (int64_t)gG * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
         T rr[6], pp[6], vv[6];
         ld6(a.r + NCMP * i, rr);
         ld6(a.p + NCMP * i, pp);
@@ -247,12 +252,12 @@ __device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, int gG, int gB
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_kry_p(KryArgs<T> a) {
-    k_kry_p_body<T>(a, gridDim.x, blockIdx.x);
+    k_kry_p_body<T>(a, blk_of_launch(nullptr));
 }
 
 // ---- v = A M^-1 p = p + Ahat p ;  sigma = (r0, v) -------------------------
 template <class T>
-__device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     bool any = false;
 #pragma unroll
@@ -263,13 +268,13 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, int gG, int gB
     if (!any) return;
     T q[6] = {0, 0, 0, 0, 0, 0};
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, a.N, a.nRed, gG, gB);
+        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
         const int64_t t0 = tl * BLK;
-        const int32_t r = (int32_t)(t0 + threadIdx.x);
+        const int32_t r = (int32_t)(t0 + k_.tid);
         if (r >= a.N) continue;
         T acc[6];
         ld6(a.p + (int64_t)NCMP * r, acc);
@@ -303,39 +308,41 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, int gG, int gB
     double qd[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) qd[c] = q[c];
-    write_partials<6>(qd, a.partials, gB);
+    write_partials<6>(qd, a.partials, k_);
 }
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_kry_v(KryArgs<T> a) {
-    k_kry_v_body<T>(a, gridDim.x, blockIdx.x);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_kry_v_body<T>(a, blk_of_launch(red));
 }
 
 template <class T>
-__device__ __forceinline__ void k_fin_v_body(const KryArgs<T>& a, int gG, int gB) {
-    bool on[6];
+__device__ __forceinline__ void k_fin_v_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
+    for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
-    double sums[6];
-    sum_partials<6>(a.partials, a.G, sums);
-    if (threadIdx.x == 0)
-        for (int c = 0; c < 6; ++c)
-            if (on[c]) a.cs[c].alpha = a.cs[c].rho / sums[c];
+    const int c = threadIdx.x;
+    CompState cs;
+    cs.active = 0;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<6>(a.partials, a.G, lds, sums);
+    if (!cs.active) return;
+    cs.alpha = cs.rho / sums[c];
+    a.cs[c] = cs;
 }
 
 template <class T>
-__global__ void __launch_bounds__(BLK) k_fin_v(KryArgs<T> a) {
-    k_fin_v_body<T>(a, gridDim.x, blockIdx.x);
+__global__ void __launch_bounds__(FBLK) k_fin_v(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_v_body<T>(a, lds);
 }
 
 // ---- s = r - alpha v ; t = A M^-1 s ; |s|, (t,s), (t,t) --------------------
 template <class T>
-__device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     T alpha[6];
     bool any = false;
@@ -350,13 +357,13 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, int gG, int gB
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, a.N, a.nRed, gG, gB);
+        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
         const int64_t t0 = tl * BLK;
-        const int32_t r = (int32_t)(t0 + threadIdx.x);
+        const int32_t r = (int32_t)(t0 + k_.tid);
         if (r >= a.N) continue;
         T sv[6], acc[6], rr[6], vv[6];
         ld6(a.r + (int64_t)NCMP * r, rr);
@@ -395,49 +402,47 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, int gG, int gB
     double qd[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) qd[i] = q[i];
-    write_partials<18>(qd, a.partials, gB);
+    write_partials<18>(qd, a.partials, k_);
 }
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_kry_t(KryArgs<T> a) {
-    k_kry_t_body<T>(a, gridDim.x, blockIdx.x);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_kry_t_body<T>(a, blk_of_launch(red));
 }
 
 template <class T>
-__device__ __forceinline__ void k_fin_t_body(const KryArgs<T>& a, int gG, int gB) {
-    bool on[6];
+__device__ __forceinline__ void k_fin_t_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
+    for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
-    double sums[18];
-    sum_partials<18>(a.partials, a.G, sums);
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
-            CompState& cs = a.cs[c];
-            const double res = sums[c] / cs.normFactor;
-            if (!a.ctl.mixed) cs.finalRes = res;
-            if (conv_inner(cs, a.ctl, res)) {
-                cs.exitAtS = 1;
-            } else {
-                cs.omega = sums[6 + c] / sums[12 + c];
-            }
-        }
+    const int c = threadIdx.x;
+    CompState cs;
+    cs.active = 0;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<18>(a.partials, a.G, lds, sums);
+    if (!cs.active) return;
+    const double res = sums[c] / cs.normFactor;
+    if (!a.ctl.mixed) cs.finalRes = res;
+    if (conv_inner(cs, a.ctl, res)) {
+        cs.exitAtS = 1;
+    } else {
+        cs.omega = sums[6 + c] / sums[12 + c];
     }
+    a.cs[c] = cs;
 }
 
 template <class T>
-__global__ void __launch_bounds__(BLK) k_fin_t(KryArgs<T> a) {
-    k_fin_t_body<T>(a, gridDim.x, blockIdx.x);
+__global__ void __launch_bounds__(FBLK) k_fin_t(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_t_body<T>(a, lds);
 }
 
 // ---- x += alpha M^-1 p + omega M^-1 s ; r = s - omega t ; |r|, (r0, r) ------
 template <class T>
-__device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_) {
     // FP64: x += alpha M^-1 p + omega M^-1 s in place.  Mixed: the inner
     // solve accumulates the same update into its FP32 correction e (from 0 at
     // the solve's first iteration) and k_fold adds e to x in FP64 before the
@@ -460,13 +465,13 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, int gG, int g
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, a.N, a.nRed, gG, gB);
+        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
         const int64_t t0 = tl * BLK;
-        const int32_t r = (int32_t)(t0 + threadIdx.x);
+        const int32_t r = (int32_t)(t0 + k_.tid);
         if (r >= a.N) continue;
         const double rd = a.rM ? a.rM[r] : 1.0;
         const int64_t j = (int64_t)NCMP * r;
@@ -513,12 +518,13 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, int gG, int g
     double qd[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) qd[i] = q[i];
-    write_partials<12>(qd, a.partials, gB);
+    write_partials<12>(qd, a.partials, k_);
 }
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_kry_xr(KryArgs<T> a) {
-    k_kry_xr_body<T>(a, gridDim.x, blockIdx.x);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_kry_xr_body<T>(a, blk_of_launch(red));
 }
 
 // ---- mixed: x += e (FP64) for the components about to be refined ----------
@@ -526,7 +532,7 @@ __global__ void __launch_bounds__(BLK) k_kry_xr(KryArgs<T> a) {
 // component waiting for refinement); the sweep's finalize then clears the
 // wait, so a correction is added once.
 template <class T>
-__device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     bool any = false;
 #pragma unroll
@@ -535,7 +541,7 @@ __device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, int gG, int gB)
         any |= on[c];
     }
     if (!any || inner_running(a)) return;
-    for (int64_t i = (int64_t)gB * BLK + threadIdx.x; i < a.N; i += (int64_t)gG * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
         double xv[6];
         T ev[6];
         ld6(a.x + NCMP * i, xv);
@@ -549,75 +555,72 @@ __device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, int gG, int gB)
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_fold(KryArgs<T> a) {
-    k_fold_body<T>(a, gridDim.x, blockIdx.x);
+    k_fold_body<T>(a, blk_of_launch(nullptr));
 }
 
 template <class T>
-__device__ __forceinline__ void k_fin_xr_body(const KryArgs<T>& a, int gG, int gB) {
-    bool on[6];
+__device__ __forceinline__ void k_fin_xr_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
+    for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
-    double sums[12];
-    sum_partials<12>(a.partials, a.G, sums);
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
-            CompState& cs = a.cs[c];
-            cs.iter += 1;
-            cs.innerIter += 1;
-            bool stop, breakdown = false;
-            if (cs.exitAtS) {
-                cs.exitAtS = 0;
+    const int c = threadIdx.x;
+    CompState cs;
+    cs.active = 0;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<12>(a.partials, a.G, lds, sums);
+    if (!cs.active) return;
+    cs.iter += 1;
+    cs.innerIter += 1;
+    bool stop, breakdown = false;
+    if (cs.exitAtS) {
+        cs.exitAtS = 0;
+        stop = true;
+    } else {
+        const double res = sums[c] / cs.normFactor;
+        if (!a.ctl.mixed) cs.finalRes = res;
+        const bool conv = conv_inner(cs, a.ctl, res);
+        bool cont = (!conv && cs.iter < a.ctl.maxIter) ||
+                    (!a.ctl.mixed && cs.iter < a.ctl.minIter);
+        if (a.ctl.mixed && cs.innerIter >= a.ctl.maxInner) cont = false;
+        stop = !cont;
+        if (cont) {
+            cs.rhoOld = cs.rho;
+            cs.rho = sums[6 + c];
+            if (fabs(cs.rho) < 1e-300 || fabs(cs.omega) < 1e-300) {
                 stop = true;
+                breakdown = true;
             } else {
-                const double res = sums[c] / cs.normFactor;
-                if (!a.ctl.mixed) cs.finalRes = res;
-                const bool conv = conv_inner(cs, a.ctl, res);
-                bool cont = (!conv && cs.iter < a.ctl.maxIter) ||
-                            (!a.ctl.mixed && cs.iter < a.ctl.minIter);
-                if (a.ctl.mixed && cs.innerIter >= a.ctl.maxInner) cont = false;
-                stop = !cont;
-                if (cont) {
-                    cs.rhoOld = cs.rho;
-                    cs.rho = sums[6 + c];
-                    if (fabs(cs.rho) < 1e-300 || fabs(cs.omega) < 1e-300) {
-                        stop = true;
-                        breakdown = true;
-                    } else {
-                        cs.beta = (cs.rho / cs.rhoOld) * (cs.alpha / cs.omega);
-                    }
-                }
-            }
-            if (stop) {
-                cs.active = 0;
-                // A breakdown ((r0, r) or omega vanishing before convergence)
-                // restarts from the true residual with r0 = r, through the same
-                // pass as a refinement sweep (at most maxRefine times); [OF9]
-                // PBiCGStab stops unconverged there instead (checkSingularity), but its
-                // DILU preconditioner meets breakdowns in other places than
-                // right Jacobi does, so stopping would leave results that differ
-                // from it by more than the tolerance.
-                if (a.ctl.mixed || breakdown || a.ctl.rb) {
-                    // mixed: fold the inner solve's correction, then refine;
-                    // red-black: the closing sweep eliminates the first colour
-                    cs.needRefine = 1;
-                    cs.foldE = a.ctl.mixed && cs.innerIter > 0 ? 1 : 0;
-                } else {
-                    cs.converged = conv_outer(cs, a.ctl, cs.finalRes);
-                }
+                cs.beta = (cs.rho / cs.rhoOld) * (cs.alpha / cs.omega);
             }
         }
     }
+    if (stop) {
+        cs.active = 0;
+        // A breakdown ((r0, r) or omega vanishing before convergence)
+        // restarts from the true residual with r0 = r, through the same
+        // pass as a refinement sweep (at most maxRefine times); [OF9]
+        // PBiCGStab stops unconverged there instead (checkSingularity), but its
+        // DILU preconditioner meets breakdowns in other places than
+        // right Jacobi does, so stopping would leave results that differ
+        // from it by more than the tolerance.
+        if (a.ctl.mixed || breakdown || a.ctl.rb) {
+            // mixed: fold the inner solve's correction, then refine;
+            // red-black: the closing sweep eliminates the first colour
+            cs.needRefine = 1;
+            cs.foldE = a.ctl.mixed && cs.innerIter > 0 ? 1 : 0;
+        } else {
+            cs.converged = conv_outer(cs, a.ctl, cs.finalRes);
+        }
+    }
+    a.cs[c] = cs;
 }
 
 template <class T>
-__global__ void __launch_bounds__(BLK) k_fin_xr(KryArgs<T> a) {
-    k_fin_xr_body<T>(a, gridDim.x, blockIdx.x);
+__global__ void __launch_bounds__(FBLK) k_fin_xr(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_xr_body<T>(a, lds);
 }
 
 // ================================== red-black ILU0 (multicolour ILU0, two colours)
@@ -639,7 +642,7 @@ __global__ void __launch_bounds__(BLK) k_fin_xr(KryArgs<T> a) {
 
 // R rows: w = D_R^-1 A_RB Ds^-1 y, y = p (SRC 0) or s = r - alpha v (SRC 1)
 template <class T, int SRC>
-__device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) {
     T* __restrict__ w = SRC == 0 ? a.v : a.t;
     T alpha[6];
     bool any = false;
@@ -651,12 +654,12 @@ __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, int gG, int gB)
     if (!any) return;
     const int64_t n = a.nRed;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, n, 0, gG, gB);
+        const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(tl * BLK + k_.tid);
         if (r >= n) continue;
         T acc[6] = {0, 0, 0, 0, 0, 0};
         const int s = r >> 6, lane = r & 63;
@@ -688,12 +691,12 @@ __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, int gG, int gB)
 
 template <class T, int SRC>
 __global__ void __launch_bounds__(BLK) k_rb_w(KryArgs<T> a) {
-    k_rb_w_body<T, SRC>(a, gridDim.x, blockIdx.x);
+    k_rb_w_body<T, SRC>(a, blk_of_launch(nullptr));
 }
 
 // B rows: v = S M^-1 p = (D_B Ds^-1) p - A_BR w ;  sigma = (r0, v)
 template <class T>
-__device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) {
     const T* __restrict__ w = a.v;
     bool on[6];
     bool any = false;
@@ -706,12 +709,12 @@ __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, int gG, int gB)
     T q[6] = {0, 0, 0, 0, 0, 0};
     const int64_t n = (int64_t)a.N - a.nRed;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, n, 0, gG, gB);
+        const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(a.nRed + tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(a.nRed + tl * BLK + k_.tid);
         if (r >= a.N) continue;
         T acc[6];
         ld6(a.p + (int64_t)NCMP * r, acc);
@@ -745,18 +748,19 @@ __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, int gG, int gB)
     double qd[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) qd[c] = q[c];
-    write_partials<6>(qd, a.partials, gB);
+    write_partials<6>(qd, a.partials, k_);
 }
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_rb_v(KryArgs<T> a) {
-    k_rb_v_body<T>(a, gridDim.x, blockIdx.x);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_rb_v_body<T>(a, blk_of_launch(red));
 }
 
 // B rows: s = r - alpha v ; t = S M^-1 s = (D_B Ds^-1) s - A_BR w' ;
 // |s|, (t, s), (t, t)
 template <class T>
-__device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) {
     const T* __restrict__ w = a.t;
     bool on[6];
     T alpha[6];
@@ -773,12 +777,12 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, int gG, int gB)
     for (int i = 0; i < 18; ++i) q[i] = 0;
     const int64_t n = (int64_t)a.N - a.nRed;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, n, 0, gG, gB);
+        const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(a.nRed + tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(a.nRed + tl * BLK + k_.tid);
         if (r >= a.N) continue;
         T sv[6], acc[6], rr[6], vv[6];
         ld6(a.r + (int64_t)NCMP * r, rr);
@@ -816,18 +820,19 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, int gG, int gB)
     double qd[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) qd[i] = q[i];
-    write_partials<18>(qd, a.partials, gB);
+    write_partials<18>(qd, a.partials, k_);
 }
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_rb_t(KryArgs<T> a) {
-    k_rb_t_body<T>(a, gridDim.x, blockIdx.x);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_rb_t_body<T>(a, blk_of_launch(red));
 }
 
 // The sweep's elimination of R (FP64): x_R = D_R^-1 (b_R - A_RB x_B) for the
 // components about to be refined; gated like the refinement sweep it opens.
 template <class T>
-__device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, int gG, int gB) {
+__device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     bool any = false;
 #pragma unroll
@@ -838,12 +843,12 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, int gG, i
     if (!any || inner_running(a)) return;
     const int64_t n = a.nRed;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, n, 0, gG, gB);
+        const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(tl * BLK + k_.tid);
         if (r >= n) continue;
         double acc[6];
         ld6(a.b + (int64_t)NCMP * r, acc);
@@ -874,7 +879,7 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, int gG, i
 
 template <class T>
 __global__ void __launch_bounds__(BLK) k_rb_backsub(KryArgs<T> a) {
-    k_rb_backsub_body<T>(a, gridDim.x, blockIdx.x);
+    k_rb_backsub_body<T>(a, blk_of_launch(nullptr));
 }
 
 // ahat of the red-black solve: A_jk / (D_j Ds_k) on R's rows, A_ij on B's
@@ -939,7 +944,7 @@ __global__ void k_rb_schur_diag(int32_t N, int32_t nRed, const int64_t* __restri
 // rT = b - A^T x (FP64) and the first wArT = (M^-1 rA, rT), after the
 // initial residual has written rA
 template <class T>
-__global__ void __launch_bounds__(BLK) k_bicg_init(KryArgs<T> a) {
+__device__ __forceinline__ void k_bicg_init_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     bool any = false;
 #pragma unroll
@@ -950,12 +955,12 @@ __global__ void __launch_bounds__(BLK) k_bicg_init(KryArgs<T> a) {
     if (!any) return;
     double q[6] = {0, 0, 0, 0, 0, 0};
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of(it, a.N, a.nRed);
+        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(tl * BLK + k_.tid);
         if (r >= a.N) continue;
         const double d = a.diag[r];
         double xv[6], y[6];
@@ -987,29 +992,41 @@ __global__ void __launch_bounds__(BLK) k_bicg_init(KryArgs<T> a) {
         }
         st6(a.r0 + (int64_t)NCMP * r, rT);
     }
-    write_partials<6>(q, a.partials);
+    write_partials<6>(q, a.partials, k_);
 }
 
 template <class T>
-__global__ void __launch_bounds__(BLK) k_fin_bicg_init(KryArgs<T> a) {
-    bool on[6];
+__global__ void __launch_bounds__(BLK) k_bicg_init(KryArgs<T> a) {
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_bicg_init_body<T>(a, blk_of_launch(red));
+}
+
+template <class T>
+__device__ __forceinline__ void k_fin_bicg_init_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
+    for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
-    double sums[6];
-    sum_partials<6>(a.partials, a.G, sums);
-    if (threadIdx.x == 0)
-        for (int c = 0; c < 6; ++c)
-            if (on[c]) a.cs[c].rho = sums[c];
+    const int c = threadIdx.x;
+    CompState cs;
+    cs.active = 0;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<6>(a.partials, a.G, lds, sums);
+    if (!cs.active) return;
+    cs.rho = sums[c];
+    a.cs[c] = cs;
+}
+
+template <class T>
+__global__ void __launch_bounds__(FBLK) k_fin_bicg_init(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_bicg_init_body<T>(a, lds);
 }
 
 // pA = M^-1 rA (+ beta pA), pT = M^-1 rT (+ beta pT)
 template <class T>
-__global__ void __launch_bounds__(BLK) k_bicg_p(KryArgs<T> a) {
+__device__ __forceinline__ void k_bicg_p_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6], first[6];
     T beta[6];
     bool any = false;
@@ -1021,7 +1038,7 @@ __global__ void __launch_bounds__(BLK) k_bicg_p(KryArgs<T> a) {
         any |= on[c];
     }
     if (!any) return;
-    for (int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x; i < a.N; i += (int64_t)gridDim.x * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
         const T rm = a.rM ? (T)a.rM[i] : (T)1;
         T rA[6], rT[6], pA[6], pT[6];
         ld6(a.r + NCMP * i, rA);
@@ -1040,9 +1057,14 @@ __global__ void __launch_bounds__(BLK) k_bicg_p(KryArgs<T> a) {
     }
 }
 
+template <class T>
+__global__ void __launch_bounds__(BLK) k_bicg_p(KryArgs<T> a) {
+    k_bicg_p_body<T>(a, blk_of_launch(nullptr));
+}
+
 // wA = A pA, wT = A^T pT; (wA, pT)
 template <class T>
-__global__ void __launch_bounds__(BLK) k_bicg_w(KryArgs<T> a) {
+__device__ __forceinline__ void k_bicg_w_body(const KryArgs<T>& a, const Blk& k_) {
     bool on[6];
     bool any = false;
 #pragma unroll
@@ -1053,12 +1075,12 @@ __global__ void __launch_bounds__(BLK) k_bicg_w(KryArgs<T> a) {
     if (!any) return;
     T q[6] = {0, 0, 0, 0, 0, 0};
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of(it, a.N, a.nRed);
+        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(tl * BLK + k_.tid);
         if (r >= a.N) continue;
         const T d = (T)a.diag[r];
         T wA[6], wT[6], pT[6];
@@ -1101,41 +1123,50 @@ __global__ void __launch_bounds__(BLK) k_bicg_w(KryArgs<T> a) {
     double qd[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) qd[c] = q[c];
-    write_partials<6>(qd, a.partials);
+    write_partials<6>(qd, a.partials, k_);
 }
 
 template <class T>
-__global__ void __launch_bounds__(BLK) k_fin_bicg_w(KryArgs<T> a) {
-    bool on[6];
+__global__ void __launch_bounds__(BLK) k_bicg_w(KryArgs<T> a) {
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_bicg_w_body<T>(a, blk_of_launch(red));
+}
+
+template <class T>
+__device__ __forceinline__ void k_fin_bicg_w_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
+    for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
-    double sums[6];
-    sum_partials<6>(a.partials, a.G, sums);
-    if (threadIdx.x == 0)
-        for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
-            CompState& cs = a.cs[c];
-            // checkSingularity(mag(wApT)/normFactor): stop; restarted from the
-            // true residual as after a PBiCGStab breakdown
-            if (fabs(sums[c]) / cs.normFactor < 1e-300) {
-                cs.active = 0;
-                cs.needRefine = 1;
-                // a correction to fold exists once this inner solve has updated e
-                cs.foldE = a.ctl.mixed && cs.innerIter > 0 ? 1 : 0;
-            } else {
-                cs.alpha = cs.rho / sums[c];
-            }
-        }
+    const int c = threadIdx.x;
+    CompState cs;
+    cs.active = 0;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<6>(a.partials, a.G, lds, sums);
+    if (!cs.active) return;
+    // checkSingularity(mag(wApT)/normFactor): stop; restarted from the
+    // true residual as after a PBiCGStab breakdown
+    if (fabs(sums[c]) / cs.normFactor < 1e-300) {
+        cs.active = 0;
+        cs.needRefine = 1;
+        // a correction to fold exists once this inner solve has updated e
+        cs.foldE = a.ctl.mixed && cs.innerIter > 0 ? 1 : 0;
+    } else {
+        cs.alpha = cs.rho / sums[c];
+    }
+    a.cs[c] = cs;
+}
+
+template <class T>
+__global__ void __launch_bounds__(FBLK) k_fin_bicg_w(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_bicg_w_body<T>(a, lds);
 }
 
 // psi += alpha pA, rA -= alpha wA, rT -= alpha wT; |rA|, (M^-1 rA, rT)
 template <class T>
-__global__ void __launch_bounds__(BLK) k_bicg_xr(KryArgs<T> a) {
+__device__ __forceinline__ void k_bicg_xr_body(const KryArgs<T>& a, const Blk& k_) {
     constexpr bool MIX = std::is_same<T, float>::value;
     bool on[6], first[6];
     double alpha[6];
@@ -1152,12 +1183,12 @@ __global__ void __launch_bounds__(BLK) k_bicg_xr(KryArgs<T> a) {
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
     for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of(it, a.N, a.nRed);
+        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(tl * BLK + threadIdx.x);
+        const int32_t r = (int32_t)(tl * BLK + k_.tid);
         if (r >= a.N) continue;
         const int64_t j = (int64_t)NCMP * r;
         const T rm = a.rM ? (T)a.rM[r] : (T)1;
@@ -1197,54 +1228,62 @@ __global__ void __launch_bounds__(BLK) k_bicg_xr(KryArgs<T> a) {
     double qd[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) qd[i] = q[i];
-    write_partials<12>(qd, a.partials);
+    write_partials<12>(qd, a.partials, k_);
 }
 
 template <class T>
-__global__ void __launch_bounds__(BLK) k_fin_bicg_xr(KryArgs<T> a) {
-    bool on[6];
+__global__ void __launch_bounds__(BLK) k_bicg_xr(KryArgs<T> a) {
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    k_bicg_xr_body<T>(a, blk_of_launch(red));
+}
+
+template <class T>
+__device__ __forceinline__ void k_fin_bicg_xr_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
+    for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
-    double sums[12];
-    sum_partials<12>(a.partials, a.G, sums);
-    if (threadIdx.x == 0) {
-        for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
-            CompState& cs = a.cs[c];
-            cs.iter += 1;
-            cs.innerIter += 1;
-            const double res = sums[c] / cs.normFactor;
-            if (!a.ctl.mixed) cs.finalRes = res;
-            const bool conv = conv_inner(cs, a.ctl, res);
-            bool cont = (!conv && cs.iter < a.ctl.maxIter) || (!a.ctl.mixed && cs.iter < a.ctl.minIter);
-            if (a.ctl.mixed && cs.innerIter >= a.ctl.maxInner) cont = false;
-            bool breakdown = false;
-            if (cont) {
-                cs.rhoOld = cs.rho;
-                cs.rho = sums[6 + c];
-                if (fabs(cs.rho) < 1e-300) {
-                    cont = false;
-                    breakdown = true;
-                } else {
-                    cs.beta = cs.rho / cs.rhoOld;
-                }
-            }
-            if (!cont) {
-                cs.active = 0;
-                if (a.ctl.mixed || breakdown) {
-                    cs.needRefine = 1;
-                    cs.foldE = a.ctl.mixed && cs.innerIter > 0 ? 1 : 0;
-                } else {
-                    cs.converged = conv_outer(cs, a.ctl, cs.finalRes);
-                }
-            }
+    const int c = threadIdx.x;
+    CompState cs;
+    cs.active = 0;
+    if (c < 6) cs = a.cs[c];
+    double* sums;
+    sum_partials<12>(a.partials, a.G, lds, sums);
+    if (!cs.active) return;
+    cs.iter += 1;
+    cs.innerIter += 1;
+    const double res = sums[c] / cs.normFactor;
+    if (!a.ctl.mixed) cs.finalRes = res;
+    const bool conv = conv_inner(cs, a.ctl, res);
+    bool cont = (!conv && cs.iter < a.ctl.maxIter) || (!a.ctl.mixed && cs.iter < a.ctl.minIter);
+    if (a.ctl.mixed && cs.innerIter >= a.ctl.maxInner) cont = false;
+    bool breakdown = false;
+    if (cont) {
+        cs.rhoOld = cs.rho;
+        cs.rho = sums[6 + c];
+        if (fabs(cs.rho) < 1e-300) {
+            cont = false;
+            breakdown = true;
+        } else {
+            cs.beta = cs.rho / cs.rhoOld;
         }
     }
+    if (!cont) {
+        cs.active = 0;
+        if (a.ctl.mixed || breakdown) {
+            cs.needRefine = 1;
+            cs.foldE = a.ctl.mixed && cs.innerIter > 0 ? 1 : 0;
+        } else {
+            cs.converged = conv_outer(cs, a.ctl, cs.finalRes);
+        }
+    }
+    a.cs[c] = cs;
+}
+
+template <class T>
+__global__ void __launch_bounds__(FBLK) k_fin_bicg_xr(KryArgs<T> a) {
+    __shared__ double lds[FIN_LDS];
+    k_fin_bicg_xr_body<T>(a, lds);
 }
 
 // float copies of the off-diagonals of A and A^T (mixed PBiCG)
@@ -1295,14 +1334,15 @@ __global__ void __launch_bounds__(BLK) k_mean6(int32_t N, const double* __restri
 #pragma unroll
         for (int c = 0; c < 6; ++c) q[c] += v[c];
     }
-    write_partials<6>(q, partials);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    write_partials<6>(q, partials, blk_of_launch(red));
 }
 
-__global__ void __launch_bounds__(BLK) k_fin_mean6(int32_t N, int G, const double* partials, CompState* cs) {
-    double sums[6];
-    sum_partials<6>(partials, G, sums);
-    if (threadIdx.x == 0)
-        for (int c = 0; c < 6; ++c) cs[c].xbar = sums[c] / N;
+__global__ void __launch_bounds__(FBLK) k_fin_mean6(int32_t N, int G, const double* partials, CompState* cs) {
+    __shared__ double lds[FIN_LDS];
+    double* sums;
+    sum_partials<6>(partials, G, lds, sums);
+    if (threadIdx.x < 6) cs[threadIdx.x].xbar = sums[threadIdx.x] / N;
 }
 
 // ----------------------------------------------------------------- driver
@@ -1324,7 +1364,7 @@ void launch_mean6(Ctx* ctx, int32_t N, const double* x, double* partials, CompSt
         ProfScope ps(ctx, "k_mean6", (double)N * 48);
         hipLaunchKernelGGL(k_mean6, dim3(grid), dim3(BLK), 0, ctx->stream, N, x, partials);
     }
-    hipLaunchKernelGGL(k_fin_mean6, dim3(1), dim3(BLK), 0, ctx->stream, N, grid, partials, cs);
+    hipLaunchKernelGGL(k_fin_mean6, dim3(1), dim3(FBLK), 0, ctx->stream, N, grid, partials, cs);
     RT_HIP(hipGetLastError());
 }
 
@@ -1659,7 +1699,7 @@ void launch_init(Ctx* ctx, SolveRun& R) {
         ProfScope ps(ctx, mixed ? "k_residual<f32>" : "k_residual<f64>", B.res(R.nValid));
         hipLaunchKernelGGL((k_residual<T, 0>), dim3(R.G), dim3(BLK), 0, ctx->stream, argsOf<T>(R));
     }
-    hipLaunchKernelGGL((k_fin_residual<T, 0>), dim3(1), dim3(BLK), 0, ctx->stream, argsOf<T>(R));
+    hipLaunchKernelGGL((k_fin_residual<T, 0>), dim3(1), dim3(FBLK), 0, ctx->stream, argsOf<T>(R));
 }
 
 // PBiCG: rT = b - A^T x and the first wArT, once the initial residual is in
@@ -1671,7 +1711,7 @@ void launch_bicg_init(Ctx* ctx, SolveRun& R) {
         ProfScope ps(ctx, mixed ? "k_bicg_init<f32>" : "k_bicg_init<f64>", B.binit(R.nValid));
         hipLaunchKernelGGL(k_bicg_init<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, argsOf<T>(R));
     }
-    hipLaunchKernelGGL(k_fin_bicg_init<T>, dim3(1), dim3(BLK), 0, ctx->stream, argsOf<T>(R));
+    hipLaunchKernelGGL(k_fin_bicg_init<T>, dim3(1), dim3(FBLK), 0, ctx->stream, argsOf<T>(R));
 }
 
 // The refinement sweep: mixed-precision fold, then the FP64 true residual and
@@ -1701,7 +1741,7 @@ void launch_refine(Ctx* ctx, SolveRun& R, double nRef, bool fold = true) {
             ProfScope ps(ctx, mixed ? "k_residual<f32>" : "k_residual<f64>", Bb.res(nRef));
             hipLaunchKernelGGL((k_residual<T, 1>), dim3(R.G), dim3(BLK), 0, ctx->stream, sweepOf<T>(R));
         }
-        hipLaunchKernelGGL((k_fin_residual<T, 1>), dim3(1), dim3(BLK), 0, ctx->stream, a);
+        hipLaunchKernelGGL((k_fin_residual<T, 1>), dim3(1), dim3(FBLK), 0, ctx->stream, a);
         return;
     }
     if (mixed && fold) {
@@ -1712,7 +1752,7 @@ void launch_refine(Ctx* ctx, SolveRun& R, double nRef, bool fold = true) {
         ProfScope ps(ctx, mixed ? "k_residual<f32>" : "k_residual<f64>", B.res(nRef));
         hipLaunchKernelGGL((k_residual<T, 1>), dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
-    hipLaunchKernelGGL((k_fin_residual<T, 1>), dim3(1), dim3(BLK), 0, ctx->stream, a);
+    hipLaunchKernelGGL((k_fin_residual<T, 1>), dim3(1), dim3(FBLK), 0, ctx->stream, a);
 }
 
 // One lockstep PBiCGStab iteration of the nAct active components.
@@ -1737,12 +1777,12 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
             ProfScope ps(ctx, mixed ? "k_bicg_w<f32>" : "k_bicg_w<f64>", B.bw(nAct));
             hipLaunchKernelGGL(k_bicg_w<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
         }
-        hipLaunchKernelGGL(k_fin_bicg_w<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_fin_bicg_w<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         {
             ProfScope ps(ctx, mixed ? "k_bicg_xr<f32>" : "k_bicg_xr<f64>", B.bxr(nAct));
             hipLaunchKernelGGL(k_bicg_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
         }
-        hipLaunchKernelGGL(k_fin_bicg_xr<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_fin_bicg_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         return;
     }
     if (R.rb) {
@@ -1764,7 +1804,7 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
             ProfScope ps(ctx, mixed ? "k_rb_v<f32>" : "k_rb_v<f64>", Bb.rbv(nAct));
             hipLaunchKernelGGL(k_rb_v<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
         }
-        hipLaunchKernelGGL(k_fin_v<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_fin_v<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         {
             ProfScope ps(ctx, mixed ? "k_rb_ws<f32>" : "k_rb_ws<f64>", Br.rbw(nAct, 1));
             hipLaunchKernelGGL((k_rb_w<T, 1>), dim3(R.Gw), dim3(BLK), 0, ctx->stream, a);
@@ -1773,12 +1813,12 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
             ProfScope ps(ctx, mixed ? "k_rb_t<f32>" : "k_rb_t<f64>", Bb.rbt(nAct));
             hipLaunchKernelGGL(k_rb_t<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
         }
-        hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         {
             ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", Bb.xr(nAct));
             hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, b);
         }
-        hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         return;
     }
     if (R.needScale) launch_scale_of<T>(ctx, R);
@@ -1790,17 +1830,17 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
         ProfScope ps(ctx, mixed ? "k_kry_v<f32>" : "k_kry_v<f64>", B.v(nAct));
         hipLaunchKernelGGL(k_kry_v<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
-    hipLaunchKernelGGL(k_fin_v<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+    hipLaunchKernelGGL(k_fin_v<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
     {
         ProfScope ps(ctx, mixed ? "k_kry_t<f32>" : "k_kry_t<f64>", B.t(nAct));
         hipLaunchKernelGGL(k_kry_t<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
-    hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+    hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
     {
         ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", B.xr(nAct));
         hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
-    hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(BLK), 0, ctx->stream, a);
+    hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
 }
 
 // rounds a non-blocking advance queues per host round trip
@@ -1957,12 +1997,20 @@ __device__ __forceinline__ int group_of(const int32_t* __restrict__ starts, int 
     return lo;
 }
 
-template <class T, void (*Body)(const KryArgs<T>&, int, int)>
+template <class T, void (*Body)(const KryArgs<T>&, const Blk&)>
 __global__ void __launch_bounds__(BLK) k_group(const KryArgs<T>* __restrict__ tab, const int32_t* __restrict__ starts,
                                                int n) {
     const int i = group_of(starts, n, blockIdx.x);
     const KryArgs<T> a = tab[i];
-    Body(a, starts[i + 1] - starts[i], blockIdx.x - starts[i]);
+    __shared__ double red[RED_MAX * (BLK / 64)];
+    Body(a, Blk{starts[i + 1] - starts[i], (int)blockIdx.x - starts[i], (int)threadIdx.x, red});
+}
+
+template <class T, void (*Body)(const KryArgs<T>&, double*)>
+__global__ void __launch_bounds__(FBLK) k_group_fin(const KryArgs<T>* __restrict__ tab) {
+    __shared__ double lds[FIN_LDS];
+    const KryArgs<T> a = tab[blockIdx.x];
+    Body(a, lds);
 }
 
 // device tables of a group: the members' arguments (whole rows; the red-black
@@ -1973,13 +2021,18 @@ struct GroupDev {
     const KryArgs<T>* A;
     const KryArgs<T>* B;
     const KryArgs<T>* S;
-    const int32_t *G, *P, *One, *W;
+    const int32_t *G, *P, *W;
     int n, totG, totP, totW;
 };
 
-template <class T, void (*Body)(const KryArgs<T>&, int, int)>
+template <class T, void (*Body)(const KryArgs<T>&, const Blk&)>
 void glaunch(hipStream_t st, const KryArgs<T>* tab, const int32_t* starts, int total, int n) {
     if (total > 0) hipLaunchKernelGGL((k_group<T, Body>), dim3(total), dim3(BLK), 0, st, tab, starts, n);
+}
+
+template <class T, void (*Body)(const KryArgs<T>&, double*)>
+void glaunch_fin(hipStream_t st, const KryArgs<T>* tab, int n) {
+    hipLaunchKernelGGL((k_group_fin<T, Body>), dim3(n), dim3(FBLK), 0, st, tab);
 }
 
 // One round as solve_advance queues it ahead for one solve: the refinement
@@ -1991,27 +2044,27 @@ void group_round(bool rb, hipStream_t st, const GroupDev<T>& d) {
         glaunch<T, &k_fold_body<T>>(st, d.B, d.P, d.totP, n);
         glaunch<T, &k_rb_backsub_body<T>>(st, d.A, d.W, d.totW, n);
         glaunch<T, &k_residual_body<T, 1>>(st, d.S, d.G, d.totG, n);
-        glaunch<T, &k_fin_residual_body<T, 1>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_residual_body<T, 1>>(st, d.A, n);
         glaunch<T, &k_kry_p_body<T>>(st, d.B, d.P, d.totP, n);
         glaunch<T, &k_rb_w_body<T, 0>>(st, d.A, d.W, d.totW, n);
         glaunch<T, &k_rb_v_body<T>>(st, d.A, d.G, d.totG, n);
-        glaunch<T, &k_fin_v_body<T>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_v_body<T>>(st, d.A, n);
         glaunch<T, &k_rb_w_body<T, 1>>(st, d.A, d.W, d.totW, n);
         glaunch<T, &k_rb_t_body<T>>(st, d.A, d.G, d.totG, n);
-        glaunch<T, &k_fin_t_body<T>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_t_body<T>>(st, d.A, n);
         glaunch<T, &k_kry_xr_body<T>>(st, d.B, d.G, d.totG, n);
-        glaunch<T, &k_fin_xr_body<T>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_xr_body<T>>(st, d.A, n);
     } else {
         glaunch<T, &k_fold_body<T>>(st, d.A, d.P, d.totP, n);
         glaunch<T, &k_residual_body<T, 1>>(st, d.A, d.G, d.totG, n);
-        glaunch<T, &k_fin_residual_body<T, 1>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_residual_body<T, 1>>(st, d.A, n);
         glaunch<T, &k_kry_p_body<T>>(st, d.A, d.P, d.totP, n);
         glaunch<T, &k_kry_v_body<T>>(st, d.A, d.G, d.totG, n);
-        glaunch<T, &k_fin_v_body<T>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_v_body<T>>(st, d.A, n);
         glaunch<T, &k_kry_t_body<T>>(st, d.A, d.G, d.totG, n);
-        glaunch<T, &k_fin_t_body<T>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_t_body<T>>(st, d.A, n);
         glaunch<T, &k_kry_xr_body<T>>(st, d.A, d.G, d.totG, n);
-        glaunch<T, &k_fin_xr_body<T>>(st, d.A, d.One, n, n);
+        glaunch_fin<T, &k_fin_xr_body<T>>(st, d.A, n);
     }
     RT_HIP(hipGetLastError());
 }
@@ -2026,8 +2079,7 @@ template <class T>
 void group_launch(SolveGroup& g) {
     const int n = (int)g.members.size();
     const size_t szA = sizeof(KryArgs<T>) * n, szI = sizeof(int32_t) * (n + 1);
-    const size_t offB = szA, offS = 2 * szA, offG = 3 * szA, offP = offG + szI, offO = offP + szI,
-                 offW = offO + szI;
+    const size_t offB = szA, offS = 2 * szA, offG = 3 * szA, offP = offG + szI, offW = offP + szI;
     const size_t bytes = offW + szI;
     int totG = 0, totP = 0, totW = 0;
     if (g.dirty) {
@@ -2044,9 +2096,8 @@ void group_launch(SolveGroup& g) {
         auto* tS = reinterpret_cast<KryArgs<T>*>(h + offS);
         auto* sG = reinterpret_cast<int32_t*>(h + offG);
         auto* sP = reinterpret_cast<int32_t*>(h + offP);
-        auto* sO = reinterpret_cast<int32_t*>(h + offO);
         auto* sW = reinterpret_cast<int32_t*>(h + offW);
-        sG[0] = sP[0] = sO[0] = sW[0] = 0;
+        sG[0] = sP[0] = sW[0] = 0;
         for (int i = 0; i < n; ++i) {
             SolveRun& R = *g.members[i].K->run;
             tA[i] = argsOf<T>(R);
@@ -2054,7 +2105,6 @@ void group_launch(SolveGroup& g) {
             tS[i] = g.rb ? sweepOf<T>(R) : argsOf<T>(R);
             sG[i + 1] = sG[i] + R.G;
             sP[i + 1] = sP[i] + point_grid(R);
-            sO[i + 1] = i + 1;
             sW[i + 1] = sW[i] + R.Gw;
         }
         // the previous launch's kernels have all finished (their pulls are back)
@@ -2070,8 +2120,8 @@ void group_launch(SolveGroup& g) {
     const unsigned char* d = static_cast<const unsigned char*>(g.tables.p);
     GroupDev<T> dv{reinterpret_cast<const KryArgs<T>*>(d), reinterpret_cast<const KryArgs<T>*>(d + offB),
                    reinterpret_cast<const KryArgs<T>*>(d + offS), reinterpret_cast<const int32_t*>(d + offG),
-                   reinterpret_cast<const int32_t*>(d + offP), reinterpret_cast<const int32_t*>(d + offO),
-                   reinterpret_cast<const int32_t*>(d + offW), n, totG, totP, totW};
+                   reinterpret_cast<const int32_t*>(d + offP), reinterpret_cast<const int32_t*>(d + offW),
+                   n, totG, totP, totW};
     for (int k = 0; k < kRoundsAhead; ++k) group_round<T>(g.rb, g.ctx->stream, dv);
     for (auto& mb : g.members) {
         SolveRun& R = *mb.K->run;

@@ -60,10 +60,46 @@ __device__ __forceinline__ int64_t tile_of(int64_t i, int64_t N, int64_t nRed = 
     return tile_of_g(i, N, nRed, gridDim.x, blockIdx.x);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
+// A row kernel's workgroup: index b of G workgroups of BLK threads, this
+// thread's index in it, and its LDS slots for partial sums ([RED_MAX][BLK/64]).
+// Bodies take it as an argument so that a launch of several solves, or a
+// workgroup made of several of these, runs them with the same arithmetic.
+constexpr int RED_MAX = 19;
+struct Blk {
+    int G, b, tid;
+    double* red;
+};
+
+__device__ __forceinline__ Blk blk_of_launch(double* red) {
+    return Blk{(int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, red};
+}
+
+// Sums of NQ per-lane values over the 64 lanes of a wavefront, halving the
+// values a lane carries at each exchange: 21 exchanges for 18 values where a
+// butterfly per value takes 108, with the butterfly's association of every
+// sum (the t pass of a 128 x 128 channel: 9.9 to 6.2 us with it).  Lane l ends
+// with the sum of value lo (valid if n > 0).
+template <int N, int O>
+__device__ __forceinline__ double wave_scatter(const double (&v)[N], int lane, int& lo, int& n) {
+    if constexpr (O == 0) {
+        return v[0];
+    } else if constexpr (N == 1) {
+        const double w[1] = {v[0] + __shfl_xor(v[0], O, 64)};
+        return wave_scatter<1, O / 2>(w, lane, lo, n);
+    } else {
+        constexpr int H = (N + 1) / 2;
+        const bool up = lane & O;
+        double w[H];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+        for (int i = 0; i < H; ++i) {
+            const double hi = H + i < N ? v[H + i] : 0.0;
+            const double keep = up ? hi : v[i], send = up ? v[i] : hi;
+            w[i] = keep + __shfl_xor(send, O, 64);
+        }
+        lo += up ? H : 0;
+        n = up ? n - H : (n < H ? n : H);
+        return wave_scatter<H, O / 2>(w, lane, lo, n);
+    }
 }
 
 // Grid reductions in two launches: every workgroup of the row kernel writes
@@ -73,57 +109,68 @@ __device__ __forceinline__ double wave_sum(double v) {
 // boundary makes the partials visible across the XCDs' L2s without per-block
 // agent-scope release fences.
 template <int NQ>
-__device__ __forceinline__ void write_partials(const double (&v)[NQ], double* partials, int blk) {
-    __shared__ double red[NQ][BLK / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        double s = wave_sum(v[q]);
-        if (lane == 0) red[q][wid] = s;
-    }
+__device__ __forceinline__ void write_partials(const double (&v)[NQ], double* partials, const Blk& k) {
+    static_assert(NQ <= RED_MAX, "partial-sum slots");
+    constexpr int W = BLK / 64;
+    int lo = 0, n = NQ;
+    const double s = wave_scatter<NQ, 32>(v, k.tid & 63, lo, n);
+    if (n > 0) k.red[lo * W + (k.tid >> 6)] = s;
     __syncthreads();
-    if (threadIdx.x < NQ) {
-        double s = 0;
-        for (int w = 0; w < BLK / 64; ++w) s += red[threadIdx.x][w];
-        partials[(int64_t)blk * NQ + threadIdx.x] = s;
+    if (k.tid < NQ && k.b < k.G) {
+        double t = 0;
+        for (int w = 0; w < W; ++w) t += k.red[k.tid * W + w];
+        partials[(int64_t)k.b * NQ + k.tid] = t;
     }
-}
-template <int NQ>
-__device__ __forceinline__ void write_partials(const double (&v)[NQ], double* partials) {
-    write_partials<NQ>(v, partials, blockIdx.x);
 }
 
-// In a one-workgroup finalize kernel: sums over the G blocks' partials
-// (thread 0 holds the result).
+// The finalize kernels' workgroup.  sum_partials: sums over the G blocks'
+// partials into sums[NQ] (LDS), by every thread of the workgroup.  The
+// partials are read as one flat array, thread t < J NQ the words t, t + J NQ,
+// ... (always quantity t % NQ), so a wavefront's loads are contiguous and
+// independent.  Latency bounds these kernels: against 256 threads with a row
+// each (144 B apart for NQ = 18) and thread 0 updating the records, the t
+// pass's finalize went from 7.0 to 3.8 us at 64 blocks (a 128 x 128 channel)
+// and from 11.8 to 8.3 us at 1280 (a 160^3 box).  The order of the sums
+// depends on G alone.
+constexpr int FBLK = 1024;
+constexpr int FIN_LDS = FBLK + 9 * RED_MAX;
 template <int NQ>
-__device__ __forceinline__ void sum_partials(const double* partials, int G, double (&sums)[NQ]) {
-    __shared__ double red[NQ][BLK / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    double acc[NQ];
+__device__ __forceinline__ void sum_partials(const double* partials, int G, double* lds, double*& sums) {
+    constexpr int J = FBLK / NQ, J2 = 8;
+    double* s2 = lds + FBLK;
+    sums = s2 + J2 * NQ;
+    const int t = threadIdx.x;
+    if (t < J * NQ) {
+        constexpr int S = J * NQ;
+        const int total = G * NQ;
+        double acc = 0;
+        int i = t;
+        for (; i + 7 * S < total; i += 8 * S) {
+            double v[8];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[q] = 0;
-    for (int i = threadIdx.x; i < G; i += BLK) {
-        const double* row = partials + (int64_t)i * NQ;
-        double tmp[NQ];
+            for (int u = 0; u < 8; ++u) v[u] = partials[i + u * S];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) tmp[q] = row[q];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) acc[q] += tmp[q];
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        double s = wave_sum(acc[q]);
-        if (lane == 0) red[q][wid] = s;
+            for (int u = 0; u < 8; ++u) acc += v[u];
+        }
+        for (; i < total; i += S) acc += partials[i];
+        lds[t] = acc;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (t < J2 * NQ) {
+        const int q = t % NQ;
+        double acc = 0;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            double s = 0;
-            for (int w = 0; w < BLK / 64; ++w) s += red[q][w];
-            sums[q] = s;
-        }
+        for (int j = t / NQ; j < J; j += J2) acc += lds[j * NQ + q];
+        s2[t] = acc;
     }
+    __syncthreads();
+    if (t < NQ) {
+        double acc = 0;
+#pragma unroll
+        for (int j = 0; j < J2; ++j) acc += s2[j * NQ + t];
+        sums[t] = acc;
+    }
+    __syncthreads();
 }
 
 // interleaved [N][6] rows: three 2-wide vector loads/stores per row
