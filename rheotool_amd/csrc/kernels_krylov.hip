@@ -79,6 +79,30 @@ __device__ __forceinline__ bool inner_running(const KryArgs<T>& a) {
     return run;
 }
 
+// The active components of a PBiCGStab round.  They are always in the same
+// inner iteration: a solve's components start together (the initial residual,
+// or a sweep that waits until no inner solve is running) and only leave.
+// In the first iteration p = r = r0, and r0 keeps that residual, so the passes
+// read r0 for all three: the sweep writes one vector instead of two, the copy
+// p = r is not made, and the second iteration takes its old p from r0.
+struct Round {
+    bool on[6];
+    bool any = false;
+    int inner = 0;  // the inner iteration of the active components
+};
+template <class T>
+__device__ __forceinline__ Round round_of(const KryArgs<T>& a) {
+    Round q;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        q.on[c] = a.cs[c].active;
+        const int i = a.cs[c].innerIter;
+        if (q.on[c]) q.inner = i;
+        q.any |= q.on[c];
+    }
+    return q;
+}
+
 template <class T, int MODE>
 __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& k_) {
     constexpr int NQ = 18;
@@ -132,7 +156,7 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& 
         }
         double bb[6];
         ld6(a.b + (int64_t)NCMP * r, bb);
-        // r and r0 are written whole (three 2-wide stores each): the entries of
+        // rows are written whole (three 2-wide stores): the entries of
         // components that are off belong to finished or frozen solves, which
         // no later kernel reads
         T rt[6];
@@ -152,8 +176,8 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& 
                 q[12 + c] += (rm * (double)rt[c]) * (double)rt[c];
             }
         }
-        st6(a.r + (int64_t)NCMP * r, rt);
-        st6(a.r0 + (int64_t)NCMP * r, rt);
+        if (MODE == 1 || !a.ctl.bicg) st6(a.r0 + (int64_t)NCMP * r, rt);
+        if (a.ctl.bicg) st6(a.r + (int64_t)NCMP * r, rt);
     }
     write_partials<NQ>(q, a.partials, k_);
 }
@@ -210,42 +234,27 @@ __global__ void __launch_bounds__(FBLK) k_fin_residual(KryArgs<T> a) {
     k_fin_residual_body<T, MODE>(a, lds);
 }
 
-// ---- p = r  |  p = r + beta (p - omega v) ---------------------------------
+// ---- p = r + beta (p - omega v), from the second inner iteration on ---------
 template <class T>
 __device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, const Blk& k_) {
-    bool on[6];
-    bool first[6];
+    const Round q = round_of(a);
+    if (!q.any || q.inner == 0) return;
     T beta[6], omega[6];
-    bool any = false, update = false;
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        first[c] = a.cs[c].innerIter == 0;
         beta[c] = (T)a.cs[c].beta;
         omega[c] = (T)a.cs[c].omega;
-        any |= on[c];
-        update |= on[c] && !first[c];
     }
-    if (!any) return;
+    const T* pOld = q.inner == 1 ? a.r0 : a.p;
     const int64_t N = a.N;
-    if (!update) {
-        // every active component starts an inner solve: p = r.  The other
-        // components' p is dead until their own restart sets it.
-        for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
-            T rr[6];
-            ld6(a.r + NCMP * i, rr);
-            st6(a.p + NCMP * i, rr);
-        }
-        return;
-    }
     for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
         T rr[6], pp[6], vv[6];
         ld6(a.r + NCMP * i, rr);
-        ld6(a.p + NCMP * i, pp);
+        ld6(pOld + NCMP * i, pp);
         ld6(a.v + NCMP * i, vv);
 #pragma unroll
         for (int c = 0; c < 6; ++c)
-            if (on[c]) pp[c] = first[c] ? rr[c] : rr[c] + beta[c] * (pp[c] - omega[c] * vv[c]);
+            if (q.on[c]) pp[c] = rr[c] + beta[c] * (pp[c] - omega[c] * vv[c]);
         st6(a.p + NCMP * i, pp);
     }
 }
@@ -258,14 +267,10 @@ __global__ void __launch_bounds__(BLK) k_kry_p(KryArgs<T> a) {
 // ---- v = A M^-1 p = p + Ahat p ;  sigma = (r0, v) -------------------------
 template <class T>
 __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_) {
-    bool on[6];
-    bool any = false;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
-    if (!any) return;
+    const Round rd = round_of(a);
+    if (!rd.any) return;
+    const bool start = rd.inner == 0;
+    const T* pv = start ? a.r0 : a.p;
     T q[6] = {0, 0, 0, 0, 0, 0};
     for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
@@ -276,8 +281,14 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_)
         const int64_t t0 = tl * BLK;
         const int32_t r = (int32_t)(t0 + k_.tid);
         if (r >= a.N) continue;
-        T acc[6];
-        ld6(a.p + (int64_t)NCMP * r, acc);
+        T acc[6], rr0[6];
+        ld6(pv + (int64_t)NCMP * r, acc);
+        if (start) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) rr0[c] = acc[c];
+        } else {
+            ld6(a.r0 + (int64_t)NCMP * r, rr0);
+        }
         if (a.dg) {
             const T dgr = (T)a.dg[r];
 #pragma unroll
@@ -294,16 +305,14 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_)
             const T av = ld_stream<T>(a.ahat + e);
             if (av == (T)0) continue;
             T pc[6];
-            ld6(a.p + (int64_t)NCMP * col, pc);
+            ld6(pv + (int64_t)NCMP * col, pc);
 #pragma unroll
             for (int c = 0; c < 6; ++c) acc[c] += av * pc[c];
         }
         st6(a.v + (int64_t)NCMP * r, acc);
-        T rr0[6];
-        ld6(a.r0 + (int64_t)NCMP * r, rr0);
 #pragma unroll
         for (int c = 0; c < 6; ++c)
-            if (on[c]) q[c] += rr0[c] * acc[c];
+            if (rd.on[c]) q[c] += rr0[c] * acc[c];
     }
     double qd[6];
 #pragma unroll
@@ -343,16 +352,12 @@ __global__ void __launch_bounds__(FBLK) k_fin_v(KryArgs<T> a) {
 // ---- s = r - alpha v ; t = A M^-1 s ; |s|, (t,s), (t,t) --------------------
 template <class T>
 __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_) {
-    bool on[6];
+    const Round rd = round_of(a);
+    if (!rd.any) return;
+    const T* rv = rd.inner == 0 ? a.r0 : a.r;
     T alpha[6];
-    bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        alpha[c] = (T)a.cs[c].alpha;
-        any |= on[c];
-    }
-    if (!any) return;
+    for (int c = 0; c < 6; ++c) alpha[c] = (T)a.cs[c].alpha;
     T q[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
@@ -366,7 +371,7 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
         const int32_t r = (int32_t)(t0 + k_.tid);
         if (r >= a.N) continue;
         T sv[6], acc[6], rr[6], vv[6];
-        ld6(a.r + (int64_t)NCMP * r, rr);
+        ld6(rv + (int64_t)NCMP * r, rr);
         ld6(a.v + (int64_t)NCMP * r, vv);
         const T dgr = a.dg ? (T)a.dg[r] : (T)1;
 #pragma unroll
@@ -385,7 +390,7 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
             const T av = ld_stream<T>(a.ahat + e);
             if (av == (T)0) continue;
             T rc[6], vc[6];
-            ld6(a.r + (int64_t)NCMP * col, rc);
+            ld6(rv + (int64_t)NCMP * col, rc);
             ld6(a.v + (int64_t)NCMP * col, vc);
 #pragma unroll
             for (int c = 0; c < 6; ++c) acc[c] += av * (rc[c] - alpha[c] * vc[c]);
@@ -393,7 +398,7 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
         st6(a.t + (int64_t)NCMP * r, acc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
+            if (!rd.on[c]) continue;
             q[c] += fabs(sv[c]);
             q[6 + c] += acc[c] * sv[c];
             q[12 + c] += acc[c] * acc[c];
@@ -448,19 +453,17 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
     // the solve's first iteration) and k_fold adds e to x in FP64 before the
     // refinement sweep, so the pass moves 4-byte instead of 8-byte x words.
     constexpr bool MIX = std::is_same<T, float>::value;
-    bool on[6], ex[6], first[6];
+    const Round rd_ = round_of(a);
+    if (!rd_.any) return;
+    const bool start = rd_.inner == 0;
+    bool ex[6];
     double alpha[6], omega[6];
-    bool any = false;
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
         ex[c] = a.cs[c].exitAtS;
-        first[c] = a.cs[c].innerIter == 0;
         alpha[c] = a.cs[c].alpha;
         omega[c] = a.cs[c].omega;
-        any |= on[c];
     }
-    if (!any) return;
     T q[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
@@ -479,20 +482,30 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
         T ev[6];
         T pp[6], rr[6], vv[6], tt[6], rr0[6];
         if constexpr (MIX) {
-            ld6(a.e + j, ev);
+            if (start) {
 #pragma unroll
-            for (int c = 0; c < 6; ++c) xv[c] = first[c] ? 0.0 : (double)ev[c];
+                for (int c = 0; c < 6; ++c) xv[c] = 0.0;
+            } else {
+                ld6(a.e + j, ev);
+#pragma unroll
+                for (int c = 0; c < 6; ++c) xv[c] = (double)ev[c];
+            }
         } else {
             ld6(a.x + j, xv);
         }
-        ld6(a.p + j, pp);
-        ld6(a.r + j, rr);
+        ld6(a.r0 + j, rr0);
         ld6(a.v + j, vv);
         ld6(a.t + j, tt);
-        ld6(a.r0 + j, rr0);
+        if (start) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) pp[c] = rr[c] = rr0[c];
+        } else {
+            ld6(a.p + j, pp);
+            ld6(a.r + j, rr);
+        }
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
+            if (!rd_.on[c]) continue;
             const double y = rd * (double)pp[c];
             if (ex[c]) {
                 xv[c] += alpha[c] * y;
@@ -644,14 +657,13 @@ __global__ void __launch_bounds__(FBLK) k_fin_xr(KryArgs<T> a) {
 template <class T, int SRC>
 __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) {
     T* __restrict__ w = SRC == 0 ? a.v : a.t;
+    const Round rd = round_of(a);
+    if (!rd.any) return;
+    const T* pv = rd.inner == 0 ? a.r0 : a.p;
+    const T* rv = rd.inner == 0 ? a.r0 : a.r;
     T alpha[6];
-    bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        alpha[c] = (T)a.cs[c].alpha;
-        any |= a.cs[c].active != 0;
-    }
-    if (!any) return;
+    for (int c = 0; c < 6; ++c) alpha[c] = (T)a.cs[c].alpha;
     const int64_t n = a.nRed;
     for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
@@ -674,12 +686,12 @@ __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) 
             if (av == (T)0) continue;
             if constexpr (SRC == 0) {
                 T pc[6];
-                ld6(a.p + (int64_t)NCMP * col, pc);
+                ld6(pv + (int64_t)NCMP * col, pc);
 #pragma unroll
                 for (int c = 0; c < 6; ++c) acc[c] += av * pc[c];
             } else {
                 T rc[6], vc[6];
-                ld6(a.r + (int64_t)NCMP * col, rc);
+                ld6(rv + (int64_t)NCMP * col, rc);
                 ld6(a.v + (int64_t)NCMP * col, vc);
 #pragma unroll
                 for (int c = 0; c < 6; ++c) acc[c] += av * (rc[c] - alpha[c] * vc[c]);
@@ -698,14 +710,10 @@ __global__ void __launch_bounds__(BLK) k_rb_w(KryArgs<T> a) {
 template <class T>
 __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) {
     const T* __restrict__ w = a.v;
-    bool on[6];
-    bool any = false;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        any |= on[c];
-    }
-    if (!any) return;
+    const Round rd = round_of(a);
+    if (!rd.any) return;
+    const bool start = rd.inner == 0;
+    const T* pv = start ? a.r0 : a.p;
     T q[6] = {0, 0, 0, 0, 0, 0};
     const int64_t n = (int64_t)a.N - a.nRed;
     for (int64_t it = 0;; ++it) {
@@ -716,8 +724,14 @@ __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) 
         }
         const int32_t r = (int32_t)(a.nRed + tl * BLK + k_.tid);
         if (r >= a.N) continue;
-        T acc[6];
-        ld6(a.p + (int64_t)NCMP * r, acc);
+        T acc[6], rr0[6];
+        ld6(pv + (int64_t)NCMP * r, acc);
+        if (start) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) rr0[c] = acc[c];
+        } else {
+            ld6(a.r0 + (int64_t)NCMP * r, rr0);
+        }
         if (a.dg) {
             const T dgr = (T)a.dg[r];
 #pragma unroll
@@ -739,11 +753,9 @@ __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) 
             for (int c = 0; c < 6; ++c) acc[c] -= av * wc[c];
         }
         st6(a.v + (int64_t)NCMP * r, acc);
-        T rr0[6];
-        ld6(a.r0 + (int64_t)NCMP * r, rr0);
 #pragma unroll
         for (int c = 0; c < 6; ++c)
-            if (on[c]) q[c] += rr0[c] * acc[c];
+            if (rd.on[c]) q[c] += rr0[c] * acc[c];
     }
     double qd[6];
 #pragma unroll
@@ -762,16 +774,12 @@ __global__ void __launch_bounds__(BLK) k_rb_v(KryArgs<T> a) {
 template <class T>
 __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) {
     const T* __restrict__ w = a.t;
-    bool on[6];
+    const Round rd = round_of(a);
+    if (!rd.any) return;
+    const T* rv = rd.inner == 0 ? a.r0 : a.r;
     T alpha[6];
-    bool any = false;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        on[c] = a.cs[c].active;
-        alpha[c] = (T)a.cs[c].alpha;
-        any |= on[c];
-    }
-    if (!any) return;
+    for (int c = 0; c < 6; ++c) alpha[c] = (T)a.cs[c].alpha;
     T q[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
@@ -785,7 +793,7 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) 
         const int32_t r = (int32_t)(a.nRed + tl * BLK + k_.tid);
         if (r >= a.N) continue;
         T sv[6], acc[6], rr[6], vv[6];
-        ld6(a.r + (int64_t)NCMP * r, rr);
+        ld6(rv + (int64_t)NCMP * r, rr);
         ld6(a.v + (int64_t)NCMP * r, vv);
         const T dgr = a.dg ? (T)a.dg[r] : (T)1;
 #pragma unroll
@@ -811,7 +819,7 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) 
         st6(a.t + (int64_t)NCMP * r, acc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
-            if (!on[c]) continue;
+            if (!rd.on[c]) continue;
             q[c] += fabs(sv[c]);
             q[6 + c] += acc[c] * sv[c];
             q[12 + c] += acc[c] * acc[c];
@@ -1650,12 +1658,14 @@ void fill_args(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
 // move all 6 components; gathered vectors counted once)
 struct Bytes {
     double N, ne, w;
-    double res(double nc) const { return N * 8.0 + ne * 12 + nc * N * (8 + 8 + 2 * w); }
-    double p(double nc, bool start) const { return nc * N * (start ? 2 : 4) * w; }
-    double v(double nc) const { return ne * (4 + w) + nc * N * 3 * w; }
+    double res(double nc) const { return N * 8.0 + ne * 12 + nc * N * (8 + 8 + w); }
+    double p(double nc) const { return nc * N * 4 * w; }
+    double v(double nc, bool start) const { return ne * (4 + w) + nc * N * (start ? 2 : 3) * w; }
     double t(double nc) const { return ne * (4 + w) + nc * N * 3 * w; }
     // FP64: x read and written in place; mixed: the FP32 correction instead
-    double xr(double nc) const { return N * 8.0 + nc * N * (w == 4 ? 8 * w : 16 + 6 * w); }
+    double xr(double nc, bool start) const {
+        return N * 8.0 + nc * N * (w == 4 ? (start ? 5 : 8) * w : 16 + (start ? 4 : 6) * w);
+    }
     double fold(double nc) const { return nc * N * (8 + 8 + w); }
     // PBiCG: rT = b - A^T x; the p pass; A pA and A^T pT; the x/r pass
     double binit(double nc) const { return N * 16.0 + ne * 12 + nc * N * (8 + 8 + 2 * w); }
@@ -1667,7 +1677,7 @@ struct Bytes {
     // second colour's v and t passes gather w and stream their own vectors;
     // the elimination of the first colour and the sweep's residual in FP64
     double rbw(double nc, int src) const { return ne * (4 + w) + nc * N * (src ? 3 : 2) * w; }
-    double rbv(double nc) const { return ne * (4 + w) + nc * N * 4 * w; }
+    double rbv(double nc, bool start) const { return ne * (4 + w) + nc * N * (start ? 3 : 4) * w; }
     double rbt(double nc) const { return ne * (4 + w) + nc * N * 5 * w; }
     double rbx(double nc) const { return N * 8.0 + ne * 12 + nc * N * (8 + 8 + 8); }
 };
@@ -1755,7 +1765,8 @@ void launch_refine(Ctx* ctx, SolveRun& R, double nRef, bool fold = true) {
     hipLaunchKernelGGL((k_fin_residual<T, 1>), dim3(1), dim3(FBLK), 0, ctx->stream, a);
 }
 
-// One lockstep PBiCGStab iteration of the nAct active components.
+// One lockstep PBiCGStab iteration of the nAct active components.  start: the
+// host knows it to be their inner solve's first (no p pass).
 template <class T>
 void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
     const bool mixed = std::is_same<T, float>::value;
@@ -1792,8 +1803,8 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
         KryArgs<T>& b = blackOf<T>(R);
         const int pg = std::max(1, std::min<int>(R.pgrid, (int)((R.N - R.nRed + BLK - 1) / BLK)));
         // w lives on the first colour's rows of v, w' on those of t
-        {
-            ProfScope ps(ctx, mixed ? "k_kry_p<f32>" : "k_kry_p<f64>", Bb.p(nAct, start));
+        if (!start) {
+            ProfScope ps(ctx, mixed ? "k_kry_p<f32>" : "k_kry_p<f64>", Bb.p(nAct));
             hipLaunchKernelGGL(k_kry_p<T>, dim3(pg), dim3(BLK), 0, ctx->stream, b);
         }
         {
@@ -1801,7 +1812,7 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
             hipLaunchKernelGGL((k_rb_w<T, 0>), dim3(R.Gw), dim3(BLK), 0, ctx->stream, a);
         }
         {
-            ProfScope ps(ctx, mixed ? "k_rb_v<f32>" : "k_rb_v<f64>", Bb.rbv(nAct));
+            ProfScope ps(ctx, mixed ? "k_rb_v<f32>" : "k_rb_v<f64>", Bb.rbv(nAct, start));
             hipLaunchKernelGGL(k_rb_v<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
         }
         hipLaunchKernelGGL(k_fin_v<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
@@ -1815,19 +1826,19 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
         }
         hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         {
-            ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", Bb.xr(nAct));
+            ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", Bb.xr(nAct, start));
             hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, b);
         }
         hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         return;
     }
     if (R.needScale) launch_scale_of<T>(ctx, R);
-    {
-        ProfScope ps(ctx, mixed ? "k_kry_p<f32>" : "k_kry_p<f64>", B.p(nAct, start));
+    if (!start) {
+        ProfScope ps(ctx, mixed ? "k_kry_p<f32>" : "k_kry_p<f64>", B.p(nAct));
         hipLaunchKernelGGL(k_kry_p<T>, dim3(R.pgrid), dim3(BLK), 0, ctx->stream, a);
     }
     {
-        ProfScope ps(ctx, mixed ? "k_kry_v<f32>" : "k_kry_v<f64>", B.v(nAct));
+        ProfScope ps(ctx, mixed ? "k_kry_v<f32>" : "k_kry_v<f64>", B.v(nAct, start));
         hipLaunchKernelGGL(k_kry_v<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
     hipLaunchKernelGGL(k_fin_v<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
@@ -1837,7 +1848,7 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
     }
     hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
     {
-        ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", B.xr(nAct));
+        ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", B.xr(nAct, start));
         hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
     hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
@@ -1927,7 +1938,7 @@ bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
         }
     }
     double nAct = 0, nRef = 0;
-    bool start = true;  // every component of the round begins an inner solve (p = r)
+    bool start = true;  // every component of the round begins an inner solve (p = r = r0)
     for (int c = 0; c < 6; ++c) {
         if (R.valid[c] <= 0) continue;
         nAct += R.host[c].active != 0;

@@ -574,11 +574,10 @@ void modelCorrectBegin(Model& M, double deltaT, const double* gradU, int iterati
     for (int q = 0; q < 6; ++q) a.valid[q] = M.valid6[q];
     a.rD = M.kry.rD.as<double>();
     a.ctl = kryCtl(M.ctl, mixed, m);
-    // the red-black solve opens with a sweep that writes r and r0 on the
-    // second colour from the eliminated first colour; the assembly's own
-    // residual then only feeds the normalisation and the initial residual
-    a.r = a.ctl.rb ? nullptr : (mixed ? M.kry.rs.p : M.kry.r.p);
-    a.r0 = a.ctl.rb ? nullptr : (mixed ? M.kry.r0s.p : M.kry.r0.p);
+    // the red-black solve opens with a sweep that writes r0 on the second
+    // colour from the eliminated first colour; the assembly's own residual
+    // then only feeds the normalisation and the initial residual
+    a.r = a.ctl.rb ? nullptr : bicg ? (mixed ? M.kry.rs.p : M.kry.r.p) : (mixed ? M.kry.r0s.p : M.kry.r0.p);
     a.nRed = m.nRed;
     a.mixed = mixed ? 1 : 0;
     a.noConv = M.scheme == DS_NONE ? 1 : 0;

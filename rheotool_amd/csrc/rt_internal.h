@@ -402,11 +402,10 @@ struct AssembleArgs {
     double* nnzOut;       // SolveState::misc[0]
     int32_t valid[6];
     // initial residual of the solve, fused into the assembly
-    void* r;              // [N][6] Krylov precision
-    void* r0;
+    void* r;              // [N][6] Krylov precision: r0 of PBiCGStab, rA of PBiCG, NULL for none
     double* rD;           // [N] 1/diag
     KryCtl ctl;
-    int32_t mixed;        // r/r0 in FP32
+    int32_t mixed;        // r in FP32
     int32_t nRed;         // colour-blocked rows: the first colour's count (tile order), 0: none
 };
 
