@@ -587,13 +587,13 @@ __global__ void __launch_bounds__(FBLK) k_fin_assemble(AssembleArgs a, int G) {
 #pragma unroll
     for (int i = 0; i < 6; ++i)
         if (i == c) on = a.valid[i] > 0;
-    CompState cs;
-    if (c < 6) cs = a.cs[c];
+    Comp cs;
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
     sum_partials<19>(a.partials, G, lds, sums);
     if (on) {
         finish_initial(cs, a.ctl, sums[c], sums[6 + c], sums[12 + c]);
-        a.cs[c] = cs;
+        cs.store(a.cs[c]);
     }
     if (c == 6) *a.nnzOut = sums[18];
 }
@@ -1362,7 +1362,7 @@ static int resident_grid(const Ctx* ctx, int cap) {
         perCU = nb;
     }
     int64_t g = std::min<int64_t>(cap, (int64_t)ctx->numCUs * perCU);
-    if (g >= 64) g = g / 8 * 8;
+    if (g >= 64 && g < cap) g = g / 8 * 8;
     return (int)std::max<int64_t>(1, g);
 }
 

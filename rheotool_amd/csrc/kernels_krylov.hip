@@ -71,6 +71,96 @@ __device__ __forceinline__ U ld_stream(const U* p) {
     else return *p;
 }
 
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uni(double v) {
+    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
+
+// The live entries of row r in column order, W at a time: f(col, av) gets W
+// columns and values (value 0: none).  A wavefront's rows are one slice, so
+// which slots are live is the same for its lanes.  The W loads of an entry's
+// column and value, and f's W gathers, are in flight together: taken one entry
+// after another, each waits for two memory round trips.
+template <int W, class T, class V, class F>
+__device__ __forceinline__ void for_entries(const KryArgs<T>& a, int32_t r, const V* vals, F&& f) {
+    const int s = uni(r >> 6);
+    const int64_t base = a.ellOff[s] + (r & 63);
+    const int width = a.ellWidth[s];
+    uint32_t m = a.slotMask ? a.slotMask[s] : 0xffffffffu;
+    if (width < 32) m &= (1u << width) - 1u;
+    m = (uint32_t)uni((int)m);
+    while (m) {
+        int32_t col[W];
+        V av[W];
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            col[j] = r;
+            av[j] = (V)0;
+            if (m) {
+                const int64_t e = base + (int64_t)SLICE * __builtin_ctz(m);
+                m &= m - 1;
+                col[j] = ld_stream<T>(a.ellCol + e);
+                av[j] = ld_stream<T>(vals + e);
+            }
+        }
+        f(col, av);
+    }
+    for (int k = 32; k < width; k += W) {
+        int32_t col[W];
+        V av[W];
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            col[j] = r;
+            av[j] = (V)0;
+            if (k + j < width) {
+                const int64_t e = base + (int64_t)SLICE * (k + j);
+                col[j] = ld_stream<T>(a.ellCol + e);
+                av[j] = ld_stream<T>(vals + e);
+            }
+        }
+        f(col, av);
+    }
+}
+
+// acc += av * src[col] (NEG: acc -= ...) over W entries; entries with no
+// coefficient (the downwind side of a face) are not gathered
+template <bool NEG, int W, class U, class V>
+__device__ __forceinline__ void gather(const U* src, const int32_t (&col)[W], const V (&av)[W], U (&acc)[6]) {
+    U g[W][6];
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+        if (av[j] != (V)0) ld6(src + (int64_t)NCMP * col[j], g[j]);
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+        if (av[j] != (V)0) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) acc[c] = NEG ? acc[c] - av[j] * g[j][c] : acc[c] + av[j] * g[j][c];
+        }
+}
+// the same of s = r - alpha v
+template <int W, class T>
+__device__ __forceinline__ void gather_s(const T* rv, const T* vv, const T (&alpha)[6], const int32_t (&col)[W],
+                                         const T (&av)[W], T (&acc)[6]) {
+    T g[W][6], h[W][6];
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+        if (av[j] != (T)0) {
+            ld6(rv + (int64_t)NCMP * col[j], g[j]);
+            ld6(vv + (int64_t)NCMP * col[j], h[j]);
+        }
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+        if (av[j] != (T)0) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) acc[c] += av[j] * (g[j][c] - alpha[c] * h[j][c]);
+        }
+}
+// entries in flight: four rows of six words (two vectors of FP64: two)
+template <class T, int NV = 1>
+constexpr int ENT = sizeof(T) * NV <= 8 ? 4 : 2;
+
 template <class T>
 __device__ __forceinline__ bool inner_running(const KryArgs<T>& a) {
     bool run = false;
@@ -95,8 +185,8 @@ __device__ __forceinline__ Round round_of(const KryArgs<T>& a) {
     Round q;
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
-        q.on[c] = a.cs[c].active;
-        const int i = a.cs[c].innerIter;
+        q.on[c] = uni(a.cs[c].active);
+        const int i = uni(a.cs[c].innerIter);
         if (q.on[c]) q.inner = i;
         q.any |= q.on[c];
     }
@@ -122,38 +212,30 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& 
     for (int c = 0; c < 6; ++c) xbar[c] = MODE == 0 ? a.cs[c].xbar : 0.0;
     // rows [rowBegin, N): all rows, or the second colour of a red-black sweep
     // (the first colour's residual is zero once it has been eliminated)
-    const int64_t nRows = (int64_t)a.N - a.rowBegin;
-    for (int64_t it = 0;; ++it) {
+    const int32_t rowB = a.rowBegin & ~(SLICE - 1);  // wavefronts on whole slices
+    const int64_t nRows = (int64_t)a.N - rowB;
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = a.rowBegin > 0 ? tile_of_g(it, nRows, 0, k_.G, k_.b) : tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
         const int64_t t0 = tl * BLK;
-        const int32_t r = (int32_t)(a.rowBegin + t0 + k_.tid);
-        if (r >= a.N) continue;
+        const int32_t r = (int32_t)(rowB + t0 + k_.tid);
+        if (r < a.rowBegin || r >= a.N) continue;
         const double d = a.diag[r];
         double y[6], xv[6];
         ld6(a.x + (int64_t)NCMP * r, xv);
 #pragma unroll
         for (int c = 0; c < 6; ++c) y[c] = d * xv[c];
         double sumA = d;
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;  // zero in every row of the slice
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            const double av = ld_stream<T>(a.aval + e);
-            if (MODE == 0) sumA += av;
-            if (av == 0.0) continue;  // upwind: the downwind side of a face has no coupling
-            double xc[6];
-            ld6(a.x + (int64_t)NCMP * col, xc);
+        for_entries<ENT<double>>(a, r, a.aval, [&](const auto& col, const auto& av) {
+            if (MODE == 0) {
 #pragma unroll
-            for (int c = 0; c < 6; ++c) y[c] += av * xc[c];
-        }
+                for (int j = 0; j < ENT<double>; ++j) sumA += av[j];
+            }
+            gather<false>(a.x, col, av, y);
+        });
         double bb[6];
         ld6(a.b + (int64_t)NCMP * r, bb);
         // rows are written whole (three 2-wide stores): the entries of
@@ -192,7 +274,7 @@ __global__ void __launch_bounds__(BLK) k_residual(KryArgs<T> a) {
 // lane c of the first wavefront updates component c's record.  (Thread 0
 // updating the six records one after another, with a memory round trip for
 // each, was most of these kernels' time.)
-template <class T, int MODE>
+template <class T, int MODE, int NT = FBLK>
 __device__ __forceinline__ void k_fin_residual_body(const KryArgs<T>& a, double* lds) {
     constexpr int NQ = 18;
     bool on = false, any = false;
@@ -204,10 +286,10 @@ __device__ __forceinline__ void k_fin_residual_body(const KryArgs<T>& a, double*
         if (i == c) on = o;
     }
     if (!any || (MODE == 1 && inner_running(a))) return;
-    CompState cs;
-    if (c < 6) cs = a.cs[c];
+    Comp cs;
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<NQ>(a.partials, a.G, lds, sums);
+    sum_partials<NQ, NT>(a.partials, a.G, lds, sums);
     if (!on) return;
     if (MODE == 0) {
         finish_initial(cs, a.ctl, sums[c], sums[6 + c], sums[12 + c]);
@@ -225,7 +307,7 @@ __device__ __forceinline__ void k_fin_residual_body(const KryArgs<T>& a, double*
             start_inner(cs, a.ctl, a.ctl.bicg ? sums[12 + c] : sums[6 + c]);
         }
     }
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T, int MODE>
@@ -242,12 +324,12 @@ __device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, const Blk& k_)
     T beta[6], omega[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
-        beta[c] = (T)a.cs[c].beta;
-        omega[c] = (T)a.cs[c].omega;
+        beta[c] = (T)uni(a.cs[c].beta);
+        omega[c] = (T)uni(a.cs[c].omega);
     }
     const T* pOld = q.inner == 1 ? a.r0 : a.p;
     const int64_t N = a.N;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < N; i += (int64_t)k_.G * BLK) {
         T rr[6], pp[6], vv[6];
         ld6(a.r + NCMP * i, rr);
         ld6(pOld + NCMP * i, pp);
@@ -269,10 +351,9 @@ template <class T>
 __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_) {
     const Round rd = round_of(a);
     if (!rd.any) return;
-    const bool start = rd.inner == 0;
-    const T* pv = start ? a.r0 : a.p;
+    const T* pv = rd.inner == 0 ? a.r0 : a.p;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -283,32 +364,13 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_)
         if (r >= a.N) continue;
         T acc[6], rr0[6];
         ld6(pv + (int64_t)NCMP * r, acc);
-        if (start) {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) rr0[c] = acc[c];
-        } else {
-            ld6(a.r0 + (int64_t)NCMP * r, rr0);
-        }
+        ld6(a.r0 + (int64_t)NCMP * r, rr0);
         if (a.dg) {
             const T dgr = (T)a.dg[r];
 #pragma unroll
             for (int c = 0; c < 6; ++c) acc[c] = dgr * acc[c];
         }
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;  // zero in every row of the slice
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            const T av = ld_stream<T>(a.ahat + e);
-            if (av == (T)0) continue;
-            T pc[6];
-            ld6(pv + (int64_t)NCMP * col, pc);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[c] += av * pc[c];
-        }
+        for_entries<ENT<T>>(a, r, a.ahat, [&](const auto& col, const auto& av) { gather<false>(pv, col, av, acc); });
         st6(a.v + (int64_t)NCMP * r, acc);
 #pragma unroll
         for (int c = 0; c < 6; ++c)
@@ -326,21 +388,21 @@ __global__ void __launch_bounds__(BLK) k_kry_v(KryArgs<T> a) {
     k_kry_v_body<T>(a, blk_of_launch(red));
 }
 
-template <class T>
+template <class T, int NT = FBLK>
 __device__ __forceinline__ void k_fin_v_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
     for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
     const int c = threadIdx.x;
-    CompState cs;
+    Comp cs;
     cs.active = 0;
-    if (c < 6) cs = a.cs[c];
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<6>(a.partials, a.G, lds, sums);
+    sum_partials<6, NT>(a.partials, a.G, lds, sums);
     if (!cs.active) return;
     cs.alpha = cs.rho / sums[c];
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T>
@@ -357,11 +419,11 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
     const T* rv = rd.inner == 0 ? a.r0 : a.r;
     T alpha[6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) alpha[c] = (T)a.cs[c].alpha;
+    for (int c = 0; c < 6; ++c) alpha[c] = (T)uni(a.cs[c].alpha);
     T q[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -379,22 +441,8 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
             sv[c] = rr[c] - alpha[c] * vv[c];
             acc[c] = a.dg ? dgr * sv[c] : sv[c];
         }
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;  // zero in every row of the slice
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            const T av = ld_stream<T>(a.ahat + e);
-            if (av == (T)0) continue;
-            T rc[6], vc[6];
-            ld6(rv + (int64_t)NCMP * col, rc);
-            ld6(a.v + (int64_t)NCMP * col, vc);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[c] += av * (rc[c] - alpha[c] * vc[c]);
-        }
+        for_entries<ENT<T, 2>>(a, r, a.ahat,
+                               [&](const auto& col, const auto& av) { gather_s(rv, a.v, alpha, col, av, acc); });
         st6(a.t + (int64_t)NCMP * r, acc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
@@ -416,18 +464,18 @@ __global__ void __launch_bounds__(BLK) k_kry_t(KryArgs<T> a) {
     k_kry_t_body<T>(a, blk_of_launch(red));
 }
 
-template <class T>
+template <class T, int NT = FBLK>
 __device__ __forceinline__ void k_fin_t_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
     for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
     const int c = threadIdx.x;
-    CompState cs;
+    Comp cs;
     cs.active = 0;
-    if (c < 6) cs = a.cs[c];
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<18>(a.partials, a.G, lds, sums);
+    sum_partials<18, NT>(a.partials, a.G, lds, sums);
     if (!cs.active) return;
     const double res = sums[c] / cs.normFactor;
     if (!a.ctl.mixed) cs.finalRes = res;
@@ -436,7 +484,7 @@ __device__ __forceinline__ void k_fin_t_body(const KryArgs<T>& a, double* lds) {
     } else {
         cs.omega = sums[6 + c] / sums[12 + c];
     }
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T>
@@ -456,26 +504,30 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
     const Round rd_ = round_of(a);
     if (!rd_.any) return;
     const bool start = rd_.inner == 0;
+    const T* pv = start ? a.r0 : a.p;
+    const T* rv = start ? a.r0 : a.r;
     bool ex[6];
     double alpha[6], omega[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
-        ex[c] = a.cs[c].exitAtS;
-        alpha[c] = a.cs[c].alpha;
-        omega[c] = a.cs[c].omega;
+        ex[c] = uni(a.cs[c].exitAtS);
+        alpha[c] = uni(a.cs[c].alpha);
+        omega[c] = uni(a.cs[c].omega);
     }
     T q[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
-    for (int64_t it = 0;; ++it) {
-        const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
+    // red-black: the second colour's rows, as the v and t passes take them
+    const int32_t first = a.ctl.rb ? a.nRed : 0, row0 = first & ~(SLICE - 1);
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
+        const int64_t tl = tile_of_g(it, (int64_t)a.N - row0, a.ctl.rb ? 0 : a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
         const int64_t t0 = tl * BLK;
-        const int32_t r = (int32_t)(t0 + k_.tid);
-        if (r >= a.N) continue;
+        const int32_t r = (int32_t)(row0 + t0 + k_.tid);
+        if (r < first || r >= a.N) continue;
         const double rd = a.rM ? a.rM[r] : 1.0;
         const int64_t j = (int64_t)NCMP * r;
         double xv[6];
@@ -493,16 +545,11 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
         } else {
             ld6(a.x + j, xv);
         }
-        ld6(a.r0 + j, rr0);
+        ld6(pv + j, pp);
+        ld6(rv + j, rr);
         ld6(a.v + j, vv);
         ld6(a.t + j, tt);
-        if (start) {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) pp[c] = rr[c] = rr0[c];
-        } else {
-            ld6(a.p + j, pp);
-            ld6(a.r + j, rr);
-        }
+        ld6(a.r0 + j, rr0);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
             if (!rd_.on[c]) continue;
@@ -534,8 +581,11 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
     write_partials<12>(qd, a.partials, k_);
 }
 
+// (FP32: held to the 102 VGPRs of five workgroups a CU, the grid of the solve's
+// passes is the least over them)
 template <class T>
-__global__ void __launch_bounds__(BLK) k_kry_xr(KryArgs<T> a) {
+__global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 4, 8)))
+k_kry_xr(KryArgs<T> a) {
     __shared__ double red[RED_MAX * (BLK / 64)];
     k_kry_xr_body<T>(a, blk_of_launch(red));
 }
@@ -554,7 +604,7 @@ __device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, const Blk& k_) 
         any |= on[c];
     }
     if (!any || inner_running(a)) return;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < a.N; i += (int64_t)k_.G * BLK) {
         double xv[6];
         T ev[6];
         ld6(a.x + NCMP * i, xv);
@@ -571,18 +621,18 @@ __global__ void __launch_bounds__(BLK) k_fold(KryArgs<T> a) {
     k_fold_body<T>(a, blk_of_launch(nullptr));
 }
 
-template <class T>
+template <class T, int NT = FBLK>
 __device__ __forceinline__ void k_fin_xr_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
     for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
     const int c = threadIdx.x;
-    CompState cs;
+    Comp cs;
     cs.active = 0;
-    if (c < 6) cs = a.cs[c];
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<12>(a.partials, a.G, lds, sums);
+    sum_partials<12, NT>(a.partials, a.G, lds, sums);
     if (!cs.active) return;
     cs.iter += 1;
     cs.innerIter += 1;
@@ -627,7 +677,7 @@ __device__ __forceinline__ void k_fin_xr_body(const KryArgs<T>& a, double* lds) 
             cs.converged = conv_outer(cs, a.ctl, cs.finalRes);
         }
     }
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T>
@@ -656,16 +706,16 @@ __global__ void __launch_bounds__(FBLK) k_fin_xr(KryArgs<T> a) {
 // R rows: w = D_R^-1 A_RB Ds^-1 y, y = p (SRC 0) or s = r - alpha v (SRC 1)
 template <class T, int SRC>
 __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) {
-    T* __restrict__ w = SRC == 0 ? a.v : a.t;
+    T* w = SRC == 0 ? a.v : a.t;
     const Round rd = round_of(a);
     if (!rd.any) return;
     const T* pv = rd.inner == 0 ? a.r0 : a.p;
     const T* rv = rd.inner == 0 ? a.r0 : a.r;
     T alpha[6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) alpha[c] = (T)a.cs[c].alpha;
+    for (int c = 0; c < 6; ++c) alpha[c] = (T)uni(a.cs[c].alpha);
     const int64_t n = a.nRed;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -674,29 +724,11 @@ __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) 
         const int32_t r = (int32_t)(tl * BLK + k_.tid);
         if (r >= n) continue;
         T acc[6] = {0, 0, 0, 0, 0, 0};
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;  // zero in every row of the slice
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            const T av = ld_stream<T>(a.ahat + e);
-            if (av == (T)0) continue;
-            if constexpr (SRC == 0) {
-                T pc[6];
-                ld6(pv + (int64_t)NCMP * col, pc);
-#pragma unroll
-                for (int c = 0; c < 6; ++c) acc[c] += av * pc[c];
-            } else {
-                T rc[6], vc[6];
-                ld6(rv + (int64_t)NCMP * col, rc);
-                ld6(a.v + (int64_t)NCMP * col, vc);
-#pragma unroll
-                for (int c = 0; c < 6; ++c) acc[c] += av * (rc[c] - alpha[c] * vc[c]);
-            }
-        }
+        if constexpr (SRC == 0)
+            for_entries<ENT<T>>(a, r, a.ahat, [&](const auto& col, const auto& av) { gather<false>(pv, col, av, acc); });
+        else
+            for_entries<ENT<T, 2>>(a, r, a.ahat,
+                                   [&](const auto& col, const auto& av) { gather_s(rv, a.v, alpha, col, av, acc); });
         st6(w + (int64_t)NCMP * r, acc);
     }
 }
@@ -709,49 +741,30 @@ __global__ void __launch_bounds__(BLK) k_rb_w(KryArgs<T> a) {
 // B rows: v = S M^-1 p = (D_B Ds^-1) p - A_BR w ;  sigma = (r0, v)
 template <class T>
 __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) {
-    const T* __restrict__ w = a.v;
+    const T* w = a.v;
     const Round rd = round_of(a);
     if (!rd.any) return;
-    const bool start = rd.inner == 0;
-    const T* pv = start ? a.r0 : a.p;
+    const T* pv = rd.inner == 0 ? a.r0 : a.p;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    const int64_t n = (int64_t)a.N - a.nRed;
-    for (int64_t it = 0;; ++it) {
+    const int32_t r0b = a.nRed & ~(SLICE - 1);  // wavefronts on whole slices
+    const int64_t n = (int64_t)a.N - r0b;
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(a.nRed + tl * BLK + k_.tid);
-        if (r >= a.N) continue;
+        const int32_t r = (int32_t)(r0b + tl * BLK + k_.tid);
+        if (r < a.nRed || r >= a.N) continue;
         T acc[6], rr0[6];
         ld6(pv + (int64_t)NCMP * r, acc);
-        if (start) {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) rr0[c] = acc[c];
-        } else {
-            ld6(a.r0 + (int64_t)NCMP * r, rr0);
-        }
+        ld6(a.r0 + (int64_t)NCMP * r, rr0);
         if (a.dg) {
             const T dgr = (T)a.dg[r];
 #pragma unroll
             for (int c = 0; c < 6; ++c) acc[c] = dgr * acc[c];
         }
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            const T av = ld_stream<T>(a.ahat + e);
-            if (av == (T)0) continue;
-            T wc[6];
-            ld6(w + (int64_t)NCMP * col, wc);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[c] -= av * wc[c];
-        }
+        for_entries<ENT<T>>(a, r, a.ahat, [&](const auto& col, const auto& av) { gather<true>(w, col, av, acc); });
         st6(a.v + (int64_t)NCMP * r, acc);
 #pragma unroll
         for (int c = 0; c < 6; ++c)
@@ -773,25 +786,26 @@ __global__ void __launch_bounds__(BLK) k_rb_v(KryArgs<T> a) {
 // |s|, (t, s), (t, t)
 template <class T>
 __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) {
-    const T* __restrict__ w = a.t;
+    const T* w = a.t;
     const Round rd = round_of(a);
     if (!rd.any) return;
     const T* rv = rd.inner == 0 ? a.r0 : a.r;
     T alpha[6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) alpha[c] = (T)a.cs[c].alpha;
+    for (int c = 0; c < 6; ++c) alpha[c] = (T)uni(a.cs[c].alpha);
     T q[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
-    const int64_t n = (int64_t)a.N - a.nRed;
-    for (int64_t it = 0;; ++it) {
+    const int32_t r0b = a.nRed & ~(SLICE - 1);  // wavefronts on whole slices
+    const int64_t n = (int64_t)a.N - r0b;
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
             continue;
         }
-        const int32_t r = (int32_t)(a.nRed + tl * BLK + k_.tid);
-        if (r >= a.N) continue;
+        const int32_t r = (int32_t)(r0b + tl * BLK + k_.tid);
+        if (r < a.nRed || r >= a.N) continue;
         T sv[6], acc[6], rr[6], vv[6];
         ld6(rv + (int64_t)NCMP * r, rr);
         ld6(a.v + (int64_t)NCMP * r, vv);
@@ -801,21 +815,7 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) 
             sv[c] = rr[c] - alpha[c] * vv[c];
             acc[c] = a.dg ? dgr * sv[c] : sv[c];
         }
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            const T av = ld_stream<T>(a.ahat + e);
-            if (av == (T)0) continue;
-            T wc[6];
-            ld6(w + (int64_t)NCMP * col, wc);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[c] -= av * wc[c];
-        }
+        for_entries<ENT<T>>(a, r, a.ahat, [&](const auto& col, const auto& av) { gather<true>(w, col, av, acc); });
         st6(a.t + (int64_t)NCMP * r, acc);
 #pragma unroll
         for (int c = 0; c < 6; ++c) {
@@ -850,7 +850,7 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, const Blk
     }
     if (!any || inner_running(a)) return;
     const int64_t n = a.nRed;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -860,21 +860,7 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, const Blk
         if (r >= n) continue;
         double acc[6];
         ld6(a.b + (int64_t)NCMP * r, acc);
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            if (k < 32 && !((live >> k) & 1u)) continue;
-            const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t col = a.ellCol[e];
-            const double av = a.aval[e];
-            if (av == 0.0) continue;
-            double xc[6];
-            ld6(a.x + (int64_t)NCMP * col, xc);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[c] -= av * xc[c];
-        }
+        for_entries<ENT<double>>(a, r, a.aval, [&](const auto& col, const auto& av) { gather<true>(a.x, col, av, acc); });
         double xv[6];
         ld6(a.x + (int64_t)NCMP * r, xv);
         const double rd = a.rD[r];
@@ -888,27 +874,6 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, const Blk
 template <class T>
 __global__ void __launch_bounds__(BLK) k_rb_backsub(KryArgs<T> a) {
     k_rb_backsub_body<T>(a, blk_of_launch(nullptr));
-}
-
-// ahat of the red-black solve: A_jk / (D_j Ds_k) on R's rows, A_ij on B's
-template <class T>
-__global__ void k_rb_scale(int32_t N, int32_t nRed, const int64_t* __restrict__ off,
-                           const int32_t* __restrict__ width, const uint32_t* __restrict__ slotMask,
-                           const int32_t* __restrict__ col, const double* __restrict__ aval,
-                           const double* __restrict__ rD, const double* __restrict__ rDs, T* __restrict__ ahat) {
-    const int64_t r = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (r >= N) return;
-    const int s = (int)(r >> 6), lane = (int)(r & 63);
-    const int64_t base = off[s] + lane;
-    const int w = width[s];
-    const uint32_t live = slotMask ? slotMask[s] : 0xffffffffu;
-    const bool red = r < nRed;
-    const double rdr = red ? rD[r] : 1.0;
-    for (int k = 0; k < w; ++k) {
-        if (k < 32 && !((live >> k) & 1u)) continue;
-        const int64_t e = base + (int64_t)SLICE * k;
-        ahat[e] = red ? (T)((aval[e] * rdr) * rDs[col[e]]) : (T)aval[e];
-    }
 }
 
 // Pivots of B for a general LDU matrix (the sparseSolver surface):
@@ -962,7 +927,7 @@ __device__ __forceinline__ void k_bicg_init_body(const KryArgs<T>& a, const Blk&
     }
     if (!any) return;
     double q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -975,19 +940,9 @@ __device__ __forceinline__ void k_bicg_init_body(const KryArgs<T>& a, const Blk&
         ld6(a.x + (int64_t)NCMP * r, xv);
 #pragma unroll
         for (int c = 0; c < 6; ++c) y[c] = d * xv[c];
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        for (int k = 0; k < width; ++k) {
-            const int64_t e = base + (int64_t)SLICE * k;
-            const double av = a.atval[e];
-            if (av == 0.0) continue;
-            const int32_t col = a.ellCol[e];
-            double xc[6];
-            ld6(a.x + (int64_t)NCMP * col, xc);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) y[c] += av * xc[c];
-        }
+        KryArgs<T> at = a;
+        at.slotMask = nullptr;
+        for_entries<ENT<double>>(at, r, a.atval, [&](const auto& col, const auto& av) { gather<false>(a.x, col, av, y); });
         double bb[6];
         ld6(a.b + (int64_t)NCMP * r, bb);
         T rA[6], rT[6];
@@ -1009,21 +964,21 @@ __global__ void __launch_bounds__(BLK) k_bicg_init(KryArgs<T> a) {
     k_bicg_init_body<T>(a, blk_of_launch(red));
 }
 
-template <class T>
+template <class T, int NT = FBLK>
 __device__ __forceinline__ void k_fin_bicg_init_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
     for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
     const int c = threadIdx.x;
-    CompState cs;
+    Comp cs;
     cs.active = 0;
-    if (c < 6) cs = a.cs[c];
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<6>(a.partials, a.G, lds, sums);
+    sum_partials<6, NT>(a.partials, a.G, lds, sums);
     if (!cs.active) return;
     cs.rho = sums[c];
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T>
@@ -1046,7 +1001,7 @@ __device__ __forceinline__ void k_bicg_p_body(const KryArgs<T>& a, const Blk& k_
         any |= on[c];
     }
     if (!any) return;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < a.N; i += (int64_t)k_.G * BLK) {
         const T rm = a.rM ? (T)a.rM[i] : (T)1;
         T rA[6], rT[6], pA[6], pT[6];
         ld6(a.r + NCMP * i, rA);
@@ -1082,7 +1037,7 @@ __device__ __forceinline__ void k_bicg_w_body(const KryArgs<T>& a, const Blk& k_
     }
     if (!any) return;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1099,29 +1054,10 @@ __device__ __forceinline__ void k_bicg_w_body(const KryArgs<T>& a, const Blk& k_
             wA[c] = d * wA[c];
             wT[c] = d * pT[c];
         }
-        const int s = r >> 6, lane = r & 63;
-        const int64_t base = a.ellOff[s] + lane;
-        const int width = a.ellWidth[s];
-        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
-        for (int k = 0; k < width; ++k) {
-            const int64_t e = base + (int64_t)SLICE * k;
-            const T av = (k < 32 && !((live >> k) & 1u)) ? (T)0 : ld_stream<T>(a.aA + e);
-            const T at = ld_stream<T>(a.aT + e);
-            if (av == (T)0 && at == (T)0) continue;
-            const int32_t col = ld_stream<T>(a.ellCol + e);
-            if (av != (T)0) {
-                T pc[6];
-                ld6(a.p + (int64_t)NCMP * col, pc);
-#pragma unroll
-                for (int c = 0; c < 6; ++c) wA[c] += av * pc[c];
-            }
-            if (at != (T)0) {
-                T pc[6];
-                ld6(a.v + (int64_t)NCMP * col, pc);
-#pragma unroll
-                for (int c = 0; c < 6; ++c) wT[c] += at * pc[c];
-            }
-        }
+        for_entries<ENT<T>>(a, r, a.aA, [&](const auto& col, const auto& av) { gather<false>(a.p, col, av, wA); });
+        KryArgs<T> at = a;
+        at.slotMask = nullptr;
+        for_entries<ENT<T>>(at, r, a.aT, [&](const auto& col, const auto& av) { gather<false>(a.v, col, av, wT); });
         st6(a.t + (int64_t)NCMP * r, wA);
         st6(a.s + (int64_t)NCMP * r, wT);
 #pragma unroll
@@ -1140,18 +1076,18 @@ __global__ void __launch_bounds__(BLK) k_bicg_w(KryArgs<T> a) {
     k_bicg_w_body<T>(a, blk_of_launch(red));
 }
 
-template <class T>
+template <class T, int NT = FBLK>
 __device__ __forceinline__ void k_fin_bicg_w_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
     for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
     const int c = threadIdx.x;
-    CompState cs;
+    Comp cs;
     cs.active = 0;
-    if (c < 6) cs = a.cs[c];
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<6>(a.partials, a.G, lds, sums);
+    sum_partials<6, NT>(a.partials, a.G, lds, sums);
     if (!cs.active) return;
     // checkSingularity(mag(wApT)/normFactor): stop; restarted from the
     // true residual as after a PBiCGStab breakdown
@@ -1163,7 +1099,7 @@ __device__ __forceinline__ void k_fin_bicg_w_body(const KryArgs<T>& a, double* l
     } else {
         cs.alpha = cs.rho / sums[c];
     }
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T>
@@ -1190,7 +1126,7 @@ __device__ __forceinline__ void k_bicg_xr_body(const KryArgs<T>& a, const Blk& k
     T q[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1245,18 +1181,18 @@ __global__ void __launch_bounds__(BLK) k_bicg_xr(KryArgs<T> a) {
     k_bicg_xr_body<T>(a, blk_of_launch(red));
 }
 
-template <class T>
+template <class T, int NT = FBLK>
 __device__ __forceinline__ void k_fin_bicg_xr_body(const KryArgs<T>& a, double* lds) {
     bool any = false;
 #pragma unroll
     for (int i = 0; i < 6; ++i) any |= a.cs[i].active != 0;
     if (!any) return;
     const int c = threadIdx.x;
-    CompState cs;
+    Comp cs;
     cs.active = 0;
-    if (c < 6) cs = a.cs[c];
+    if (c < 6) cs.load(a.cs[c]);
     double* sums;
-    sum_partials<12>(a.partials, a.G, lds, sums);
+    sum_partials<12, NT>(a.partials, a.G, lds, sums);
     if (!cs.active) return;
     cs.iter += 1;
     cs.innerIter += 1;
@@ -1285,7 +1221,7 @@ __device__ __forceinline__ void k_fin_bicg_xr_body(const KryArgs<T>& a, double* 
             cs.converged = conv_outer(cs, a.ctl, cs.finalRes);
         }
     }
-    a.cs[c] = cs;
+    cs.store(a.cs[c]);
 }
 
 template <class T>
@@ -1309,20 +1245,28 @@ __global__ void k_rdiag(int32_t N, const double* __restrict__ diag, double* __re
     if (r < N) rD[r] = 1.0 / diag[r];
 }
 template <class T>
-__global__ void k_scale(int32_t N, const int64_t* __restrict__ off, const int32_t* __restrict__ width,
-                        const uint32_t* __restrict__ slotMask, const int32_t* __restrict__ col,
-                        const double* __restrict__ aval, const double* __restrict__ rD, T* __restrict__ ahat) {
-    const int64_t r = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (r >= N) return;
-    const int s = (int)(r >> 6), lane = (int)(r & 63);
-    const int64_t base = off[s] + lane;
-    const int w = width[s];
-    const uint32_t live = slotMask ? slotMask[s] : 0xffffffffu;
-    for (int k = 0; k < w; ++k) {
-        if (k < 32 && !((live >> k) & 1u)) continue;
-        const int64_t e = base + (int64_t)SLICE * k;
-        ahat[e] = rD ? (T)(aval[e] * rD[col[e]]) : (T)aval[e];
+__device__ __forceinline__ void k_scale_body(const KryArgs<T>& a, const Blk& k_) {
+    T* ahat = const_cast<T*>(a.ahat);
+    for (int64_t r = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && r < a.N; r += (int64_t)k_.G * BLK) {
+        const int s = (int)(r >> 6), lane = (int)(r & 63);
+        const int64_t base = a.ellOff[s] + lane;
+        const int w = a.ellWidth[s];
+        const uint32_t live = a.slotMask ? a.slotMask[s] : 0xffffffffu;
+        // red-black: A_jk / (D_j Ds_k) on the first colour's rows, A_ij on the second's
+        const bool red = r < a.nRed;
+        const double rdr = a.ctl.rb && red ? a.rD[r] : 1.0;
+        for (int k = 0; k < w; ++k) {
+            if (k < 32 && !((live >> k) & 1u)) continue;
+            const int64_t e = base + (int64_t)SLICE * k;
+            const double av = a.aval[e];
+            if (a.ctl.rb) ahat[e] = red ? (T)((av * rdr) * a.rM[a.ellCol[e]]) : (T)av;
+            else ahat[e] = a.rM ? (T)(av * a.rM[a.ellCol[e]]) : (T)av;
+        }
     }
+}
+template <class T>
+__global__ void __launch_bounds__(BLK) k_scale(KryArgs<T> a) {
+    k_scale_body<T>(a, blk_of_launch(nullptr));
 }
 
 // ---- mean of x per component (normalisation factor's gAverage(psi)) ---------
@@ -1351,6 +1295,631 @@ __global__ void __launch_bounds__(FBLK) k_fin_mean6(int32_t N, int G, const doub
     double* sums;
     sum_partials<6>(partials, G, lds, sums);
     if (threadIdx.x < 6) cs[threadIdx.x].xbar = sums[threadIdx.x] / N;
+}
+
+// ============================================ resident solve (small meshes)
+// The whole solve in one launch.  On a mesh of some ten thousand cells a pass
+// is a few microseconds of dependent loads and a launch costs as much again; a
+// 128 x 128 channel's step spent two thirds of its time in the solve's 38
+// launches and five host round trips.  Here P workgroups of RBLK threads stay
+// for the solve: each runs the row kernels' bodies for its share of their
+// workgroups (the same tiles, the same partial sums), a barrier between the
+// passes replaces the launch, and every workgroup finalizes each reduction by
+// itself on its own copy of the component records, so all take the same
+// branches without asking the host.  The fields are the bits the launches give.
+//
+// The barrier is one of the XCDs' own (an atomic in the L2 its workgroups share)
+// and, where the workgroups are on several XCDs, one of their last arrivals:
+// those alone write their L2 back (release) and drop what it holds of the others'
+// (acquire).  As one counter for all, with every workgroup fencing, a barrier of
+// 98 workgroups took 4.7 us.  A solve that fits one XCD (workgroups are dealt
+// round-robin over the eight, so every eighth one of the grid takes part) needs
+// no L2 traffic at all.  Where each workgroup runs is read from the hardware.
+//
+// A workgroup is one tile of BLK rows, so that few waves share a SIMD: a pass of
+// one row a thread is bound by instruction issue and latency (512 threads took
+// 2.6 us for the x/r pass, 256 take 1.2 us).
+//
+// The barrier needs the workgroups resident together: no more are launched than
+// fit, but other streams and processes may hold the CUs, so the wait is bounded:
+// a workgroup that polls maxPolls times sets the top bit of the counters and
+// leaves, which the others see in their own waits.  The records on the device
+// and the saved vectors then still hold the solve's start, and the host runs it
+// by launches.
+constexpr int RBLK = 256, RSUB = RBLK / BLK;
+constexpr int XCDS = 8;
+// workgroups a CU holds: FP32 solves are held to 256 registers a lane for two,
+// FP64 ones take up to 350 (held to 256 they spill, and a 128 x 128 channel's
+// step took 200 us instead of 179)
+template <class T>
+constexpr int RES_PER_CU = sizeof(T) == 4 ? 2 : 1;
+constexpr uint32_t RES_FAIL = 0x80000000u;
+
+template <class T>
+struct ResArgs {
+    KryArgs<T> a, b, s;   // all rows; red-black: the second colour's rows, its sweep residual
+    int32_t P, pg, Gw;    // workgroups; row-kernel workgroups of the pointwise and first-colour passes
+    int32_t X;            // row-kernel workgroups with a tile: the first X of a.G
+    int32_t doScale;
+    uint32_t maxPolls;
+    SolveState* st;
+    // NULL when P = 1: x [N][6], and where the assembly's residual starts the
+    // solve (not red-black, whose first sweep makes it) r0 and PBiCG's r
+    double* xSave;
+};
+
+struct ResBar {
+    SolveState* st;
+    int P, nXcd, nHere;    // workgroups; XCDs they are on; workgroups on this one
+    uint32_t* here;        // this XCD's counters: arrivals, barriers passed, departures
+    uint32_t maxPolls, ph, one;  // ph: barriers so far; one: 1, unknown to the compiler
+    int* bad;
+};
+template <int SCOPE>
+__device__ __forceinline__ uint32_t at_add(uint32_t* p, uint32_t v) {
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, SCOPE);
+}
+// Polls *p (an atomic add of 0: L2 executes it, no L1 copy is read) until its low
+// bits reach target; returns with RES_FAIL set if a wait gave up, this or another
+template <int SCOPE>
+__device__ __forceinline__ uint32_t res_poll(uint32_t* p, uint32_t v, uint32_t target, const ResBar& B) {
+    for (uint32_t n = 0; v < target;) {
+        if (++n > B.maxPolls) return __hip_atomic_fetch_or(p, RES_FAIL, __ATOMIC_RELAXED, SCOPE) | RES_FAIL;
+        __builtin_amdgcn_s_sleep(1);
+        v = at_add<SCOPE>(p, B.one - 1u);
+    }
+    return v;
+}
+// Before the first pass: counts the workgroups on each XCD and waits for all of
+// them, with a counter of its own and every workgroup fencing.
+__device__ __forceinline__ bool res_enter(ResBar& B) {
+    if (B.P == 1) {
+        __syncthreads();
+        return true;
+    }
+    constexpr int AG = __HIP_MEMORY_SCOPE_AGENT;
+    const uint32_t x = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7u;  // hwreg XCC_ID, bits 0..3
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        at_add<AG>(&B.st->bar[8 + x], 1u);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        const uint32_t v = res_poll<AG>(B.st->bar, at_add<AG>(B.st->bar, 1u) + 1u, (uint32_t)B.P, B);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        *B.bad = ((v | at_add<AG>(B.st->bar, B.one - 1u)) & RES_FAIL) != 0;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __syncthreads();
+    B.nXcd = 0;
+    for (int i = 0; i < XCDS; ++i)
+        B.nXcd += __hip_atomic_load(&B.st->bar[8 + i], __ATOMIC_RELAXED, AG) != 0;
+    B.nHere = (int)__hip_atomic_load(&B.st->bar[8 + x], __ATOMIC_RELAXED, AG);
+    B.here = B.st->barL2[x];
+    return *B.bad == 0;
+}
+// Every wave's stores have reached its L2 before the first wave arrives; no wave
+// goes on before that one has dropped the CU's L1 (the load after the fence
+// returns behind it).
+__device__ __forceinline__ bool res_barrier(ResBar& B) {
+    if (B.P == 1) {
+        __syncthreads();
+        return true;
+    }
+    constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP, AG = __HIP_MEMORY_SCOPE_AGENT;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    ++B.ph;
+    if (threadIdx.x == 0) {
+        uint32_t v = at_add<WG>(&B.here[0], B.one) + 1u;
+        const uint32_t full = B.ph * (uint32_t)B.nHere;
+        if (B.nXcd == 1) {
+            v = res_poll<WG>(&B.here[0], v, full, B);
+        } else if (v == full) {
+            v = 0;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            uint32_t* g = &B.st->bar[2];
+            v = res_poll<AG>(g, at_add<AG>(g, 1u) + 1u, B.ph * (uint32_t)B.nXcd, B);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            v |= at_add<AG>(g, B.one - 1u);
+            v = at_add<WG>(&B.here[1], (v & RES_FAIL) + B.one) | (v & RES_FAIL);
+        } else {
+            v = res_poll<WG>(&B.here[1], at_add<WG>(&B.here[1], B.one - 1u), B.ph, B);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        v |= at_add<WG>(&B.here[B.nXcd == 1 ? 0 : 1], B.one - 1u);
+        *B.bad = (v & RES_FAIL) != 0;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __syncthreads();
+    return *B.bad == 0;
+}
+// Past the last barrier: the last workgroup of an XCD, and the last of all, leave
+// their counters at zero for the next launch.
+__device__ __forceinline__ void res_leave(ResBar& B) {
+    if (B.P == 1 || threadIdx.x != 0) return;
+    constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP, AG = __HIP_MEMORY_SCOPE_AGENT;
+    if (at_add<WG>(&B.here[2], B.one) + 1u == (uint32_t)B.nHere)
+        for (int i = 0; i < 3; ++i) (void)__hip_atomic_exchange(&B.here[i], 0u, __ATOMIC_RELAXED, WG);
+    if (at_add<AG>(&B.st->bar[1], 1u) + 1u == (uint32_t)B.P)
+        for (int i = 0; i < 8 + XCDS; ++i) __hip_atomic_store(&B.st->bar[i], 0u, __ATOMIC_RELAXED, AG);
+}
+
+// RF_RB_ROW, RF_BICG_ROW: every thread keeps one row (red-black: one of each
+// colour) for the whole solve, its matrix entries and its words of the vectors
+// in registers, and only the vectors that other rows gather go to memory.
+enum ResForm { RF_JACOBI = 0, RF_REDBLACK = 1, RF_BICG = 2, RF_RB_ROW = 3, RF_BICG_ROW = 4 };
+constexpr int ROW_W = 6;  // entries of a kept row
+
+// A row of a [N][6] vector by its byte offset: 32 bits (a resident mesh has at
+// most RES_MAX_ROWS rows), so that an address is a scalar base and one register.
+template <class T>
+__device__ __forceinline__ uint32_t row_off(int32_t r) {
+    return (uint32_t)r * (uint32_t)(NCMP * sizeof(T));
+}
+template <class T>
+__device__ __forceinline__ const T* at_off(const T* p, uint32_t off) {
+    return reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + off);
+}
+template <class T>
+__device__ __forceinline__ T* at_off(T* p, uint32_t off) {
+    return reinterpret_cast<T*>(reinterpret_cast<char*>(p) + off);
+}
+
+// the entries of a kept row in column order; 0 where there is none
+template <class T>
+struct RowEnts {
+    uint32_t off[ROW_W];  // of the column's row
+    T val[ROW_W];
+    // SCALE 0: vals as they are; 1, 2: the FP64 matrix scaled for the red-black
+    // solve's first, second colour (k_scale_body's arithmetic)
+    template <int SCALE, class V>
+    __device__ __forceinline__ void load(const KryArgs<T>& a, int32_t r, const V* vals, bool masked) {
+        const int s = r >= 0 ? r >> 6 : 0;
+        const int64_t base = a.ellOff[s] + (r & 63);
+        const int width = r >= 0 ? a.ellWidth[s] : 0;
+        const uint32_t live = masked && a.slotMask ? a.slotMask[s] : 0xffffffffu;
+        V v[ROW_W];
+        int32_t col[ROW_W];
+#pragma unroll
+        for (int k = 0; k < ROW_W; ++k) {
+            col[k] = 0;
+            v[k] = (V)0;
+            if (k < width && ((live >> k) & 1u)) {
+                const int64_t e = base + (int64_t)SLICE * k;
+                col[k] = a.ellCol[e];
+                v[k] = vals[e];
+            }
+        }
+        if constexpr (SCALE == 1) {
+            const double rdr = r >= 0 ? a.rD[r] : 1.0;
+            double m[ROW_W];
+#pragma unroll
+            for (int k = 0; k < ROW_W; ++k) m[k] = v[k] != (V)0 ? a.rM[col[k]] : 0.0;
+#pragma unroll
+            for (int k = 0; k < ROW_W; ++k) val[k] = (T)((v[k] * rdr) * m[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < ROW_W; ++k) val[k] = (T)v[k];
+        }
+#pragma unroll
+        for (int k = 0; k < ROW_W; ++k) off[k] = row_off<T>(col[k]);
+    }
+    // acc += val src[col] (NEG: -=), three rows in flight
+    template <bool NEG>
+    __device__ __forceinline__ void gather(const T* src, T (&acc)[6]) const {
+#pragma unroll
+        for (int k0 = 0; k0 < ROW_W; k0 += 3) {
+            T g[3][6];
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (val[k0 + j] != (T)0) ld6(at_off(src, off[k0 + j]), g[j]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (val[k0 + j] != (T)0) {
+                    const T v = val[k0 + j];
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) acc[c] = NEG ? acc[c] - v * g[j][c] : acc[c] + v * g[j][c];
+                }
+        }
+    }
+    // the same of s = r - alpha v
+    __device__ __forceinline__ void gather_s(const T* rv, const T* vv, const T (&alpha)[6], T (&acc)[6]) const {
+#pragma unroll
+        for (int k0 = 0; k0 < ROW_W; k0 += 3) {
+            T g[3][6], h[3][6];
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (val[k0 + j] != (T)0) {
+                    ld6(at_off(rv, off[k0 + j]), g[j]);
+                    ld6(at_off(vv, off[k0 + j]), h[j]);
+                }
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (val[k0 + j] != (T)0) {
+                    const T v = val[k0 + j];
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) acc[c] += v * (g[j][c] - alpha[c] * h[j][c]);
+                }
+        }
+    }
+};
+
+template <class T, int FORM>
+__device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
+    constexpr bool RB = FORM == RF_REDBLACK || FORM == RF_RB_ROW, BICG = FORM == RF_BICG || FORM == RF_BICG_ROW;
+    constexpr bool MIX = std::is_same<T, float>::value;
+    __shared__ CompState cs[6];
+    __shared__ double lds[FIN_LDS];
+    __shared__ double red[RSUB][RED_MAX * (BLK / 64)];
+    __shared__ int bad;
+    const int sub = threadIdx.x / BLK, tid = threadIdx.x % BLK, P = m.P;
+    for (int i = threadIdx.x; i < (int)(sizeof(cs) / 8); i += RBLK)
+        reinterpret_cast<double*>(cs)[i] = reinterpret_cast<const double*>(m.a.cs)[i];
+    __syncthreads();
+    KryArgs<T> a = m.a, b = m.b, sw = m.s;
+    a.cs = b.cs = sw.cs = cs;
+    // the x/r pass has partial sums of its own: the t pass's may still be read
+    KryArgs<T> ax = a, af = a;
+    ax.partials = af.partials = a.partials + (int64_t)24 * a.G;
+    // the finalizers sum the workgroups that have a tile: the others add zeros
+    KryArgs<T> an = a;
+    an.G = af.G = m.X;
+    ResBar bar{m.st, P, 1, P, nullptr, m.maxPolls, 0, (uint32_t)(m.P > 0), &bad};
+    auto wait = [&] { return res_barrier(bar); };
+    // one pass of the row kernels: workgroups 0 .. X-1 of G, RSUB at a time
+    auto passOf = [&](int X, int G, auto&& body) {
+        for (int v0 = p * RSUB; v0 < X; v0 += P * RSUB) {
+            body(Blk{v0 + sub < X ? G : 0, v0 + sub, tid, red[sub]});
+            if (X > P * RSUB) __syncthreads();  // the partial-sum slots are used again
+        }
+    };
+    auto pass = [&](int G, auto&& body) { passOf(min(G, m.X), G, body); };
+    auto passAll = [&](int G, auto&& body) { passOf(G, G, body); };
+    const int X0 = P * RSUB;
+    if (m.xSave) {
+        const int64_t n6 = (int64_t)NCMP * a.N;
+        for (int64_t i = (int64_t)p * RBLK + threadIdx.x; i < n6; i += (int64_t)P * RBLK) {
+            m.xSave[i] = a.x[i];
+            if constexpr (!RB) reinterpret_cast<T*>(m.xSave + n6)[i] = a.r0[i];
+            if constexpr (BICG) reinterpret_cast<T*>(m.xSave + 2 * n6)[i] = a.r[i];
+        }
+    }
+    if (m.doScale && FORM < RF_RB_ROW) {
+        if constexpr (BICG) {
+            // the float copies of A and A^T, by rows
+            if constexpr (MIX)
+                for (int64_t r = (int64_t)p * RBLK + threadIdx.x; r < a.N; r += (int64_t)P * RBLK) {
+                    const int64_t base = a.ellOff[r >> 6] + (r & 63);
+                    for (int k = 0; k < a.ellWidth[r >> 6]; ++k) {
+                        const int64_t e = base + (int64_t)SLICE * k;
+                        const_cast<T*>(a.aA)[e] = (T)a.aval[e];
+                        const_cast<T*>(a.aT)[e] = (T)a.atval[e];
+                    }
+                }
+        } else {
+            passAll(X0, [&](const Blk& k) { k_scale_body<T>(a, k); });
+        }
+    }
+    bool ok = res_enter(bar);
+    // the kept rows: tile p RSUB + sub of the rows (red-black: of each colour)
+    constexpr bool ROW = FORM == RF_RB_ROW || FORM == RF_BICG_ROW;
+    const Blk kRow{p * RSUB + sub < m.X ? a.G : 0, p * RSUB + sub, tid, red[sub]};
+    int32_t rR = -1, rB = -1;
+    RowEnts<T> eR, eB;  // red-black: the first and the second colour's row; PBiCG: A^T's and A's
+    T w0[6], wr[6], wp[6], wv[6], dgB = (T)1;
+    using XT = std::conditional_t<MIX, float, double>;
+    XT X[6];
+    double rdB = 1.0;
+    uint32_t oR = 0, oB = 0;
+    if constexpr (ROW) {
+        const int64_t i = (int64_t)(p * RSUB + sub) * BLK + tid;
+        if constexpr (RB) {
+            const int64_t rb = (a.nRed & ~(SLICE - 1)) + i;
+            if (i < a.nRed) rR = (int32_t)i;
+            if (rb >= a.nRed && rb < a.N) rB = (int32_t)rb;
+            eR.template load<1>(a, rR, a.aval, true);
+            eB.template load<2>(a, rB, a.aval, true);
+            if (rB >= 0 && a.dg) dgB = (T)a.dg[rB];
+        } else {
+            if (i < a.N) rB = (int32_t)i;
+            // the FP32 solve's float copies of A and A^T are made here
+            eB.template load<0>(a, rB, a.aval, true);
+            eR.template load<0>(a, rB, a.atval, false);
+            if (rB >= 0) dgB = (T)a.diag[rB];
+        }
+        if (rB >= 0 && a.rM) rdB = a.rM[rB];
+        if (rR >= 0) oR = row_off<T>(rR);
+        if (rB >= 0) oB = row_off<T>(rB);
+#pragma unroll
+        for (int c = 0; c < 6; ++c) w0[c] = wr[c] = wp[c] = wv[c] = (T)0, X[c] = 0;
+    }
+    for (int round = 0; ok && round < 100000; ++round) {
+        bool act = false, ref = false, fold = false;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            if (a.valid[c] <= 0) continue;
+            act |= cs[c].active != 0;
+            ref |= cs[c].needRefine != 0;
+            fold |= cs[c].needRefine && cs[c].foldE;
+        }
+        if (!act && !ref) break;
+        if (!act) {
+            if (fold) {
+                passAll(m.pg, [&](const Blk& k) { k_fold_body<T>(RB ? b : a, k); });
+                ok = wait();
+            }
+            if constexpr (RB) {
+                if (ok) {
+                    pass(m.Gw, [&](const Blk& k) { k_rb_backsub_body<T>(a, k); });
+                    ok = wait();
+                }
+            }
+            if (!ok) break;
+            pass(a.G, [&](const Blk& k) { k_residual_body<T, 1>(RB ? sw : a, k); });
+            ok = wait();
+            if (!ok) break;
+            k_fin_residual_body<T, 1, RBLK>(an, lds);
+            __syncthreads();
+            continue;
+        }
+        if constexpr (FORM == RF_RB_ROW) {
+            const Round rd = round_of(a);
+            const bool start = rd.inner == 0;
+            const T* pv = start ? a.r0 : a.p;
+            const T* rv = start ? a.r0 : a.r;
+            if (start) {
+                if (rB >= 0) ld6(at_off(a.r0, oB), w0);
+                if constexpr (!MIX)
+                    if (rB >= 0) ld6(at_off(a.x, oB), X);
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    wr[c] = wp[c] = w0[c];
+                    if constexpr (MIX) X[c] = 0.0f;
+                }
+            } else {
+                T be[6], om[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    be[c] = (T)uni(cs[c].beta);
+                    om[c] = (T)uni(cs[c].omega);
+                }
+#pragma unroll
+                for (int c = 0; c < 6; ++c)
+                    if (rd.on[c]) wp[c] = wr[c] + be[c] * (wp[c] - om[c] * wv[c]);
+                if (rB >= 0) st6(at_off(a.p, oB), wp);
+                ok = wait();
+                if (!ok) break;
+            }
+            {
+                T acc[6] = {0, 0, 0, 0, 0, 0};
+                eR.template gather<false>(pv, acc);
+                if (rR >= 0) st6(at_off(a.v, oR), acc);
+            }
+            ok = wait();
+            if (!ok) break;
+            {
+#pragma unroll
+                for (int c = 0; c < 6; ++c) wv[c] = a.dg ? dgB * wp[c] : wp[c];
+                eB.template gather<true>(a.v, wv);
+                double q[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) q[c] = rd.on[c] && rB >= 0 ? (T)0 + w0[c] * wv[c] : (T)0;
+                if (rB >= 0) st6(at_off(a.v, oB), wv);
+                write_partials<6>(q, a.partials, kRow);
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_v_body<T, RBLK>(an, lds);
+            __syncthreads();
+            T al[6];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) al[c] = (T)uni(cs[c].alpha);
+            {
+                T acc[6] = {0, 0, 0, 0, 0, 0};
+                eR.gather_s(rv, a.v, al, acc);
+                if (rR >= 0) st6(at_off(a.t, oR), acc);
+            }
+            ok = wait();
+            if (!ok) break;
+            T wt[6];
+            {
+                T sv[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    sv[c] = wr[c] - al[c] * wv[c];
+                    wt[c] = a.dg ? dgB * sv[c] : sv[c];
+                }
+                eB.template gather<true>(a.t, wt);
+                double q[18];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    const bool o = rd.on[c] && rB >= 0;
+                    q[c] = o ? (T)fabs(sv[c]) : (T)0;
+                    q[6 + c] = o ? (T)0 + wt[c] * sv[c] : (T)0;
+                    q[12 + c] = o ? (T)0 + wt[c] * wt[c] : (T)0;
+                }
+                write_partials<18>(q, a.partials, kRow);
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_t_body<T, RBLK>(an, lds);
+            __syncthreads();
+            {
+                double q[12], alphas[6], omegas[6];
+                bool ex[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    alphas[c] = uni(cs[c].alpha);
+                    omegas[c] = uni(cs[c].omega);
+                    ex[c] = uni(cs[c].exitAtS);
+                }
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    q[c] = q[6 + c] = (T)0;
+                    if (!rd.on[c]) continue;
+                    const double alpha = alphas[c], omega = omegas[c];
+                    double xv = X[c];
+                    const double y = rdB * (double)wp[c];
+                    if (ex[c]) {
+                        xv += alpha * y;
+                    } else {
+                        const T sv = wr[c] - (T)alpha * wv[c];
+                        const double z = rdB * (double)sv;
+                        xv += alpha * y + omega * z;
+                        const T rn = sv - (T)omega * wt[c];
+                        wr[c] = rn;
+                        if (rB >= 0) {
+                            q[c] = (T)fabs(rn);
+                            q[6 + c] = (T)0 + w0[c] * rn;
+                        }
+                    }
+                    X[c] = (XT)xv;
+                }
+                if (rB >= 0) {
+                    st6(at_off(a.r, oB), wr);
+                    if constexpr (MIX) st6(at_off(a.e, oB), X);
+                    else st6(at_off(a.x, oB), X);
+                }
+                write_partials<12>(q, af.partials, kRow);
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_xr_body<T, RBLK>(af, lds);
+            __syncthreads();
+        } else if constexpr (FORM == RF_BICG_ROW) {
+            const Round rd = round_of(a);
+            const bool start = rd.inner == 0;
+            if (start) {
+                if (rB >= 0) ld6(at_off(a.r, oB), wr);
+                if (rB >= 0) ld6(at_off(a.r0, oB), w0);
+                if constexpr (!MIX)
+                    if (rB >= 0) ld6(at_off(a.x, oB), X);
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    wp[c] = wv[c] = (T)0;
+                    if constexpr (MIX) X[c] = 0.0f;
+                }
+            }
+            const T rm = a.rM ? (T)rdB : (T)1;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                if (!rd.on[c]) continue;
+                const T be = (T)uni(cs[c].beta);
+                const T wA = rm * wr[c], wT = rm * w0[c];
+                wp[c] = start ? wA : wA + be * wp[c];
+                wv[c] = start ? wT : wT + be * wv[c];
+            }
+            if (rB >= 0) {
+                st6(at_off(a.p, oB), wp);
+                st6(at_off(a.v, oB), wv);
+            }
+            ok = wait();
+            if (!ok) break;
+            T wA[6], wT[6];
+            {
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    wA[c] = dgB * wp[c];
+                    wT[c] = dgB * wv[c];
+                }
+                eB.template gather<false>(a.p, wA);
+                eR.template gather<false>(a.v, wT);
+                double q[6];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) q[c] = rd.on[c] && rB >= 0 ? (T)0 + wA[c] * wv[c] : (T)0;
+                write_partials<6>(q, a.partials, kRow);
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_bicg_w_body<T, RBLK>(an, lds);
+            __syncthreads();
+            {
+                double q[12];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) {
+                    q[c] = q[6 + c] = (T)0;
+                    if (!uni(cs[c].active)) continue;
+                    const double alpha = uni(cs[c].alpha);
+                    X[c] = (XT)((double)X[c] + alpha * (double)wp[c]);
+                    wr[c] = wr[c] - (T)alpha * wA[c];
+                    w0[c] = w0[c] - (T)alpha * wT[c];
+                    if (rB >= 0) {
+                        q[c] = (T)fabs(wr[c]);
+                        q[6 + c] = (T)0 + (rm * wr[c]) * w0[c];
+                    }
+                }
+                if (rB >= 0) {
+                    if constexpr (MIX) st6(at_off(a.e, oB), X);
+                    else st6(at_off(a.x, oB), X);
+                }
+                write_partials<12>(q, af.partials, kRow);
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_bicg_xr_body<T, RBLK>(af, lds);
+            __syncthreads();
+        } else if constexpr (BICG) {
+            passAll(m.pg, [&](const Blk& k) { k_bicg_p_body<T>(a, k); });
+            ok = wait();
+            if (!ok) break;
+            pass(a.G, [&](const Blk& k) { k_bicg_w_body<T>(a, k); });
+            ok = wait();
+            if (!ok) break;
+            k_fin_bicg_w_body<T, RBLK>(an, lds);
+            __syncthreads();
+            pass(a.G, [&](const Blk& k) { k_bicg_xr_body<T>(ax, k); });
+            ok = wait();
+            if (!ok) break;
+            k_fin_bicg_xr_body<T, RBLK>(af, lds);
+            __syncthreads();
+        } else {
+            if (round_of(a).inner > 0) {
+                passAll(m.pg, [&](const Blk& k) { k_kry_p_body<T>(RB ? b : a, k); });
+                ok = wait();
+                if (!ok) break;
+            }
+            if constexpr (RB) {
+                pass(m.Gw, [&](const Blk& k) { k_rb_w_body<T, 0>(a, k); });
+                ok = wait();
+                if (!ok) break;
+                pass(a.G, [&](const Blk& k) { k_rb_v_body<T>(a, k); });
+            } else {
+                pass(a.G, [&](const Blk& k) { k_kry_v_body<T>(a, k); });
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_v_body<T, RBLK>(an, lds);
+            __syncthreads();
+            if constexpr (RB) {
+                pass(m.Gw, [&](const Blk& k) { k_rb_w_body<T, 1>(a, k); });
+                ok = wait();
+                if (!ok) break;
+                pass(a.G, [&](const Blk& k) { k_rb_t_body<T>(a, k); });
+            } else {
+                pass(a.G, [&](const Blk& k) { k_kry_t_body<T>(a, k); });
+            }
+            ok = wait();
+            if (!ok) break;
+            k_fin_t_body<T, RBLK>(an, lds);
+            __syncthreads();
+            pass(a.G, [&](const Blk& k) { k_kry_xr_body<T>(ax, k); });
+            ok = wait();
+            if (!ok) break;
+            k_fin_xr_body<T, RBLK>(af, lds);
+            __syncthreads();
+        }
+    }
+    if (ok && p == 0)
+        for (int i = threadIdx.x; i < (int)(sizeof(cs) / 8); i += RBLK)
+            reinterpret_cast<double*>(m.a.cs)[i] = reinterpret_cast<const double*>(cs)[i];
+    if (ok) res_leave(bar);
+}
+
+// workgroup b of the grid: b % XCDS is the XCD it is dealt to; xcd < 0: on all
+template <class T, int FORM>
+__global__ void __launch_bounds__(RBLK, RES_PER_CU<T>) k_solve_one(ResArgs<T> m, int xcd) {
+    if (xcd >= 0 && (int)(blockIdx.x % XCDS) != xcd) return;
+    solve_resident<T, FORM>(m, xcd >= 0 ? blockIdx.x / XCDS : blockIdx.x);
 }
 
 // ----------------------------------------------------------------- driver
@@ -1420,7 +1989,10 @@ void Krylov::ensure(Mesh& m, bool mixed, bool bicg) {
         r = DBuf(); r0 = DBuf(); p = DBuf(); v = DBuf(); t = DBuf();
         rs = DBuf(); r0s = DBuf(); ps = DBuf(); vs = DBuf(); ts = DBuf(); es = DBuf();
         ahat32 = DBuf(); ahat64 = DBuf();
-        partials = ctx->alloc((size_t)grid * 24 * sizeof(double));
+        // the x/r pass of a resident solve has 12 more partial sums per workgroup
+        partials = ctx->alloc((size_t)grid * (N <= RES_MAX_ROWS ? 36 : 24) * sizeof(double));
+        xSave = DBuf();
+        if (N <= RES_MAX_ROWS && grid > RSUB) xSave = ctx->alloc(3 * vec * 8);
         state = ctx->alloc(sizeof(SolveState));
         RT_HIP(hipMemsetAsync(state.p, 0, sizeof(SolveState), ctx->stream));
         rD = ctx->alloc(std::max<size_t>(1, (size_t)m.N) * sizeof(double));
@@ -1468,7 +2040,7 @@ struct SolveRun {
     bool rb = false;                  // red-black ILU0: Krylov on the second colour's Schur complement
     double nRed = 0;                  // first colour's rows
     KryArgs<float> bf{};              // red-black: af/ad shifted to the second colour's rows
-    KryArgs<double> bd{};             // (the pointwise passes p, x/r and the fold)
+    KryArgs<double> bd{};             // (the pointwise passes p and the fold)
     KryArgs<float> sf{};              // red-black: the residual restricted to the second colour
     KryArgs<double> sd{};
     int64_t nEll = 0;                 // all ELL entries (the float copies of A, A^T)
@@ -1476,6 +2048,12 @@ struct SolveRun {
     bool ownsHost = false;            // hostState is a pinned block of ctx
     bool pending = false, done = false;
     int rounds = 0;
+    // the whole solve in one launch of P workgroups (k_solve_one / k_solve_group)
+    bool resident = false, resLaunched = false;
+    int P = 1, X = 1, form = 0;
+    uint32_t maxPolls = 0;
+    double* xSave = nullptr;
+    SolveState* st = nullptr;
     ~SolveRun() {
         if (hostState && ownsHost) ctx->givePinnedBlock(hostState);
         if (ev) (void)hipEventDestroy(ev);
@@ -1543,7 +2121,7 @@ int solve_grid(const Ctx* ctx, int cap, bool rb, bool bicg) {
         pc = least;
     }
     int64_t g = std::min<int64_t>(cap, (int64_t)ctx->numCUs * pc);
-    if (g >= 64) g = g / 8 * 8;
+    if (g >= 64 && g < cap) g = g / 8 * 8;
     return (int)std::max<int64_t>(1, g);
 }
 
@@ -1566,7 +2144,7 @@ int rb_wide_grid(const Ctx* ctx, int cap) {
         perCU = least;
     }
     int64_t g = std::min<int64_t>(cap, (int64_t)ctx->numCUs * perCU);
-    if (g >= 64) g = g / 8 * 8;
+    if (g >= 64 && g < cap) g = g / 8 * 8;
     return (int)std::max<int64_t>(1, g);
 }
 
@@ -1688,15 +2266,9 @@ template <class T>
 void launch_scale_of(Ctx* ctx, SolveRun& R) {
     const bool mixed = std::is_same<T, float>::value;
     KryArgs<T>& a = argsOf<T>(R);
-    if (R.rb) {
-        ProfScope ps(ctx, mixed ? "k_rb_scale<f32>" : "k_rb_scale<f64>", R.ne * (4 + 8 + sizeof(T)) + R.N * 8);
-        hipLaunchKernelGGL(k_rb_scale<T>, dim3(kblk((int64_t)R.N)), dim3(BLK), 0, ctx->stream, a.N, a.nRed, a.ellOff,
-                           a.ellWidth, a.slotMask, a.ellCol, a.aval, a.rD, a.rM, const_cast<T*>(a.ahat));
-    } else {
-        ProfScope ps(ctx, mixed ? "k_scale<f32>" : "k_scale<f64>", R.ne * (4 + 8 + sizeof(T)) + R.N * 8);
-        hipLaunchKernelGGL(k_scale<T>, dim3(kblk((int64_t)R.N)), dim3(BLK), 0, ctx->stream, a.N, a.ellOff,
-                           a.ellWidth, a.slotMask, a.ellCol, a.aval, a.rM, const_cast<T*>(a.ahat));
-    }
+    ProfScope ps(ctx, R.rb ? (mixed ? "k_rb_scale<f32>" : "k_rb_scale<f64>") : (mixed ? "k_scale<f32>" : "k_scale<f64>"),
+                 R.ne * (4 + 8 + sizeof(T)) + R.N * 8);
+    hipLaunchKernelGGL(k_scale<T>, dim3(kblk((int64_t)R.N)), dim3(BLK), 0, ctx->stream, a);
     RT_HIP(hipGetLastError());
     R.needScale = false;
 }
@@ -1827,7 +2399,7 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
         hipLaunchKernelGGL(k_fin_t<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         {
             ProfScope ps(ctx, mixed ? "k_kry_xr<f32>" : "k_kry_xr<f64>", Bb.xr(nAct, start));
-            hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, b);
+            hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
         }
         hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
         return;
@@ -1852,6 +2424,99 @@ void launch_iter(Ctx* ctx, SolveRun& R, double nAct, bool start) {
         hipLaunchKernelGGL(k_kry_xr<T>, dim3(R.G), dim3(BLK), 0, ctx->stream, a);
     }
     hipLaunchKernelGGL(k_fin_xr<T>, dim3(1), dim3(FBLK), 0, ctx->stream, a);
+}
+
+// the workgroups of a member's pointwise passes (p, fold)
+int point_grid(const SolveRun& R) {
+    if (!R.rb) return R.pgrid;
+    return std::max(1, std::min<int>(R.pgrid, (int)((R.N - R.nRed + BLK - 1) / BLK)));
+}
+
+// Whether the solve runs as one resident launch, and its workgroups (a row a
+// thread): a mesh of at most RES_MAX_ROWS rows, with the workspace it needs and
+// no kernel timing (which charges every pass its bytes).
+// f(kernel instantiation of the form)
+template <class T, class F>
+auto with_form(int form, F&& f) {
+    switch (form) {
+    case RF_REDBLACK: return f(std::integral_constant<int, RF_REDBLACK>{});
+    case RF_BICG: return f(std::integral_constant<int, RF_BICG>{});
+    case RF_RB_ROW: return f(std::integral_constant<int, RF_RB_ROW>{});
+    case RF_BICG_ROW: return f(std::integral_constant<int, RF_BICG_ROW>{});
+    default: return f(std::integral_constant<int, RF_JACOBI>{});
+    }
+}
+
+template <class T>
+bool resident_fits(int form) {
+    return with_form<T>(form, [](auto F) {
+        static int perCU = -1;  // the same on every gfx950 device
+        if (perCU < 0) {
+            int nb = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_solve_one<T, decltype(F)::value>, RBLK, 0) != hipSuccess)
+                nb = 0;
+            perCU = nb;
+        }
+        return perCU >= RES_PER_CU<T>;
+    });
+}
+
+template <class T>
+void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
+    Krylov& K = *sa.kry;
+    R.resident = R.resLaunched = false;
+    if (sa.ctl->residentPolls == 0 || ctx->profiling || K.N > RES_MAX_ROWS) return;
+    if (R.G % 8 == 0 || K.partials.bytes < (size_t)36 * K.grid * sizeof(double)) return;
+    const Mesh& m = *sa.mesh;
+    // row-kernel workgroups with a tile (their tiles in order: G is no multiple of 8)
+    const int32_t row0 = R.rb ? m.nRed & ~(SLICE - 1) : 0;
+    R.X = std::max((int)kblk(m.N - row0), R.rb ? (int)kblk(m.nRed) : 1);
+    if (R.X > R.G) return;
+    R.P = (R.X + RSUB - 1) / RSUB;
+    const bool row = m.maxWidth <= ROW_W;
+    R.form = R.bicg ? (row ? RF_BICG_ROW : RF_BICG) : R.rb ? (row ? RF_RB_ROW : RF_REDBLACK) : RF_JACOBI;
+    if (R.P > ctx->numCUs / 2) return;
+    // Measured (us a step, by launches / resident): rows kept, red-black FP64 233 /
+    // 146 at 4096 cells, 285 / 207 at 16384, 356 / 299 at 65536, PBiCG 511 / 326
+    // at 16384; the passes over memory of the other forms 338 / 266 at 16384,
+    // 385 / 349 at 36864, 466 / 475 at 65536
+    if (R.form < RF_RB_ROW && m.N > RES_MAX_ROWS / 2) return;
+    if (R.P > 1 && !K.xSave.p) return;
+    if (!resident_fits<T>(R.form)) return;
+    R.maxPolls = sa.ctl->residentPolls;
+    R.xSave = R.P > 1 ? K.xSave.as<double>() : nullptr;
+    R.st = K.state.as<SolveState>();
+    R.resident = true;
+}
+
+template <class T>
+ResArgs<T> resident_args(SolveRun& R) {
+    ResArgs<T> m{};
+    m.a = argsOf<T>(R);
+    m.b = R.rb ? blackOf<T>(R) : m.a;
+    m.s = R.rb ? sweepOf<T>(R) : m.a;
+    m.P = R.P;
+    m.pg = point_grid(R);
+    m.Gw = R.Gw;
+    m.X = R.X;
+    m.doScale = R.needScale ? 1 : 0;
+    m.maxPolls = R.maxPolls;
+    m.st = R.st;
+    m.xSave = R.xSave;
+    return m;
+}
+
+template <class T>
+void launch_resident(Ctx* ctx, SolveRun& R) {
+    const ResArgs<T> m = resident_args<T>(R);
+    // on one XCD if they fit there
+    const int xcd = R.P <= RES_PER_CU<T> * ctx->numCUs / XCDS ? ctx->xcd : -1;
+    const int grid = xcd < 0 ? R.P : R.P == 1 ? xcd + 1 : XCDS * R.P;
+    with_form<T>(R.form, [&](auto F) {
+        hipLaunchKernelGGL((k_solve_one<T, decltype(F)::value>), dim3(grid), dim3(RBLK), 0, ctx->stream, m, xcd);
+    });
+    RT_HIP(hipGetLastError());
+    R.resLaunched = true;
 }
 
 // rounds a non-blocking advance queues per host round trip
@@ -1906,20 +2571,84 @@ void solve_begin(Ctx* ctx, const SolveArgs& sa) {
     R.rounds = 0;
     if (mixed) {
         fill_args<float>(ctx, sa, R);
+        choose_resident<float>(ctx, sa, R);
         if (!sa.initDone) launch_init<float>(ctx, R);
         if (bicg) launch_bicg_init<float>(ctx, R);
     } else {
         fill_args<double>(ctx, sa, R);
+        choose_resident<double>(ctx, sa, R);
         if (!sa.initDone) launch_init<double>(ctx, R);
         if (bicg) launch_bicg_init<double>(ctx, R);
     }
     RT_HIP(hipGetLastError());
+    if (R.resident) {
+        // nothing to decide on the host before the resident launch; the event
+        // is what a group's stream waits for
+        R.pending = false;
+        if (R.ev) RT_HIP(hipEventRecord(R.ev, ctx->stream));
+        return;
+    }
     queue_pull(ctx, K, R);
 }
+
+namespace {
+
+// components of the state last pulled that are still iterating or waiting for a sweep
+void open_components(const SolveRun& R, double& nAct, double& nRef) {
+    nAct = nRef = 0;
+    for (int c = 0; c < 6; ++c) {
+        if (R.valid[c] <= 0) continue;
+        nAct += R.host[c].active != 0;
+        nRef += R.host[c].needRefine != 0;
+    }
+}
+
+// A resident launch whose state is back.  True: the solve is finished.  A
+// workgroup's wait that gave up leaves the counters set; the records then
+// either are final (it gave up behind the last barrier, which every workgroup
+// had reached) or still the start's, and the solve is run by launches from the
+// saved x.
+bool resident_done(Ctx* ctx, SolveRun& R) {
+    double nAct, nRef;
+    open_components(R, nAct, nRef);
+    uint32_t any = R.hostState->bar[0] | R.hostState->bar[2];
+    for (const auto& x : R.hostState->barL2) any |= x[0] | x[1];
+    const bool gaveUp = (any & RES_FAIL) != 0;
+    if (gaveUp) {
+        launch_fill(ctx, reinterpret_cast<double*>(R.st->bar), sizeof(R.st->bar) / 8, 0.0);
+        launch_fill(ctx, reinterpret_cast<double*>(R.st->barL2), sizeof(R.st->barL2) / 8, 0.0);
+    }
+    if (nAct == 0 && nRef == 0) return true;
+    if (!gaveUp) return true;  // the round limit
+    const size_t n6 = (size_t)6 * (size_t)R.N;
+    const size_t w = R.mixed ? sizeof(float) : sizeof(double);
+    const size_t nv = (n6 * w + 15) / 16 * 16;  // whole 16-byte words; the buffers are padded to 256
+    launch_copy(ctx, R.xSave, R.mixed ? R.af.x : R.ad.x, n6 * sizeof(double));
+    if (!R.rb) launch_copy(ctx, R.xSave + n6, R.mixed ? (void*)R.af.r0 : (void*)R.ad.r0, nv);
+    if (R.bicg) launch_copy(ctx, R.xSave + 2 * n6, R.mixed ? (void*)R.af.r : (void*)R.ad.r, nv);
+    R.resident = R.resLaunched = false;
+    R.needScale = R.nEll > 0;
+    return false;
+}
+
+}  // namespace
 
 bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
     SolveRun& R = *K.run;
     if (R.done) return true;
+    if (R.resident && !R.resLaunched && !block && R.P > 1) {
+        // many solves advanced without batching would launch their barriers on
+        // many streams at once, more workgroups than fit together
+        R.resident = false;
+        queue_pull(ctx, K, R);
+        return false;
+    }
+    if (R.resident && !R.resLaunched) {
+        if (R.mixed) launch_resident<float>(ctx, R);
+        else launch_resident<double>(ctx, R);
+        queue_pull(ctx, K, R);
+        return false;
+    }
     if (R.pending) {
         if (block) {
             if (R.ev) RT_HIP(hipEventSynchronize(R.ev));
@@ -1936,6 +2665,10 @@ bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
             R.ne = R.hostState->misc[0];
             R.neFromDevice = false;
         }
+    }
+    if (R.resident && resident_done(ctx, R)) {
+        R.done = true;
+        return true;
     }
     double nAct = 0, nRef = 0;
     bool start = true;  // every component of the round begins an inner solve (p = r = r0)
@@ -2017,6 +2750,14 @@ __global__ void __launch_bounds__(BLK) k_group(const KryArgs<T>* __restrict__ ta
     Body(a, Blk{starts[i + 1] - starts[i], (int)blockIdx.x - starts[i], (int)threadIdx.x, red});
 }
 
+// map: per workgroup of the grid its member and index in it, -1 for none
+template <class T, int FORM>
+__global__ void __launch_bounds__(RBLK, RES_PER_CU<T>) k_solve_group(const ResArgs<T>* __restrict__ tab, const int2* __restrict__ map) {
+    const int2 w = map[blockIdx.x];
+    if (w.x < 0) return;
+    solve_resident<T, FORM>(tab[w.x], w.y);
+}
+
 template <class T, void (*Body)(const KryArgs<T>&, double*)>
 __global__ void __launch_bounds__(FBLK) k_group_fin(const KryArgs<T>* __restrict__ tab) {
     __shared__ double lds[FIN_LDS];
@@ -2063,7 +2804,7 @@ void group_round(bool rb, hipStream_t st, const GroupDev<T>& d) {
         glaunch<T, &k_rb_w_body<T, 1>>(st, d.A, d.W, d.totW, n);
         glaunch<T, &k_rb_t_body<T>>(st, d.A, d.G, d.totG, n);
         glaunch_fin<T, &k_fin_t_body<T>>(st, d.A, n);
-        glaunch<T, &k_kry_xr_body<T>>(st, d.B, d.G, d.totG, n);
+        glaunch<T, &k_kry_xr_body<T>>(st, d.A, d.G, d.totG, n);
         glaunch_fin<T, &k_fin_xr_body<T>>(st, d.A, n);
     } else {
         glaunch<T, &k_fold_body<T>>(st, d.A, d.P, d.totP, n);
@@ -2080,10 +2821,78 @@ void group_round(bool rb, hipStream_t st, const GroupDev<T>& d) {
     RT_HIP(hipGetLastError());
 }
 
-// the workgroups of a member's pointwise passes (p, fold)
-int point_grid(const SolveRun& R) {
-    if (!R.rb) return R.pgrid;
-    return std::max(1, std::min<int>(R.pgrid, (int)((R.N - R.nRed + BLK - 1) / BLK)));
+// page-locked staging and device memory for a group's tables
+void group_tables(SolveGroup& g, size_t bytes) {
+    if (g.hostBytes < bytes) {
+        if (g.hostTables) (void)hipHostFree(g.hostTables);
+        g.hostTables = nullptr;
+        RT_HIP(hipHostMalloc(&g.hostTables, bytes, hipHostMallocDefault));
+        g.hostBytes = bytes;
+    }
+    if (g.tables.bytes < bytes) g.tables = g.ctx->alloc(bytes);
+}
+
+// A group of resident solves: every member's whole solve, in launches that
+// place at most RES_PER_CU workgroups per CU.  A member goes to the XCD with the fewest
+// workgroups so far (the largest members first would pack tighter; a queue's
+// order keeps its latency).
+template <class T>
+void group_launch_resident(SolveGroup& g) {
+    const int n = (int)g.members.size();
+    struct Launch {
+        std::vector<int2> map;
+        int load[XCDS] = {0};
+        int form = 0;
+    };
+    std::vector<Launch> launches;
+    const int cap = RES_PER_CU<T> * g.ctx->numCUs / XCDS;
+    for (int i = 0; i < n; ++i) {
+        const int P = g.members[i].K->run->P, form = g.members[i].K->run->form;
+        const bool spread = P > cap;  // more than an XCD's CUs: over all of them
+        const int need = spread ? (P + XCDS - 1) / XCDS : P;
+        int x = 0;
+        if (!launches.empty()) {
+            const int* ld = launches.back().load;
+            x = (int)((spread ? std::max_element(ld, ld + XCDS) : std::min_element(ld, ld + XCDS)) - ld);
+        }
+        if (launches.empty() || launches.back().form != form || launches.back().load[x] + need > cap) {
+            launches.emplace_back();
+            launches.back().form = form;
+            x = 0;
+        }
+        Launch& L = launches.back();
+        for (int p = 0; p < P; ++p) {
+            if (spread) x = p % XCDS;
+            const size_t b = (size_t)XCDS * L.load[x]++ + x;
+            if (L.map.size() <= b) L.map.resize(b + 1, int2{-1, 0});
+            L.map[b] = int2{i, p};
+        }
+    }
+    size_t blocks = 0;
+    for (auto& L : launches) blocks += L.map.size();
+    const size_t szA = sizeof(ResArgs<T>) * n, bytes = szA + sizeof(int2) * blocks;
+    group_tables(g, bytes);
+    auto* tab = static_cast<ResArgs<T>*>(g.hostTables);
+    auto* map = reinterpret_cast<int2*>(static_cast<unsigned char*>(g.hostTables) + szA);
+    for (int i = 0; i < n; ++i) tab[i] = resident_args<T>(*g.members[i].K->run);
+    for (auto& L : launches) map = std::copy(L.map.begin(), L.map.end(), map);
+    RT_HIP(hipMemcpyAsync(g.tables.p, g.hostTables, bytes, hipMemcpyHostToDevice, g.ctx->stream));
+    const auto* dt = static_cast<const ResArgs<T>*>(g.tables.p);
+    const auto* dm = reinterpret_cast<const int2*>(static_cast<const unsigned char*>(g.tables.p) + szA);
+    for (auto& L : launches) {
+        const dim3 grid((unsigned)L.map.size());
+        with_form<T>(L.form, [&](auto F) {
+            hipLaunchKernelGGL((k_solve_group<T, decltype(F)::value>), grid, dim3(RBLK), 0, g.ctx->stream, dt, dm);
+        });
+        dm += L.map.size();
+    }
+    RT_HIP(hipGetLastError());
+    for (auto& mb : g.members) {
+        mb.K->run->resLaunched = true;
+        queue_pull(g.ctx, *mb.K, *mb.K->run);
+    }
+    g.launched = true;
+    ++g.launches;
 }
 
 template <class T>
@@ -2094,13 +2903,7 @@ void group_launch(SolveGroup& g) {
     const size_t bytes = offW + szI;
     int totG = 0, totP = 0, totW = 0;
     if (g.dirty) {
-        if (g.hostBytes < bytes) {
-            if (g.hostTables) (void)hipHostFree(g.hostTables);
-            g.hostTables = nullptr;
-            RT_HIP(hipHostMalloc(&g.hostTables, bytes, hipHostMallocDefault));
-            g.hostBytes = bytes;
-        }
-        if (g.tables.bytes < bytes) g.tables = g.ctx->alloc(bytes);
+        group_tables(g, bytes);
         unsigned char* h = static_cast<unsigned char*>(g.hostTables);
         auto* tA = reinterpret_cast<KryArgs<T>*>(h);
         auto* tB = reinterpret_cast<KryArgs<T>*>(h + offB);
@@ -2149,8 +2952,9 @@ SolveGroup::~SolveGroup() {
     if (hostTables) (void)hipHostFree(hostTables);
 }
 
-bool solve_groupable(const Krylov& K, bool* mixed, bool* rb) {
+bool solve_groupable(const Krylov& K, bool* mixed, bool* rb, bool* resident) {
     if (!K.run || K.run->bicg || !K.run->ev) return false;
+    if (resident) *resident = K.run->resident;
     if (mixed) *mixed = K.run->mixed;
     if (rb) *rb = K.run->rb;
     return true;
@@ -2158,12 +2962,12 @@ bool solve_groupable(const Krylov& K, bool* mixed, bool* rb) {
 
 void group_join(SolveGroup& g, Krylov& K, hipStream_t home) {
     SolveRun& R = *K.run;
-    if (R.bicg || R.mixed != g.mixed || R.rb != g.rb || !R.ev)
+    if (R.bicg || R.mixed != g.mixed || R.rb != g.rb || R.resident != g.resident || !R.ev)
         throw Error{RT_E_BAD_ARG, "group_join: the solve does not belong to this group"};
     // the group's stream waits for the solve's own queued work (the assembly,
     // the initial residual and the first state pull)
     RT_HIP(hipStreamWaitEvent(g.ctx->stream, R.ev, 0));
-    if (R.needScale) {  // the scaled matrix its first iteration would build
+    if (R.needScale && !R.resident) {  // the scaled matrix its first iteration would build
         if (R.mixed) launch_scale_of<float>(g.ctx, R);
         else launch_scale_of<double>(g.ctx, R);
     }
@@ -2207,12 +3011,19 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
     for (size_t i = 0; i < g.members.size();) {
         SolveRun& R = *g.members[i].K->run;
         double nAct = 0, nRef = 0;
-        for (int c = 0; c < 6; ++c) {
-            if (R.valid[c] <= 0) continue;
-            nAct += R.host[c].active != 0;
-            nRef += R.host[c].needRefine != 0;
+        open_components(R, nAct, nRef);
+        bool fin;
+        if (R.resident) {
+            fin = R.resLaunched;
+            if (fin && !resident_done(g.ctx, R)) {
+                // its resident launch gave up: by launches, to the end
+                while (!solve_advance(g.ctx, *g.members[i].K, true)) {
+                }
+            }
+        } else {
+            fin = (nAct == 0 && nRef == 0) || R.rounds >= 100000;
         }
-        if ((nAct == 0 && nRef == 0) || R.rounds >= 100000) {
+        if (fin) {
             if (!drained) {
                 RT_HIP(hipEventCreateWithFlags(&drained, hipEventDisableTiming));
                 RT_HIP(hipEventRecord(drained, g.ctx->stream));
@@ -2228,8 +3039,14 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
     }
     if (drained) RT_HIP(hipEventDestroy(drained));  // released once the waits are satisfied
     if (g.members.empty()) return;
-    if (g.mixed) group_launch<float>(g);
-    else group_launch<double>(g);
+    if (g.resident) {
+        if (g.mixed) group_launch_resident<float>(g);
+        else group_launch_resident<double>(g);
+    } else if (g.mixed) {
+        group_launch<float>(g);
+    } else {
+        group_launch<double>(g);
+    }
 }
 
 void solve_finish(Krylov& K, rt_solver_perf perf[6]) {
@@ -2254,12 +3071,17 @@ void solve_lockstep(Ctx* ctx, const SolveArgs& a, rt_solver_perf perf[6]) {
     solve_finish(*a.kry, perf);
 }
 
+// Workgroups of the row kernels: one per tile up to eight per CU.  A multiple of
+// 8 gives each XCD a slab of the tiles; it has to be large enough that every
+// tile of the two colours' slabs has a workgroup: with the next smaller multiple
+// a few workgroups walked two tiles and the pass took twice as long (397 tiles
+// on 392 workgroups).  Meshes that may be solved resident take no slabs: tile t
+// is workgroup t's.
 int grid_for(const Ctx* ctx, int32_t N) {
     const int64_t need = ((int64_t)N + BLK - 1) / BLK;
     const int64_t cap = (int64_t)ctx->numCUs * 8;
-    int64_t g = need < cap ? need : cap;
-    if (g >= 64) g = g / 8 * 8;
-    return (int)std::max<int64_t>(1, g);
+    if (N <= RES_MAX_ROWS) return (int)std::max<int64_t>(1, need % 8 == 0 ? need + 1 : need);
+    return (int)std::min(((need + 7) / 8 + 1) * 8, cap);
 }
 
 }  // namespace rt

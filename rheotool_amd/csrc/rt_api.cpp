@@ -4,6 +4,7 @@
 // handles, the constitutiveEq run-time selection from dictionary text, the
 // correct() sequence and the sparseSolver<symmTensor>::solve surface.
 #include <algorithm>
+#include <atomic>
 #include <cctype>
 #include <cmath>
 #include <cstring>
@@ -224,6 +225,7 @@ Controls parseControls(const char* text) {
     if (e->scalar("minIter", v)) c.minIter = (int)v;
     if (e->scalar("innerRelTol", v)) c.innerRelTol = v;
     if (e->scalar("maxRefine", v)) c.maxRefine = (int)v;
+    if (e->scalar("residentPolls", v)) c.residentPolls = v > 0 ? (uint32_t)std::min(v, 1e9) : 0u;
     if (e->word("precision", s)) {
         if (s == "mixed") c.mixed = true;
         else if (s == "double") c.mixed = false;
@@ -640,6 +642,7 @@ size_t modelBytesEstimate(int32_t N, int32_t F, int32_t NB, int64_t nEll, bool m
     // Krylov: r r0 p v t (and the mixed solve's correction e) x 6 components,
     // rD, ahat, partials, state
     by += 6 * n * (mixed ? 6 * 4 : 5 * 8) + 8 * n + ne * (mixed ? 4 : 8) + 2048 * 24 * 8 + 4096;
+    if (N <= RES_MAX_ROWS) by += 3 * 6 * 8 * n + 2048 * 12 * 8;  // resident solve: its saved start, more partials
     // staging for AoS transfers (9 comps)
     by += 9 * 8 * n;
     if (gradU) by += 9 * 8 * n;      // the prescribed gradient
@@ -771,6 +774,8 @@ int rt_ctx_create(int device, size_t hbm_budget, rt_ctx** out) {
             throw Error{RT_E_NO_DEVICE, std::string("device ") + std::to_string(device) + " is " +
                                             prop.gcnArchName + "; this library is built for gfx950"};
         x.numCUs = prop.multiProcessorCount;
+        static std::atomic<unsigned> made{0};
+        x.xcd = (int)(made.fetch_add(1) % 8);
         x.budget = hbm_budget;
         RT_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
         noallocInit(device);
@@ -1247,12 +1252,12 @@ int rt_model_correct_iter(rt_model* model, double deltaT, const double* gradU, i
                     throw Error{e.code, "mode " + mode->impl.name + ": " + e.msg};
                 }
             }
-            bool same = true, mixed0 = false, rb0 = false;
+            bool same = true, mixed0 = false, rb0 = false, res0 = false;
             for (size_t i = 0; i < M.modes.size(); ++i) {
-                bool mx = false, rb = false;
-                if (!solve_groupable(M.modes[i]->impl.kry, &mx, &rb)) same = false;
-                if (i == 0) mixed0 = mx, rb0 = rb;
-                else if (mx != mixed0 || rb != rb0) same = false;
+                bool mx = false, rb = false, res = false;
+                if (!solve_groupable(M.modes[i]->impl.kry, &mx, &rb, &res)) same = false;
+                if (i == 0) mixed0 = mx, rb0 = rb, res0 = res;
+                else if (mx != mixed0 || rb != rb0 || res != res0) same = false;
             }
             if (!same) {  // PBiCG, or modes with different solve forms: one after another
                 for (rt_model* mode : M.modes)
@@ -1263,6 +1268,7 @@ int rt_model_correct_iter(rt_model* model, double deltaT, const double* gradU, i
                 G.ctx = M.ctx;
                 G.mixed = mixed0;
                 G.rb = rb0;
+                G.resident = res0;
                 for (rt_model* mode : M.modes) group_join(G, mode->impl.kry, M.ctx->stream);
                 std::vector<Krylov*> done;
                 while (!G.members.empty()) {

@@ -74,28 +74,50 @@ __device__ __forceinline__ Blk blk_of_launch(double* red) {
     return Blk{(int)gridDim.x, (int)blockIdx.x, (int)threadIdx.x, red};
 }
 
-// Sums of NQ per-lane values over the 64 lanes of a wavefront, halving the
-// values a lane carries at each exchange: 21 exchanges for 18 values where a
-// butterfly per value takes 108, with the butterfly's association of every
-// sum (the t pass of a 128 x 128 channel: 9.9 to 6.2 us with it).  Lane l ends
-// with the sum of value lo (valid if n > 0).
+// Lane exchanges inside a wavefront, on the VALU (a shuffle through LDS has ten
+// times their latency).  Level O pairs lanes l and l ^ O (l ^ 7 at O = 4, the
+// mirror of a half row).
+template <int O>
+__device__ __forceinline__ uint32_t lane_pair(uint32_t v) {
+    constexpr int ctrl = O == 8 ? 0x128 : O == 4 ? 0x141 : O == 2 ? 0x4e : 0xb1;
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, ctrl, 0xf, 0xf, false);
+}
+// a + its pair's a on the lanes without bit O, b + its pair's b on the others
+template <int O>
+__device__ __forceinline__ double pair_sum(double a, double b, bool up) {
+    const uint32_t al = (uint32_t)__double2loint(a), ah = (uint32_t)__double2hiint(a);
+    const uint32_t bl = (uint32_t)__double2loint(b), bh = (uint32_t)__double2hiint(b);
+    if constexpr (O == 32 || O == 16) {
+        // swaps the lanes with bit O of a for those without of b
+        auto sw = [](uint32_t x, uint32_t y) {
+            if constexpr (O == 32) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+            else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        };
+        const auto l = sw(al, bl), h = sw(ah, bh);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    } else {
+        const double keep = up ? b : a;
+        const uint32_t sl = up ? al : bl, sh = up ? ah : bh;
+        return keep + __hiloint2double((int)lane_pair<O>(sh), (int)lane_pair<O>(sl));
+    }
+}
+
+// Sums of N per-lane values over the 64 lanes of a wavefront, halving the values
+// a lane carries at each exchange: 21 exchanges for 18 values where a butterfly
+// per value takes 108.  Lane l ends with the sum of value lo (valid if n > 0).
 template <int N, int O>
 __device__ __forceinline__ double wave_scatter(const double (&v)[N], int lane, int& lo, int& n) {
     if constexpr (O == 0) {
         return v[0];
     } else if constexpr (N == 1) {
-        const double w[1] = {v[0] + __shfl_xor(v[0], O, 64)};
+        const double w[1] = {pair_sum<O>(v[0], v[0], lane & O)};
         return wave_scatter<1, O / 2>(w, lane, lo, n);
     } else {
         constexpr int H = (N + 1) / 2;
         const bool up = lane & O;
         double w[H];
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
-            const double hi = H + i < N ? v[H + i] : 0.0;
-            const double keep = up ? hi : v[i], send = up ? v[i] : hi;
-            w[i] = keep + __shfl_xor(send, O, 64);
-        }
+        for (int i = 0; i < H; ++i) w[i] = pair_sum<O>(v[i], H + i < N ? v[H + i] : 0.0, up);
         lo += up ? H : 0;
         n = up ? n - H : (n < H ? n : H);
         return wave_scatter<H, O / 2>(w, lane, lo, n);
@@ -134,15 +156,16 @@ __device__ __forceinline__ void write_partials(const double (&v)[NQ], double* pa
 // depends on G alone.
 constexpr int FBLK = 1024;
 constexpr int FIN_LDS = FBLK + 9 * RED_MAX;
-template <int NQ>
+// NT: threads of the workgroup that runs it (each takes FBLK / NT of the sums)
+template <int NQ, int NT = FBLK>
 __device__ __forceinline__ void sum_partials(const double* partials, int G, double* lds, double*& sums) {
-    constexpr int J = FBLK / NQ, J2 = 8;
+    constexpr int J = FBLK / NQ, J2 = 8, S = J * NQ;
     double* s2 = lds + FBLK;
     sums = s2 + J2 * NQ;
-    const int t = threadIdx.x;
-    if (t < J * NQ) {
-        constexpr int S = J * NQ;
-        const int total = G * NQ;
+    const int total = G * NQ;
+#pragma unroll
+    for (int t = threadIdx.x; t < FBLK; t += NT) {
+        if (t >= S) break;
         double acc = 0;
         int i = t;
         for (; i + 7 * S < total; i += 8 * S) {
@@ -156,6 +179,7 @@ __device__ __forceinline__ void sum_partials(const double* partials, int G, doub
         lds[t] = acc;
     }
     __syncthreads();
+    const int t = threadIdx.x;
     if (t < J2 * NQ) {
         const int q = t % NQ;
         double acc = 0;
@@ -172,6 +196,25 @@ __device__ __forceinline__ void sum_partials(const double* partials, int G, doub
     }
     __syncthreads();
 }
+
+// A component record in registers, field by field (copied as a whole the
+// compiler keeps it in memory).
+struct Comp {
+    double rho, rhoOld, alpha, omega, beta, normFactor, initRes, finalRes, innerTarget;
+    int32_t iter, active, converged, solved, exitAtS, needRefine, nRefine, innerIter, foldE;
+    __device__ __forceinline__ void load(const CompState& c) {
+        rho = c.rho, rhoOld = c.rhoOld, alpha = c.alpha, omega = c.omega, beta = c.beta;
+        normFactor = c.normFactor, initRes = c.initRes, finalRes = c.finalRes, innerTarget = c.innerTarget;
+        iter = c.iter, active = c.active, converged = c.converged, solved = c.solved, exitAtS = c.exitAtS;
+        needRefine = c.needRefine, nRefine = c.nRefine, innerIter = c.innerIter, foldE = c.foldE;
+    }
+    __device__ __forceinline__ void store(CompState& c) const {
+        c.rho = rho, c.rhoOld = rhoOld, c.alpha = alpha, c.omega = omega, c.beta = beta;
+        c.normFactor = normFactor, c.initRes = initRes, c.finalRes = finalRes, c.innerTarget = innerTarget;
+        c.iter = iter, c.active = active, c.converged = converged, c.solved = solved, c.exitAtS = exitAtS;
+        c.needRefine = needRefine, c.nRefine = nRefine, c.innerIter = innerIter, c.foldE = foldE;
+    }
+};
 
 // interleaved [N][6] rows: three 2-wide vector loads/stores per row
 template <class T> struct Vec2;
@@ -242,15 +285,15 @@ __device__ __forceinline__ void symmetry_value(const double sf[3], const double 
 // ------------------------------------------------- Krylov control (OpenFOAM)
 // SolverPerformance::checkConvergence: final < tolerance, or relTol > 0 and
 // final < relTol * initial
-__device__ __forceinline__ bool conv_outer(const CompState& c, const KryCtl& k, double res) {
+__device__ __forceinline__ bool conv_outer(const Comp& c, const KryCtl& k, double res) {
     return res < k.tol || (k.relTol > 0 && res < k.relTol * c.initRes);
 }
-__device__ __forceinline__ bool conv_inner(const CompState& c, const KryCtl& k, double res) {
+__device__ __forceinline__ bool conv_inner(const Comp& c, const KryCtl& k, double res) {
     return k.mixed ? res < c.innerTarget : conv_outer(c, k, res);
 }
 
 // begin an inner Krylov solve on a component whose r, r0 were just set
-__device__ __forceinline__ void start_inner(CompState& c, const KryCtl& k, double rr) {
+__device__ __forceinline__ void start_inner(Comp& c, const KryCtl& k, double rr) {
     c.innerIter = 0;
     c.rho = rr;
     c.exitAtS = 0;
@@ -264,7 +307,7 @@ __device__ __forceinline__ void start_inner(CompState& c, const KryCtl& k, doubl
 }
 
 // after the initial residual: normalisation factor, initial residual, start
-__device__ __forceinline__ void finish_initial(CompState& cs, const KryCtl& k, double absR, double rr,
+__device__ __forceinline__ void finish_initial(Comp& cs, const KryCtl& k, double absR, double rr,
                                                double nrm) {
     cs.normFactor = nrm + 1e-20;
     cs.initRes = absR / cs.normFactor;

@@ -68,6 +68,7 @@ struct Ctx {
     rt_ctx* handle = nullptr;
     int device = 0;
     int numCUs = 256;
+    int xcd = 0;  // where its resident solves run: contexts take turns
     hipStream_t stream = nullptr;
     size_t budget = 0, inUse = 0;
     std::string lastError;
@@ -195,6 +196,9 @@ struct Controls {
     bool mixed = false;
     double innerRelTol = 1e-5;  // FP32 inner solve reduction per refinement sweep
     int maxRefine = 12;
+    // polls after which a workgroup of a resident solve stops waiting for the
+    // others (about 0.1 s) and the solve is run by launches; 0: always by launches
+    uint32_t residentPolls = 200000;
 };
 // Parses an fvSolution-style entry; throws Error.
 Controls parseControls(const char* text);
@@ -231,12 +235,20 @@ struct SolveState {
     CompState c[6];
     int32_t anyActive;
     double misc[8];  // misc[0]: ELL entries in live slots of the solve's matrix (set by the assembly)
+    // barriers of a resident solve, zero between launches (top bit: a wait gave
+    // up).  bar: [0] entered, [1] left, [2] the XCDs' barrier, [8 + x] workgroups on
+    // XCD x; barL2[x]: XCD x's own, a cache line each (arrivals, barriers, departures)
+    alignas(128) uint32_t bar[32];
+    alignas(128) uint32_t barL2[8][32];
 };
 
 struct SolveRun;  // host side of a resumable solve (kernels_krylov.hip)
 struct SolveRunDeleter {
     void operator()(SolveRun* r) const;
 };
+
+// Rows up to which a solve runs as one resident launch (kernels_krylov.hip)
+constexpr int32_t RES_MAX_ROWS = 65536;
 
 // Workspace of the lockstep Krylov solver (all 6 components, SoA).
 struct Krylov {
@@ -255,7 +267,8 @@ struct Krylov {
     DBuf rD;               // double [N]    1/diag
     DBuf rDs;              // double [N]    red-black: 1/diag of the Schur complement
                            // (the ILU0 diagonal) where it differs from 1/diag
-    DBuf partials;         // double [grid][24]
+    DBuf partials;         // double [grid][24] (36 on a mesh of at most RES_MAX_ROWS rows)
+    DBuf xSave;            // FP64 [3][N][6] the start of a resident solve of several workgroups
     DBuf state;            // SolveState
     std::unique_ptr<SolveRun, SolveRunDeleter> run;
     // set when the buffers above are views into the no-allocation scratch
@@ -511,7 +524,7 @@ int grid_for(const Ctx* ctx, int32_t N);
 // rounds run on the group's stream.
 struct SolveGroup {
     Ctx* ctx = nullptr;  // the group's stream and table memory
-    bool mixed = false, rb = false;
+    bool mixed = false, rb = false, resident = false;
     struct Member {
         Krylov* K;
         hipStream_t home;  // the stream the solve was begun on (and continues on)
@@ -526,7 +539,7 @@ struct SolveGroup {
     ~SolveGroup();
 };
 // a begun solve that grouped rounds can run (PBiCGStab), and its group class
-bool solve_groupable(const Krylov& K, bool* mixed, bool* rb);
+bool solve_groupable(const Krylov& K, bool* mixed, bool* rb, bool* resident = nullptr);
 // adds a begun solve: the group's stream waits for the work queued on `home`
 void group_join(SolveGroup& g, Krylov& K, hipStream_t home);
 // Polls the members' states without blocking.  Members whose solve has

@@ -27,9 +27,12 @@ namespace rt {
 namespace {
 
 constexpr size_t kScratchBytes = RT_NOALLOC_SCRATCH_BYTES;
+// behind the scratch bytes the meshes share: the reduction partials (at most
+// 2048 workgroups of 36 sums) and the solver state
+constexpr size_t kTailBytes = size_t(1) << 20;
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kTailBytes];
 
 struct Slot {
     std::once_flag once;
@@ -178,8 +181,24 @@ int solveNoAlloc(Ctx* c, const Mesh& mc, const rt_ldu_symm* sys, double* psi, co
     const bool rb = kryCtl(ctl, mixed, m).rb != 0;
     double* dS = rb ? (double*)cv.take((size_t)2 * std::max(1, N) * 8) : nullptr;
     K.rD = view((size_t)std::max(1, N) * 8);
-    K.partials = view((size_t)grid * 24 * sizeof(double));
-    K.state = view(sizeof(SolveState));
+    // the partials and the state count against the limit at the sizes that set
+    // it (24 sums a workgroup, the workgroups rounded down, 1280 bytes)
+    const int64_t tiles = ((int64_t)N + 255) / 256, g0 = std::min<int64_t>(tiles, (int64_t)c->numCUs * 8);
+    cv.take((size_t)(g0 >= 64 ? g0 / 8 * 8 : std::max<int64_t>(1, g0)) * 24 * sizeof(double));
+    cv.take(1280);
+    Carve tail{static_cast<char*>(slot.ptr) + kScratchBytes};
+    const bool small = N <= RES_MAX_ROWS;
+    const size_t partBytes = (size_t)grid * (small ? 36 : 24) * sizeof(double);
+    K.partials = DBuf::viewOf(tail.take(partBytes), partBytes);
+    K.state = DBuf::viewOf(tail.take(sizeof(SolveState)), sizeof(SolveState));
+    K.xSave = DBuf();
+    if (small) {
+        // a resident solve's saved start, where it fits: without it the solve runs by launches
+        const size_t base = cv.off;
+        DBuf save = view(3 * n6 * 8);
+        if (cv.off <= kScratchBytes) K.xSave = std::move(save);
+        else cv.off = base;
+    }
     if (cv.off > kScratchBytes) {
         K.r = DBuf(); K.r0 = DBuf(); K.p = DBuf(); K.v = DBuf(); K.t = DBuf();
         K.rs = DBuf(); K.r0s = DBuf(); K.ps = DBuf(); K.vs = DBuf(); K.ts = DBuf(); K.es = DBuf();

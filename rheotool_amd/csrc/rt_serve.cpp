@@ -65,11 +65,11 @@ struct rt_server {
     int64_t nextTicket = 1;
     std::string defaultControls = "solver PBiCGStab; preconditioner DILU; tolerance 1e-10; relTol 0; "
                                   "maxIter 1000; precision mixed;";
-    // batched Krylov rounds: one group per (precision, preconditioner form),
-    // on the stream of a context of the server's own
+    // batched Krylov rounds: one group per (resident or not, precision,
+    // preconditioner form), on the stream of a context of the server's own
     bool batching = true;
     rt_ctx* gctx = nullptr;
-    SolveGroup groups[4];
+    SolveGroup groups[8];
     std::map<Krylov*, Request*> byKrylov;
 };
 
@@ -142,12 +142,13 @@ void admit(rt_server* S, Request* r, int slot) {
         modelCorrectBegin(r->model->impl, r->deltaT, r->gradU);
         RT_HIP(hipEventCreateWithFlags(&r->done, hipEventDisableTiming));
         r->state = Request::RUNNING;
-        bool mixed = false, rb = false;
-        if (S->batching && solve_groupable(M.kry, &mixed, &rb)) {
-            const int g = (mixed ? 2 : 0) + (rb ? 1 : 0);
+        bool mixed = false, rb = false, resident = false;
+        if (S->batching && solve_groupable(M.kry, &mixed, &rb, &resident)) {
+            const int g = (resident ? 4 : 0) + (mixed ? 2 : 0) + (rb ? 1 : 0);
             SolveGroup& G = S->groups[g];
             G.mixed = mixed;
             G.rb = rb;
+            G.resident = resident;
             group_join(G, M.kry, c->impl.stream);
             r->group = g;
             S->byKrylov[&M.kry] = r;
