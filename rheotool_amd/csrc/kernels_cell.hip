@@ -594,8 +594,12 @@ __global__ void __launch_bounds__(FBLK) k_fin_assemble(AssembleArgs a, int G) {
     if (on) {
         finish_initial(cs, a.ctl, sums[c], sums[6 + c], sums[12 + c]);
         cs.store(a.cs[c]);
+        if (a.host) cs.store(a.host->c[c]);
     }
-    if (c == 6) *a.nnzOut = sums[18];
+    if (c == 6) {
+        *a.nnzOut = sums[18];
+        if (a.host) a.host->misc[0] = sums[18];
+    }
 }
 
 // ----------------------------------------------------------- calcEig + tau
@@ -704,9 +708,10 @@ __device__ __forceinline__ bool orthonormalize3(double* W) {
 
 __global__ void __launch_bounds__(BLK) k_eig_tau(int32_t N, ModelParams p, const double* __restrict__ theta,
                                                  double* __restrict__ eigVal, double* __restrict__ eigVec,
-                                                 double* __restrict__ tau, const double* __restrict__ fOld) {
+                                                 double* __restrict__ tau, const double* __restrict__ fOld,
+                                                 SolveGate gate) {
     const int64_t r = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (r >= N) return;
+    if (r >= N || (gate.done && *gate.done != gate.epoch)) return;
     double th[6], ev[3], V[9], W[9];
     ld6(theta + (int64_t)NCMP * r, th);
 #pragma unroll
@@ -804,9 +809,27 @@ __global__ void k_eigvals_to_tensor(int32_t N, const double* __restrict__ ev,
     t[5] = t[6] = t[7] = 0.0;
     t[8] = ev[2 * (int64_t)N + r];
 }
-__global__ void k_add(int64_t n, const double* __restrict__ in, double* __restrict__ out) {
+// multiMode's tau: the modes' fields summed in their order, from 0; SUM_MAX a
+// launch (one pass over each field: filling the sum and adding a mode at a time
+// read and wrote it once more per mode)
+constexpr int SUM_MAX = 8;
+struct SumArgs {
+    const double* in[SUM_MAX];
+    int n;
+    bool first;
+};
+__global__ void __launch_bounds__(BLK) k_sum(int64_t n2, SumArgs a, double2* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (i < n) out[i] = out[i] + in[i];
+    if (i >= n2) return;
+    double2 v[SUM_MAX];
+#pragma unroll
+    for (int k = 0; k < SUM_MAX; ++k)
+        if (k < a.n) v[k] = reinterpret_cast<const double2*>(a.in[k])[i];
+    double2 s = a.first ? make_double2(0.0, 0.0) : out[i];
+#pragma unroll
+    for (int k = 0; k < SUM_MAX; ++k)
+        if (k < a.n) s.x = s.x + v[k].x, s.y = s.y + v[k].y;
+    out[i] = s;
 }
 
 __global__ void k_fill(double* p, int64_t n, double v) {
@@ -1411,13 +1434,13 @@ void launch_assemble(Ctx* ctx, const AssembleArgs& a, int grid) {
     RT_HIP(hipGetLastError());
 }
 void launch_eig_tau(Ctx* ctx, int32_t N, const ModelParams& prm, const double* theta,
-                    double* eigVal, double* eigVec, double* tau, const double* fOld) {
+                    double* eigVal, double* eigVec, double* tau, const double* fOld, SolveGate gate) {
     // theta 48 + previous eigenvectors 72 in; eigenvalues 24, eigenvectors 72, tau 48 out
     // (tau NULL: the eigen state only)
     const double tauBytes = tau ? 48 + (modelKeepsFactor(prm.kind) ? 8 : 0) : 0;
     ProfScope ps(ctx, "k_eig_tau", (double)N * (48 + 72 + 24 + 72 + tauBytes));
     hipLaunchKernelGGL(k_eig_tau, dim3(nblk(N)), dim3(BLK), 0, ctx->stream, N, prm, theta, eigVal,
-                       eigVec, tau, fOld);
+                       eigVec, tau, fOld, gate);
     RT_HIP(hipGetLastError());
 }
 void launch_aos_to_soa(Ctx* ctx, int32_t N, int nc, const double* aos, const int32_t* perm, double* soa) {
@@ -1443,10 +1466,15 @@ void launch_copy(Ctx* ctx, const void* src, void* dst, size_t bytes) {
     hipLaunchKernelGGL(k_copy, dim3(grid), dim3(BLK), 0, ctx->stream, n16, (const double2*)src, (double2*)dst);
     RT_HIP(hipGetLastError());
 }
-void launch_add(Ctx* ctx, int64_t n, const double* in, double* out) {
+void launch_sum(Ctx* ctx, int64_t n, const std::vector<const double*>& in, double* out) {
     if (n <= 0) return;
-    ProfScope ps(ctx, "k_add", (double)n * 24);
-    hipLaunchKernelGGL(k_add, dim3((unsigned)((n + BLK - 1) / BLK)), dim3(BLK), 0, ctx->stream, n, in, out);
+    for (size_t k = 0; k < in.size() || k == 0; k += SUM_MAX) {
+        SumArgs a{};
+        a.first = k == 0;
+        for (a.n = 0; a.n < SUM_MAX && k + a.n < in.size(); ++a.n) a.in[a.n] = in[k + a.n];
+        ProfScope ps(ctx, "k_sum", (double)n * 8 * (a.n + (a.first ? 1 : 2)));
+        hipLaunchKernelGGL(k_sum, dim3(nblk(n / 2)), dim3(BLK), 0, ctx->stream, n / 2, a, (double2*)out);
+    }
     RT_HIP(hipGetLastError());
 }
 

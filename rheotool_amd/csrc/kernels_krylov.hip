@@ -20,6 +20,8 @@
 // solve of the FP64-refined "mixed" solve).  x (theta), b, the matrix used
 // for the true residual and the grid-level reductions are FP64; per-thread
 // partial sums use T.
+#include <cstring>
+
 #include "rt_device.h"
 
 namespace rt {
@@ -51,6 +53,7 @@ struct KryArgs {
     const double* atval;
     double* partials;
     CompState* cs;
+    CompState* host;     // page-locked copy of the records the host reads, or NULL
     int32_t valid[6];
     KryCtl ctl;
     int32_t G;           // workgroups of the row kernels (partials rows)
@@ -308,6 +311,7 @@ __device__ __forceinline__ void k_fin_residual_body(const KryArgs<T>& a, double*
         }
     }
     cs.store(a.cs[c]);
+    if (a.host) cs.store(a.host[c]);
 }
 
 template <class T, int MODE>
@@ -678,6 +682,7 @@ __device__ __forceinline__ void k_fin_xr_body(const KryArgs<T>& a, double* lds) 
         }
     }
     cs.store(a.cs[c]);
+    if (a.host) cs.store(a.host[c]);
 }
 
 template <class T>
@@ -1100,6 +1105,7 @@ __device__ __forceinline__ void k_fin_bicg_w_body(const KryArgs<T>& a, double* l
         cs.alpha = cs.rho / sums[c];
     }
     cs.store(a.cs[c]);
+    if (a.host) cs.store(a.host[c]);
 }
 
 template <class T>
@@ -1222,6 +1228,7 @@ __device__ __forceinline__ void k_fin_bicg_xr_body(const KryArgs<T>& a, double* 
         }
     }
     cs.store(a.cs[c]);
+    if (a.host) cs.store(a.host[c]);
 }
 
 template <class T>
@@ -1341,8 +1348,9 @@ struct ResArgs {
     int32_t P, pg, Gw;    // workgroups; row-kernel workgroups of the pointwise and first-colour passes
     int32_t X;            // row-kernel workgroups with a tile: the first X of a.G
     int32_t doScale;
-    uint32_t maxPolls;
+    uint32_t maxPolls, epoch;  // epoch: this launch, what resDone or resFail is set to
     SolveState* st;
+    SolveState* host;     // the page-locked copy, or NULL
     // NULL when P = 1: x [N][6], and where the assembly's residual starts the
     // solve (not red-black, whose first sweep makes it) r0 and PBiCG's r
     double* xSave;
@@ -1558,6 +1566,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     __syncthreads();
     KryArgs<T> a = m.a, b = m.b, sw = m.s;
     a.cs = b.cs = sw.cs = cs;
+    a.host = b.host = sw.host = nullptr;
     // the x/r pass has partial sums of its own: the t pass's may still be read
     KryArgs<T> ax = a, af = a;
     ax.partials = af.partials = a.partials + (int64_t)24 * a.G;
@@ -1910,8 +1919,15 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
         }
     }
     if (ok && p == 0)
-        for (int i = threadIdx.x; i < (int)(sizeof(cs) / 8); i += RBLK)
-            reinterpret_cast<double*>(m.a.cs)[i] = reinterpret_cast<const double*>(cs)[i];
+        for (int i = threadIdx.x; i < (int)(sizeof(cs) / 8); i += RBLK) {
+            const double w = reinterpret_cast<const double*>(cs)[i];
+            reinterpret_cast<double*>(m.a.cs)[i] = w;
+            if (m.host) reinterpret_cast<double*>(m.host->c)[i] = w;
+        }
+    if (threadIdx.x == 0 && (!ok || p == 0)) {
+        (ok ? m.st->resDone : m.st->resFail) = m.epoch;
+        if (m.host) (ok ? m.host->resDone : m.host->resFail) = m.epoch;
+    }
     if (ok) res_leave(bar);
 }
 
@@ -2051,7 +2067,7 @@ struct SolveRun {
     // the whole solve in one launch of P workgroups (k_solve_one / k_solve_group)
     bool resident = false, resLaunched = false;
     int P = 1, X = 1, form = 0;
-    uint32_t maxPolls = 0;
+    uint32_t maxPolls = 0, epoch = 0;
     double* xSave = nullptr;
     SolveState* st = nullptr;
     ~SolveRun() {
@@ -2185,6 +2201,7 @@ void fill_args(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     }
     a.partials = K.partials.as<double>();
     a.cs = st->c;
+    a.host = R.ownsHost ? R.hostState->c : nullptr;
     for (int c = 0; c < 6; ++c) a.valid[c] = sa.valid[c];
     a.ctl = kryCtl(*sa.ctl, mixed, m);
     R.G = solve_grid<T>(ctx, K.grid, a.ctl.rb != 0, sa.ctl->solver == SV_PBICG);
@@ -2501,7 +2518,9 @@ ResArgs<T> resident_args(SolveRun& R) {
     m.X = R.X;
     m.doScale = R.needScale ? 1 : 0;
     m.maxPolls = R.maxPolls;
+    m.epoch = R.epoch = ++R.ctx->resEpoch;
     m.st = R.st;
+    m.host = R.ownsHost ? R.hostState : nullptr;
     m.xSave = R.xSave;
     return m;
 }
@@ -2522,14 +2541,39 @@ void launch_resident(Ctx* ctx, SolveRun& R) {
 // rounds a non-blocking advance queues per host round trip
 constexpr int kRoundsAhead = 3;
 
+// The records' way to the host: the kernels write the page-locked copy
+// themselves, so only the event is left (a copy was a kernel of 2 to 5 us and a
+// launch in every round trip); a caller's pageable block is copied to.
 void queue_pull(Ctx* ctx, Krylov& K, SolveRun& R) {
-    SolveState* st = K.state.as<SolveState>();
-    RT_HIP(hipMemcpyAsync(R.hostState, st, sizeof(SolveState), hipMemcpyDeviceToHost, ctx->stream));
+    if (!R.ownsHost)
+        RT_HIP(hipMemcpyAsync(R.hostState, K.state.as<SolveState>(), sizeof(SolveState), hipMemcpyDeviceToHost,
+                              ctx->stream));
     if (R.ev) RT_HIP(hipEventRecord(R.ev, ctx->stream));
     R.pending = true;
 }
 
 }  // namespace
+
+SolveState* solve_prepare(Ctx* ctx, Krylov& K, SolveState* hostStatus) {
+    if (K.run && hostStatus && K.run->hostState != hostStatus) K.run.reset();
+    if (!K.run) {
+        static_assert(sizeof(SolveState) <= Ctx::kPinnedBlock, "status block too small");
+        K.run.reset(new SolveRun);
+        K.run->ctx = ctx;
+        if (hostStatus) {
+            // the caller's pageable block, no event: a blocking solve waits on
+            // the stream (the no-allocation path)
+            K.run->hostState = hostStatus;
+        } else {
+            K.run->hostState = static_cast<SolveState*>(ctx->takePinnedBlock());
+            memset(static_cast<void*>(K.run->hostState), 0, sizeof(SolveState));
+            K.run->ownsHost = true;
+            RT_HIP(hipEventCreateWithFlags(&K.run->ev, hipEventDisableTiming));
+        }
+        K.run->host = K.run->hostState->c;
+    }
+    return K.run->ownsHost ? K.run->hostState : nullptr;
+}
 
 void solve_begin(Ctx* ctx, const SolveArgs& sa) {
     Mesh& m = *sa.mesh;
@@ -2538,23 +2582,9 @@ void solve_begin(Ctx* ctx, const SolveArgs& sa) {
     const bool bicg = sa.ctl->solver == SV_PBICG;
     K.ensure(m, mixed, bicg);
     if (bicg && !sa.atval) throw Error{RT_E_BAD_ARG, "PBiCG needs the transposed matrix"};
-    if (K.run && sa.hostStatus && K.run->hostState != sa.hostStatus) K.run.reset();
-    if (!K.run) {
-        static_assert(sizeof(SolveState) <= Ctx::kPinnedBlock, "status block too small");
-        K.run.reset(new SolveRun);
-        K.run->ctx = ctx;
-        if (sa.hostStatus) {
-            // the caller's pageable block, no event: a blocking solve waits on
-            // the stream (the no-allocation path)
-            K.run->hostState = sa.hostStatus;
-        } else {
-            K.run->hostState = static_cast<SolveState*>(ctx->takePinnedBlock());
-            K.run->ownsHost = true;
-            RT_HIP(hipEventCreateWithFlags(&K.run->ev, hipEventDisableTiming));
-        }
-        K.run->host = K.run->hostState->c;
-    }
+    (void)solve_prepare(ctx, K, sa.hostStatus);
     SolveRun& R = *K.run;
+    R.ctx = ctx;
     R.mixed = mixed;
     R.G = K.grid;
     R.pgrid = std::min<int>(K.grid, (int)kblk(m.N));
@@ -2607,19 +2637,13 @@ void open_components(const SolveRun& R, double& nAct, double& nRef) {
 // workgroup's wait that gave up leaves the counters set; the records then
 // either are final (it gave up behind the last barrier, which every workgroup
 // had reached) or still the start's, and the solve is run by launches from the
-// saved x.
+// saved vectors.
 bool resident_done(Ctx* ctx, SolveRun& R) {
-    double nAct, nRef;
-    open_components(R, nAct, nRef);
-    uint32_t any = R.hostState->bar[0] | R.hostState->bar[2];
-    for (const auto& x : R.hostState->barL2) any |= x[0] | x[1];
-    const bool gaveUp = (any & RES_FAIL) != 0;
-    if (gaveUp) {
+    if (R.hostState->resFail == R.epoch) {
         launch_fill(ctx, reinterpret_cast<double*>(R.st->bar), sizeof(R.st->bar) / 8, 0.0);
         launch_fill(ctx, reinterpret_cast<double*>(R.st->barL2), sizeof(R.st->barL2) / 8, 0.0);
     }
-    if (nAct == 0 && nRef == 0) return true;
-    if (!gaveUp) return true;  // the round limit
+    if (R.hostState->resDone == R.epoch) return true;
     const size_t n6 = (size_t)6 * (size_t)R.N;
     const size_t w = R.mixed ? sizeof(float) : sizeof(double);
     const size_t nv = (n6 * w + 15) / 16 * 16;  // whole 16-byte words; the buffers are padded to 256
@@ -2633,6 +2657,19 @@ bool resident_done(Ctx* ctx, SolveRun& R) {
 
 }  // namespace
 
+bool solve_queue_resident(Ctx* ctx, Krylov& K, SolveGate& gate) {
+    SolveRun& R = *K.run;
+    if (!R.resident || R.resLaunched || R.done) return false;
+    if (R.mixed) launch_resident<float>(ctx, R);
+    else launch_resident<double>(ctx, R);
+    queue_pull(ctx, K, R);
+    gate = SolveGate{&R.st->resDone, R.epoch};
+    return true;
+}
+
+bool solve_resident(const Krylov& K) { return K.run->resident; }
+SolveGate solve_gate(const Krylov& K) { return SolveGate{&K.run->st->resDone, K.run->epoch}; }
+
 bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
     SolveRun& R = *K.run;
     if (R.done) return true;
@@ -2643,12 +2680,8 @@ bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
         queue_pull(ctx, K, R);
         return false;
     }
-    if (R.resident && !R.resLaunched) {
-        if (R.mixed) launch_resident<float>(ctx, R);
-        else launch_resident<double>(ctx, R);
-        queue_pull(ctx, K, R);
-        return false;
-    }
+    SolveGate gate;
+    if (solve_queue_resident(ctx, K, gate)) return false;
     if (R.pending) {
         if (block) {
             if (R.ev) RT_HIP(hipEventSynchronize(R.ev));

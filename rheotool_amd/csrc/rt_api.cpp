@@ -572,6 +572,7 @@ void modelCorrectBegin(Model& M, double deltaT, const double* gradU, int iterati
     a.partials = M.kry.partials.as<double>();
     a.cs = st->c;
     a.nnzOut = &st->misc[0];
+    a.host = solve_prepare(ctx, M.kry);
     for (int q = 0; q < 6; ++q) M.valid6[q] = M.scalar() ? (q == 0 ? 1 : -1) : m.valid[q];
     for (int q = 0; q < 6; ++q) a.valid[q] = M.valid6[q];
     a.rD = M.kry.rD.as<double>();
@@ -610,13 +611,16 @@ void modelCorrectBegin(Model& M, double deltaT, const double* gradU, int iterati
     solve_begin(ctx, sa);
 }
 
+// calcEig and tau (the fluidity has neither)
+void modelEigTau(Model& M, SolveGate gate) {
+    if (M.scalar()) return;
+    launch_eig_tau(M.ctx, M.mesh->N, M.prm, M.theta.as<double>(), M.eigVal.as<double>(), M.eigVec.as<double>(),
+                   M.tau.as<double>(), modelKeepsFactor(M.prm.kind) ? M.fOld.as<double>() : nullptr, gate);
+}
+
 void modelCorrectFinish(Model& M) {
-    Ctx* ctx = M.ctx;
     solve_finish(M.kry, M.perf);
-    if (M.scalar()) return;  // the fluidity has no eigen state or tau
-    launch_eig_tau(ctx, M.mesh->N, M.prm, M.theta.as<double>(), M.eigVal.as<double>(),
-                   M.eigVec.as<double>(), M.tau.as<double>(),
-                   modelKeepsFactor(M.prm.kind) ? M.fOld.as<double>() : nullptr);
+    modelEigTau(M, SolveGate{});
 }
 
 bool modelCorrectAdvance(Model& M, bool block) {
@@ -627,6 +631,16 @@ bool modelCorrectAdvance(Model& M, bool block) {
 
 void modelCorrect(Model& M, double deltaT, const double* gradU, int iteration) {
     modelCorrectBegin(M, deltaT, gradU, iteration);
+    SolveGate gate;
+    if (solve_queue_resident(M.ctx, M.kry, gate)) {
+        // the whole step is queued; the eigen/tau kernel runs if the solve finishes
+        modelEigTau(M, gate);
+        RT_HIP(hipStreamSynchronize(M.ctx->stream));
+        if (solve_advance(M.ctx, M.kry, true) && solve_resident(M.kry)) {
+            solve_finish(M.kry, M.perf);
+            return;
+        }
+    }
     while (!modelCorrectAdvance(M, true)) {
     }
     RT_HIP(hipStreamSynchronize(M.ctx->stream));
@@ -1060,6 +1074,13 @@ void allocModelState(Model& M) {
     }
 }
 
+// tau of a multiMode model: the sum of the modes' tau (multiMode.C:219-227)
+void sumModes(Model& M) {
+    std::vector<const double*> in;
+    for (const rt_model* mode : M.modes) in.push_back(mode->impl.tau.as<double>());
+    launch_sum(M.ctx, (int64_t)6 * M.mesh->N, in, M.tau.as<double>());
+}
+
 // multiMode models whose modes' solves may run as one group: two or more
 // modes on the model's own context, no fluidity equation (BMP solves it
 // before theta), and no profiling (a profiled run charges each launch to
@@ -1253,6 +1274,7 @@ int rt_model_correct_iter(rt_model* model, double deltaT, const double* gradU, i
                 }
             }
             bool same = true, mixed0 = false, rb0 = false, res0 = false;
+            bool summed = false;  // tau is the sum of the modes' final tau
             for (size_t i = 0; i < M.modes.size(); ++i) {
                 bool mx = false, rb = false, res = false;
                 if (!solve_groupable(M.modes[i]->impl.kry, &mx, &rb, &res)) same = false;
@@ -1271,20 +1293,36 @@ int rt_model_correct_iter(rt_model* model, double deltaT, const double* gradU, i
                 G.resident = res0;
                 for (rt_model* mode : M.modes) group_join(G, mode->impl.kry, M.ctx->stream);
                 std::vector<Krylov*> done;
+                if (res0) {
+                    // the whole step is queued: the solves in one launch, each
+                    // mode's eigen/tau (run if its solve finishes) and the sum
+                    group_advance(G, done);
+                    for (rt_model* mode : M.modes) modelEigTau(mode->impl, solve_gate(mode->impl.kry));
+                    sumModes(M);
+                    summed = true;
+                }
                 while (!G.members.empty()) {
                     RT_HIP(hipStreamSynchronize(M.ctx->stream));  // the queued rounds' states are back
                     done.clear();
                     group_advance(G, done);
                     for (Krylov* K : done)
-                        for (rt_model* mode : M.modes)
-                            if (&mode->impl.kry == K) modelCorrectFinish(mode->impl);
+                        for (rt_model* mode : M.modes) {
+                            if (&mode->impl.kry != K) continue;
+                            if (solve_resident(*K)) {
+                                solve_finish(*K, mode->impl.perf);
+                            } else {
+                                modelCorrectFinish(mode->impl);
+                                summed = false;
+                            }
+                        }
                 }
-                RT_HIP(hipStreamSynchronize(M.ctx->stream));  // the group's tables are read no more
+                // the group's tables are read no more
+                if (!summed) RT_HIP(hipStreamSynchronize(M.ctx->stream));
             }
-            const int64_t n = (int64_t)6 * M.mesh->N;
-            launch_fill(M.ctx, M.tau.as<double>(), n, 0.0);
-            for (rt_model* mode : M.modes) launch_add(M.ctx, n, mode->impl.tau.as<double>(), M.tau.as<double>());
-            RT_HIP(hipStreamSynchronize(M.ctx->stream));
+            if (!summed) {
+                sumModes(M);
+                RT_HIP(hipStreamSynchronize(M.ctx->stream));
+            }
         });
         if (rc != RT_OK) return rc;
         for (rt_model* mode : M.modes)
@@ -1305,9 +1343,7 @@ int rt_model_correct_iter(rt_model* model, double deltaT, const double* gradU, i
             if (rc == RT_W_NOT_CONVERGED) worst = rc;
         }
         const int rc = guarded(M.ctx, [&] {
-            const int64_t n = (int64_t)6 * M.mesh->N;
-            launch_fill(M.ctx, M.tau.as<double>(), n, 0.0);
-            for (rt_model* mode : M.modes) launch_add(M.ctx, n, mode->impl.tau.as<double>(), M.tau.as<double>());
+            sumModes(M);
         });
         return rc != RT_OK ? rc : worst;
     }

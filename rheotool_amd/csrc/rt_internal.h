@@ -68,6 +68,7 @@ struct Ctx {
     rt_ctx* handle = nullptr;
     int device = 0;
     int numCUs = 256;
+    uint32_t resEpoch = 0;  // resident launches so far
     int xcd = 0;  // where its resident solves run: contexts take turns
     hipStream_t stream = nullptr;
     size_t budget = 0, inUse = 0;
@@ -235,6 +236,7 @@ struct SolveState {
     CompState c[6];
     int32_t anyActive;
     double misc[8];  // misc[0]: ELL entries in live slots of the solve's matrix (set by the assembly)
+    uint32_t resDone, resFail;  // the resident launch (its epoch) that finished, whose wait gave up
     // barriers of a resident solve, zero between launches (top bit: a wait gave
     // up).  bar: [0] entered, [1] left, [2] the XCDs' barrier, [8 + x] workgroups on
     // XCD x; barL2[x]: XCD x's own, a cache line each (arrivals, barriers, departures)
@@ -413,6 +415,7 @@ struct AssembleArgs {
     double* partials;     // [grid][19] residual sums, entries in live slots
     CompState* cs;
     double* nnzOut;       // SolveState::misc[0]
+    SolveState* host;     // page-locked copy of the solve's records, or NULL
     int32_t valid[6];
     // initial residual of the solve, fused into the assembly
     void* r;              // [N][6] Krylov precision: r0 of PBiCGStab, rA of PBiCG, NULL for none
@@ -437,8 +440,14 @@ void launch_div_tau(Ctx* ctx, const AssembleArgs& a, const double* tau, const do
                     int grid);
 // tauTotal() -> out [N][6]
 void launch_tau_total(Ctx* ctx, const AssembleArgs& a, const double* tau, double etaS, double* out, int grid);
+// A kernel queued behind a resident solve does nothing if that launch gave up
+// (*done is not its epoch); done NULL: no condition
+struct SolveGate {
+    const uint32_t* done = nullptr;
+    uint32_t epoch = 0;
+};
 void launch_eig_tau(Ctx* ctx, int32_t N, const ModelParams& prm, const double* theta,
-                    double* eigVal, double* eigVec, double* tau, const double* fOld);
+                    double* eigVal, double* eigVec, double* tau, const double* fOld, SolveGate gate = SolveGate{});
 void launch_aos_to_soa(Ctx* ctx, int32_t N, int ncomp, const double* aos, const int32_t* perm,
                        double* soa);
 void launch_soa_to_aos(Ctx* ctx, int32_t N, int ncomp, const double* soa, const int32_t* perm,
@@ -456,8 +465,8 @@ void launch_eigvals_from_tensor(Ctx* ctx, int32_t N, const double* aos9, const i
                                 double* eigVal);
 void launch_eigvals_to_tensor(Ctx* ctx, int32_t N, const double* eigVal, const int32_t* perm,
                               double* aos9);
-// out[i] += in[i], i < n
-void launch_add(Ctx* ctx, int64_t n, const double* in, double* out);
+// out[i] = 0 + in[0][i] + in[1][i] + ..., i < n (n even)
+void launch_sum(Ctx* ctx, int64_t n, const std::vector<const double*>& in, double* out);
 void launch_fill(Ctx* ctx, double* p, int64_t n, double v);
 void launch_copy(Ctx* ctx, const void* src, void* dst, size_t bytes);
 
@@ -511,6 +520,14 @@ void solve_lockstep(Ctx* ctx, const SolveArgs& a, rt_solver_perf perf[6]);
 // host (block = false returns false immediately when it is not yet) and
 // returns true when every component is finished; finish fills perf.
 void solve_begin(Ctx* ctx, const SolveArgs& a);
+// the host's copy of the records, made before the assembly that fills it (NULL:
+// a caller's pageable block)
+SolveState* solve_prepare(Ctx* ctx, Krylov& K, SolveState* hostStatus = nullptr);
+// a begun solve that runs as one resident launch: queues it, true; work queued
+// behind it with its gate runs only if it finishes
+bool solve_queue_resident(Ctx* ctx, Krylov& K, SolveGate& gate);
+SolveGate solve_gate(const Krylov& K);  // of a resident solve queued by its group
+bool solve_resident(const Krylov& K);   // a finished solve: its resident launch did it
 bool solve_advance(Ctx* ctx, Krylov& K, bool block);
 void solve_finish(Krylov& K, rt_solver_perf perf[6]);
 
@@ -561,6 +578,7 @@ void noallocInit(int device);
 // current iterate with the saved oldTime
 void modelCorrectBegin(Model& M, double deltaT, const double* gradU, int iteration = -1);
 bool modelCorrectAdvance(Model& M, bool block);
+void modelEigTau(Model& M, SolveGate gate);  // calcEig and tau (launched)
 // after the solve: its performance record, then calcEig and tau (launched)
 void modelCorrectFinish(Model& M);
 void modelCorrect(Model& M, double deltaT, const double* gradU, int iteration = -1);
