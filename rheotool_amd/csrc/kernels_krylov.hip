@@ -1988,7 +1988,7 @@ KryCtl kryCtl(const Controls& C, bool mixed, const Mesh& m) {
     return k;
 }
 
-void Krylov::ensure(Mesh& m, bool mixed, bool bicg) {
+void Krylov::ensure(Ctx* run, Mesh& m, bool mixed, bool bicg) {
     if (!ctx) ctx = m.ctx;
     const size_t vec = (size_t)6 * m.N;
     if (noAlloc) {
@@ -2010,7 +2010,10 @@ void Krylov::ensure(Mesh& m, bool mixed, bool bicg) {
         xSave = DBuf();
         if (N <= RES_MAX_ROWS && grid > RSUB) xSave = ctx->alloc(3 * vec * 8);
         state = ctx->alloc(sizeof(SolveState));
-        RT_HIP(hipMemsetAsync(state.p, 0, sizeof(SolveState), ctx->stream));
+        // on the solve's stream: on the mesh's, behind other work, the zeros could
+        // land on records the assembly had written
+        static_assert(sizeof(SolveState) % 8 == 0, "filled by 8-byte words");
+        launch_fill(run, state.as<double>(), sizeof(SolveState) / 8, 0.0);
         rD = ctx->alloc(std::max<size_t>(1, (size_t)m.N) * sizeof(double));
     }
     if (!mixed && !r.p) {
@@ -2580,7 +2583,7 @@ void solve_begin(Ctx* ctx, const SolveArgs& sa) {
     Krylov& K = *sa.kry;
     const bool mixed = sa.ctl->mixed;
     const bool bicg = sa.ctl->solver == SV_PBICG;
-    K.ensure(m, mixed, bicg);
+    K.ensure(ctx, m, mixed, bicg);
     if (bicg && !sa.atval) throw Error{RT_E_BAD_ARG, "PBiCG needs the transposed matrix"};
     (void)solve_prepare(ctx, K, sa.hostStatus);
     SolveRun& R = *K.run;

@@ -516,7 +516,7 @@ void modelCorrectBegin(Model& M, double deltaT, const double* gradU, int iterati
     Mesh& m = *M.mesh;
     const int32_t N = m.N;
     const bool bicg = M.ctl.solver == SV_PBICG;
-    M.kry.ensure(m, M.ctl.mixed, bicg);
+    M.kry.ensure(ctx, m, M.ctl.mixed, bicg);
     if (!M.diag.p) {
         M.diag = ctx->alloc((size_t)N * 8);
         M.aval = ctx->alloc((size_t)std::max<int64_t>(1, m.nEll) * 8);
@@ -1574,7 +1574,7 @@ int rt_symm_solve(rt_ctx* ctx, const rt_mesh* mesh, const rt_ldu_symm* sys, doub
         std::unique_ptr<Krylov> Kp(new Krylov);  // workspace of this call
         Krylov& K = *Kp;
         const bool bicg = ctl.solver == SV_PBICG;
-        K.ensure(m, ctl.mixed, bicg);
+        K.ensure(c, m, ctl.mixed, bicg);
         DBuf dD = c->alloc((size_t)N * 8), dA = c->alloc((size_t)std::max<int64_t>(1, m.nEll) * 8),
              dB = c->alloc((size_t)6 * N * 8), dX = c->alloc((size_t)6 * N * 8),
              dLo = c->alloc((size_t)std::max(1, F) * 8), dUp = c->alloc((size_t)std::max(1, F) * 8);

@@ -276,7 +276,9 @@ struct Krylov {
     // set when the buffers above are views into the no-allocation scratch
     // array: ensure() then refuses to allocate instead of calling hipMalloc
     bool noAlloc = false;
-    void ensure(Mesh& m, bool mixed, bool bicg = false);
+    // run: the context whose stream the solve uses, which a server's slots do not
+    // share with the mesh's (the buffers' owner)
+    void ensure(Ctx* run, Mesh& m, bool mixed, bool bicg = false);
 };
 
 // ------------------------------------------------------------------- model
