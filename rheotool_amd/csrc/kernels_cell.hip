@@ -353,18 +353,28 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(3, 8))
         double offY[6] = {0, 0, 0, 0, 0, 0};
         double divDiag = 0.0, sumOff = 0.0, sumAv = 0.0, netPhi = 0.0;
         const bool haveGrad = a.gradU != nullptr;
+        // A face's loads are a chain (its column, then that row's velocity and
+        // theta), and 12 wavefronts a CU do not cover it: the column comes in
+        // face order, not through the face id and slot, and loads with the slot
+        // and flux one face ahead.  160^3 mixed 790 -> 672 us, 128^3 377 -> 312.
+        // (Two faces' gathers in flight spill 70 to 185 registers.)
+        int32_t ccN = RT_FID_PAD;
+        int slotN = 0;
+        double phN = 0.0;
+        if (width > 0) ccN = a.eCol[base], slotN = a.ellSlot[base], phN = a.ePhi[base];
         for (int k = 0; k < width; ++k) {
             const int64_t e = base + (int64_t)SLICE * k;  // face-order entry
-            const int32_t fid = a.ellFid[e];
-            const int slot = a.ellSlot[e];
-            if (fid == RT_FID_PAD) {
+            const int32_t cc = ccN;
+            const int slot = slotN;
+            const double phRaw = phN;
+            if (k + 1 < width) ccN = a.eCol[e + SLICE], slotN = a.ellSlot[e + SLICE], phN = a.ePhi[e + SLICE];
+            if (cc == RT_FID_PAD) {
                 if (!staged) a.aval[base + (int64_t)SLICE * slot] = 0.0;
                 if (a.atval) a.atval[base + (int64_t)SLICE * slot] = 0.0;
                 continue;
             }
-            const bool own = fid >= 0;
+            const bool own = cc >= 0;
             const int64_t ec = base + (int64_t)SLICE * slot;  // column-order slot
-            const double phRaw = a.ePhi[e];
             netPhi += own ? phRaw : -phRaw;
             const double ph = a.noConv ? 0.0 : phRaw;
             const double upw = ph >= 0 ? 1.0 : 0.0;
@@ -372,7 +382,7 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(3, 8))
             const double upper = (1.0 - upw) * ph;
             const double val = own ? upper : lower;
             if (a.atval) a.atval[ec] = own ? lower : upper;  // A^T: the face's other coefficient
-            const int32_t c = a.ellCol[ec];
+            const int32_t c = own ? cc : ~cc;
             if (staged) {
 #pragma unroll
                 for (int j = 0; j < STAGE_W; ++j)
@@ -928,12 +938,14 @@ __global__ void __launch_bounds__(BLK) k_grad_theta(AssembleArgs a, double* __re
         const int s = r >> 6, lane = r & 63;
         const int64_t base = a.ellOff[s] + lane;
         const int width = a.ellWidth[s];
+        int32_t ccN = width > 0 ? a.eCol[base] : RT_FID_PAD;  // the next face's column loads ahead
         for (int k = 0; k < width; ++k) {
             const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t fid = a.ellFid[e];
-            if (fid == RT_FID_PAD) continue;
-            const bool own = fid >= 0;
-            const int32_t c = a.ellCol[base + (int64_t)SLICE * a.ellSlot[e]];
+            const int32_t cc = ccN;
+            if (k + 1 < width) ccN = a.eCol[e + SLICE];
+            if (cc == RT_FID_PAD) continue;
+            const bool own = cc >= 0;
+            const int32_t c = own ? cc : ~cc;
             double thc[6];
             ld6(a.theta + (int64_t)NCMP * c, thc);
             const double wf = a.eW[e];
@@ -1015,12 +1027,14 @@ __global__ void __launch_bounds__(BLK) k_defc(AssembleArgs a, const double* __re
         const int s = r >> 6, lane = r & 63;
         const int64_t base = a.ellOff[s] + lane;
         const int width = a.ellWidth[s];
+        int32_t ccN = width > 0 ? a.eCol[base] : RT_FID_PAD;  // the next face's column loads ahead
         for (int k = 0; k < width; ++k) {
             const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t fid = a.ellFid[e];
-            if (fid == RT_FID_PAD) continue;
-            const bool own = fid >= 0;
-            const int32_t c = a.ellCol[base + (int64_t)SLICE * a.ellSlot[e]];
+            const int32_t cc = ccN;
+            if (k + 1 < width) ccN = a.eCol[e + SLICE];
+            if (cc == RT_FID_PAD) continue;
+            const bool own = cc >= 0;
+            const int32_t c = own ? cc : ~cc;
             const double ph = a.ePhi[e];
             const double upw = ph >= 0 ? 1.0 : 0.0;
             const double2 cc01 = reinterpret_cast<const double2*>(C4)[2 * (int64_t)c];
@@ -1069,10 +1083,10 @@ void launch_defc(Ctx* ctx, const AssembleArgs& a, int scheme, const double* C4, 
     const double N = a.N, ne = (double)a.nEll;
     {
         // theta own + gathers (counted once), face data, boundary, gradient out
-        ProfScope ps(ctx, "k_grad_theta", N * (48 + 8 + 144) + ne * (4 + 1 + 4 + 32));
+        ProfScope ps(ctx, "k_grad_theta", N * (48 + 8 + 144) + ne * (4 + 32));
         hipLaunchKernelGGL(k_grad_theta, dim3(grid), dim3(BLK), 0, ctx->stream, a, gradTh);
     }
-    ProfScope ps(ctx, "k_defc", N * (48 + 32 + 144 + 48) + ne * (4 + 1 + 4 + 8));
+    ProfScope ps(ctx, "k_defc", N * (48 + 32 + 144 + 48) + ne * (4 + 8));
     switch (scheme) {
     case DS_CUBISTA:
         hipLaunchKernelGGL(k_defc<DS_CUBISTA>, dim3(grid), dim3(BLK), 0, ctx->stream, a, C4, gradTh, souT);
@@ -1138,12 +1152,14 @@ __global__ void __launch_bounds__(BLK) k_div_tau(AssembleArgs a, const double* _
         const int s = r >> 6, lane = r & 63;
         const int64_t base = a.ellOff[s] + lane;
         const int width = a.ellWidth[s];
+        int32_t ccN = width > 0 ? a.eCol[base] : RT_FID_PAD;  // the next face's column loads ahead
         for (int k = 0; k < width; ++k) {
             const int64_t e = base + (int64_t)SLICE * k;
-            const int32_t fid = a.ellFid[e];
-            if (fid == RT_FID_PAD) continue;
-            const bool own = fid >= 0;
-            const int32_t c = a.ellCol[base + (int64_t)SLICE * a.ellSlot[e]];
+            const int32_t cc = ccN;
+            if (k + 1 < width) ccN = a.eCol[e + SLICE];
+            if (cc == RT_FID_PAD) continue;
+            const bool own = cc >= 0;
+            const int32_t c = own ? cc : ~cc;
             double tc[6];
             ld6(tau + (int64_t)NCMP * c, tc);
             const double wf = a.eW[e];
@@ -1262,12 +1278,14 @@ __device__ __forceinline__ void gauss_grad_u(const AssembleArgs& a, int32_t r, d
     const int s = r >> 6, lane = r & 63;
     const int64_t base = a.ellOff[s] + lane;
     const int width = a.ellWidth[s];
+    int32_t ccN = width > 0 ? a.eCol[base] : RT_FID_PAD;  // the next face's column loads ahead
     for (int k = 0; k < width; ++k) {
         const int64_t e = base + (int64_t)SLICE * k;
-        const int32_t fid = a.ellFid[e];
-        if (fid == RT_FID_PAD) continue;
-        const bool own = fid >= 0;
-        const int32_t c = a.ellCol[base + (int64_t)SLICE * a.ellSlot[e]];
+        const int32_t cc = ccN;
+        if (k + 1 < width) ccN = a.eCol[e + SLICE];
+        if (cc == RT_FID_PAD) continue;
+        const bool own = cc >= 0;
+        const int32_t c = own ? cc : ~cc;
         const double wf = a.eW[e];
         const double2 c01 = reinterpret_cast<const double2*>(a.U)[2 * (int64_t)c];
         const double Uc[3] = {c01.x, c01.y, a.U[4 * (int64_t)c + 2]};
@@ -1350,10 +1368,10 @@ void launch_div_tau(Ctx* ctx, const AssembleArgs& a, const double* tau, const do
                     int stab, int lap, double gam, double* G, const double* C4, const double* bDc, double* out,
                     int grid) {
     if (stab != 0) {
-        ProfScope ps(ctx, "k_grad_u", (double)a.N * (32 + 8 + 72) + (double)a.nEll * (4 + 1 + 4 + 32));
+        ProfScope ps(ctx, "k_grad_u", (double)a.N * (32 + 8 + 72) + (double)a.nEll * (4 + 32));
         hipLaunchKernelGGL(k_grad_u, dim3(grid), dim3(BLK), 0, ctx->stream, a, G);
     }
-    ProfScope ps(ctx, "k_div_tau", (double)a.N * (48 + 8 + 24) + (double)a.nEll * (4 + 1 + 4 + 32));
+    ProfScope ps(ctx, "k_div_tau", (double)a.N * (48 + 8 + 24) + (double)a.nEll * (4 + 32));
 #define RT_DIVTAU(S, L) \
     hipLaunchKernelGGL((k_div_tau<S, L>), dim3(grid), dim3(BLK), 0, ctx->stream, a, tau, tauB, rho, gam, G, C4, bDc, out)
     if (stab == 0) RT_DIVTAU(0, 0);
@@ -1366,7 +1384,7 @@ void launch_div_tau(Ctx* ctx, const AssembleArgs& a, const double* tau, const do
 }
 
 void launch_tau_total(Ctx* ctx, const AssembleArgs& a, const double* tau, double etaS, double* out, int grid) {
-    ProfScope ps(ctx, "k_tau_total", (double)a.N * (32 + 8 + 48 + 48) + (double)a.nEll * (4 + 1 + 4 + 32));
+    ProfScope ps(ctx, "k_tau_total", (double)a.N * (32 + 8 + 48 + 48) + (double)a.nEll * (4 + 32));
     hipLaunchKernelGGL(k_tau_total, dim3(grid), dim3(BLK), 0, ctx->stream, a, tau, etaS, out);
     RT_HIP(hipGetLastError());
 }
@@ -1424,7 +1442,7 @@ void launch_assemble(Ctx* ctx, const AssembleArgs& a, int grid) {
     const double w = a.mixed ? 4 : 8;
     const double by = (double)a.N * (48 + 96 + 32 + 8 + 48 + 8 + 8 + (a.r ? 6 * w : 0) + (a.thetaOld ? 48 : 0) +
                                      (a.tauOld ? 48 : 0) + (a.aux ? 8 : 0)) +
-                      (double)a.nEll * (4 + 1 + 4 + 8 + 8 + (a.gradU ? 0 : 24 + 8));
+                      (double)a.nEll * (4 + 1 + 8 + 8 + (a.gradU ? 0 : 24 + 8));
     int g;
     {
         ProfScope ps(ctx, a.mixed ? "k_assemble<f32>" : "k_assemble<f64>", by);

@@ -489,6 +489,7 @@ AssembleArgs meshArgs(Model& M) {
     a.ellCol = m.ellCol.as<int32_t>();
     a.ellFid = m.ellFid.as<int32_t>();
     a.ellSlot = m.ellSlot.as<uint8_t>();
+    a.eCol = m.eCol.as<int32_t>();
     a.eSf = m.eSf.as<double>();
     a.eW = m.eW.as<double>();
     a.ePhi = M.ePhi.as<double>();

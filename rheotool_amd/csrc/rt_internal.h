@@ -165,6 +165,8 @@ struct Mesh {
     DBuf ellCol;    // int32 [nEll]  column order
     DBuf ellFid;    // int32 [nEll]  face order
     DBuf ellSlot;   // uint8 [nEll]  face-order entry -> column-order slot
+    DBuf eCol;      // int32 [nEll]  face order, the column c: c on the owner's row of the
+                    // face, ~c on the neighbour's; RT_FID_PAD for padding
     DBuf eSf;       // double [3][nEll] face order, Sf signed for the row's side
     DBuf eW;        // double [nEll] face order, linear weight of the face
     DBuf bPtr;      // int32 [N+1]   boundary faces of each row (non-empty patches)
@@ -378,6 +380,7 @@ struct AssembleArgs {
     const int32_t* ellCol;
     const int32_t* ellFid;
     const uint8_t* ellSlot;
+    const int32_t* eCol;
     const double* eSf;    // [3][nEll]
     const double* eW;
     const double* ePhi;

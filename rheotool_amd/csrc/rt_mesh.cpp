@@ -286,7 +286,7 @@ void buildMesh(Ctx* ctx, const rt_mesh_desc* d, int renumber, Mesh& m) {
     }
     m.nEll = off[m.nSlices];
     const int64_t nE = std::max<int64_t>(1, m.nEll);
-    std::vector<int32_t> ecol(nE), efid(nE);
+    std::vector<int32_t> ecol(nE), efid(nE), ecolF(nE);
     std::vector<uint8_t> eslot(nE, 0);
     std::vector<double> esf(3 * nE, 0.0), ew(nE, 0.0);
     std::vector<std::pair<int32_t, int>> byCol;  // (column, face-order index)
@@ -298,6 +298,7 @@ void buildMesh(Ctx* ctx, const rt_mesh_desc* d, int renumber, Mesh& m) {
             if (r >= N) {
                 for (int k = 0; k < W; ++k) {
                     ecol[at(k)] = 0;
+                    ecolF[at(k)] = RT_FID_PAD;
                     efid[at(k)] = RT_FID_PAD;
                     eslot[at(k)] = (uint8_t)k;
                 }
@@ -318,12 +319,15 @@ void buildMesh(Ctx* ctx, const rt_mesh_desc* d, int renumber, Mesh& m) {
                 const bool own = fid >= 0;
                 const int64_t f = own ? fid : -(int64_t)fid - 1;
                 efid[at(k)] = fid;
+                const int32_t col = m.perm[rcol[rptr[c] + k]];
+                ecolF[at(k)] = own ? col : ~col;
                 eslot[at(k)] = (uint8_t)slotOf[k];
                 for (int q = 0; q < 3; ++q) esf[q * nE + at(k)] = own ? d->Sf[3 * f + q] : -d->Sf[3 * f + q];
                 ew[at(k)] = d->weights[f];
             }
             for (int k = deg; k < W; ++k) {
                 ecol[at(k)] = r;
+                ecolF[at(k)] = RT_FID_PAD;
                 efid[at(k)] = RT_FID_PAD;
                 eslot[at(k)] = (uint8_t)k;
             }
@@ -358,6 +362,7 @@ void buildMesh(Ctx* ctx, const rt_mesh_desc* d, int renumber, Mesh& m) {
     upload(ctx, m.ellCol, ecol);
     upload(ctx, m.ellFid, efid);
     upload(ctx, m.ellSlot, eslot);
+    upload(ctx, m.eCol, ecolF);
     upload(ctx, m.eSf, esf);
     upload(ctx, m.eW, ew);
     upload(ctx, m.bPtr, bptr);
