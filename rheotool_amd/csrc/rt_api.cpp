@@ -427,7 +427,7 @@ void modelUploadState(Model& M, const double* theta, const double* eigVals, cons
         wait = true;  // phi6 is local
     }
     uploadAos(c, st, theta, (int64_t)6 * N);
-    launch_permute_rows(c, N, 6, 6, st.as<double>(), perm, M.theta.as<double>());
+    launch_rows_in6(c, m, st.as<double>(), M.theta.as<double>());
     if (eigVals) {
         uploadAos(c, st, eigVals, (int64_t)9 * N);
         launch_eigvals_from_tensor(c, N, st.as<double>(), perm, M.eigVal.as<double>());
@@ -438,7 +438,7 @@ void modelUploadState(Model& M, const double* theta, const double* eigVals, cons
     }
     if (tau) {
         uploadAos(c, st, tau, (int64_t)6 * N);
-        launch_permute_rows(c, N, 6, 6, st.as<double>(), perm, M.tau.as<double>());
+        launch_rows_in6(c, m, st.as<double>(), M.tau.as<double>());
     }
     if (wait) RT_HIP(hipStreamSynchronize(c->stream));
     M.hasState = true;
@@ -452,7 +452,7 @@ void modelUploadFlow(Model& M, const double* U, const double* Ub, const double* 
     RT_HIP(hipSetDevice(c->device));
     DBuf& st = staging(c).buf;
     uploadAos(c, st, U, (int64_t)3 * m.N);
-    launch_permute_rows(c, m.N, 3, 4, st.as<double>(), m.permD.as<int32_t>(), M.U.as<double>());
+    launch_rows_in3(c, m, st.as<double>(), M.U.as<double>());
     if (m.NB > 0) {  // [NB][3] -> [3][NB]
         uploadAos(c, st, Ub, (int64_t)3 * m.NB);
         launch_aos_to_soa(c, m.NB, 3, st.as<double>(), nullptr, M.Ub.as<double>());
@@ -1380,8 +1380,8 @@ int rt_model_get(const rt_model* model, int field, double* out) {
         const size_t bytes = (size_t)nc * N * 8;
         if (st.bytes < bytes) st = c->alloc(bytes);
         const int32_t* perm = m.permD.as<int32_t>();
-        if (field == RT_THETA) launch_unpermute_rows(c, N, 6, 6, M.theta.as<double>(), perm, st.as<double>());
-        else if (field == RT_TAU) launch_unpermute_rows(c, N, 6, 6, M.tau.as<double>(), perm, st.as<double>());
+        if (field == RT_THETA) launch_rows_out6(c, m, M.theta.as<double>(), st.as<double>());
+        else if (field == RT_TAU) launch_rows_out6(c, m, M.tau.as<double>(), st.as<double>());
         else if (field == RT_EIGVALS) launch_eigvals_to_tensor(c, N, M.eigVal.as<double>(), perm, st.as<double>());
         else launch_soa_to_aos(c, N, 9, M.eigVec.as<double>(), perm, st.as<double>());
         if (M.scalar()) {  // Phi is component xx
@@ -1443,7 +1443,7 @@ int rt_model_div_tau(rt_model* model, const double* tauB, double* out) {
                        d.as<double>(), grid_for(c, N));
         DBuf& st = staging(c).buf;
         if (st.bytes < (size_t)3 * N * 8) st = c->alloc((size_t)3 * N * 8);
-        launch_unpermute_rows(c, N, 3, 3, d.as<double>(), m.permD.as<int32_t>(), st.as<double>());
+        launch_rows_out3(c, m, d.as<double>(), st.as<double>());
         RT_HIP(hipMemcpyAsync(out, st.p, (size_t)3 * N * 8, hipMemcpyDeviceToHost, c->stream));
         RT_HIP(hipStreamSynchronize(c->stream));
     });
@@ -1509,7 +1509,7 @@ int rt_model_tau_total(rt_model* model, double* out) {
         launch_tau_total(c, meshArgs(F), M.tau.as<double>(), M.prm.etaS, d.as<double>(), grid_for(c, N));
         DBuf& st = staging(c).buf;
         if (st.bytes < (size_t)6 * N * 8) st = c->alloc((size_t)6 * N * 8);
-        launch_unpermute_rows(c, N, 6, 6, d.as<double>(), m.permD.as<int32_t>(), st.as<double>());
+        launch_rows_out6(c, m, d.as<double>(), st.as<double>());
         RT_HIP(hipMemcpyAsync(out, st.p, (size_t)6 * N * 8, hipMemcpyDeviceToHost, c->stream));
         RT_HIP(hipStreamSynchronize(c->stream));
     });
@@ -1590,10 +1590,10 @@ int rt_symm_solve(rt_ctx* ctx, const rt_mesh* mesh, const rt_ldu_symm* sys, doub
         if (bicg) launch_ldu_to_ell(c, m, dUp.as<double>(), dLo.as<double>(), K.atval.as<double>());  // A^T
         DBuf& st = staging(c).buf;
         uploadAos(c, st, src.data(), (int64_t)6 * N);
-        launch_permute_rows(c, N, 6, 6, st.as<double>(), m.permD.as<int32_t>(), dB.as<double>());
+        launch_rows_in6(c, m, st.as<double>(), dB.as<double>());
         RT_HIP(hipStreamSynchronize(c->stream));
         uploadAos(c, st, psi, (int64_t)6 * N);
-        launch_permute_rows(c, N, 6, 6, st.as<double>(), m.permD.as<int32_t>(), dX.as<double>());
+        launch_rows_in6(c, m, st.as<double>(), dX.as<double>());
         // gAverage(psi) per component for the normalisation factor
         SolveState* ss = K.state.as<SolveState>();
         for (int q = 0; q < 6; ++q) {
@@ -1622,7 +1622,7 @@ int rt_symm_solve(rt_ctx* ctx, const rt_mesh* mesh, const rt_ldu_symm* sys, doub
             sa.rDs = dS.as<double>();
         }
         solve_lockstep(c, sa, perf);
-        launch_unpermute_rows(c, N, 6, 6, dX.as<double>(), m.permD.as<int32_t>(), st.as<double>());
+        launch_rows_out6(c, m, dX.as<double>(), st.as<double>());
         RT_HIP(hipMemcpyAsync(psi, st.p, (size_t)6 * N * 8, hipMemcpyDeviceToHost, c->stream));
         RT_HIP(hipStreamSynchronize(c->stream));
     });

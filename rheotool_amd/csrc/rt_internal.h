@@ -178,6 +178,7 @@ struct Mesh {
     DBuf bDc;       // double [NB] patch delta coefficients 1/|n (n & (Cf - C_P))|; empty
                     // unless cell and boundary face centres are given
     DBuf permD;     // int32 [N] internal row -> external cell
+    DBuf rowD;      // int32 [N] external cell -> internal row
     double meanAbsBandwidth = 0;
     // two-colourable cell graphs (hexahedral and quadrilateral meshes) are
     // stored colour by colour: rows [0, nRed) have only neighbours in
@@ -457,13 +458,13 @@ void launch_aos_to_soa(Ctx* ctx, int32_t N, int ncomp, const double* aos, const 
                        double* soa);
 void launch_soa_to_aos(Ctx* ctx, int32_t N, int ncomp, const double* soa, const int32_t* perm,
                        double* aos);
-// gather rows of an interleaved [N][nc] array: out[r] = in[perm[r]] (perm null: copy),
-// padding the destination stride ncOut >= nc with zeros
-void launch_permute_rows(Ctx* ctx, int32_t N, int nc, int ncOut, const double* in, const int32_t* perm,
-                         double* out);
-// scatter rows back: out[perm[r]] = in[r] (first nc of ncIn components)
-void launch_unpermute_rows(Ctx* ctx, int32_t N, int ncIn, int nc, const double* in, const int32_t* perm,
-                           double* out);
+// interleaved rows between the caller's cell order and the device's row order:
+// in6/out6 of six components, out3 of three, in3 three into rows of four (the
+// last one zero)
+void launch_rows_in6(Ctx* ctx, const Mesh& m, const double* in, double* out);
+void launch_rows_in3(Ctx* ctx, const Mesh& m, const double* in, double* out);
+void launch_rows_out6(Ctx* ctx, const Mesh& m, const double* in, double* out);
+void launch_rows_out3(Ctx* ctx, const Mesh& m, const double* in, double* out);
 // per-entry face flux: ePhi[e] = phi[face of entry e]
 void launch_face_to_entry(Ctx* ctx, const Mesh& m, const double* phi, double* ePhi);
 void launch_eigvals_from_tensor(Ctx* ctx, int32_t N, const double* aos9, const int32_t* perm,

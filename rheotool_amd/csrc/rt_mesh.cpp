@@ -395,6 +395,7 @@ void buildMesh(Ctx* ctx, const rt_mesh_desc* d, int renumber, Mesh& m) {
         upload(ctx, m.bDc, dcb);
     }
     upload(ctx, m.permD, m.iperm);
+    upload(ctx, m.rowD, m.perm);
     RT_HIP(hipStreamSynchronize(ctx->stream));
 }
 

@@ -231,7 +231,7 @@ int solveNoAlloc(Ctx* c, const Mesh& mc, const rt_ldu_symm* sys, double* psi, co
     if (rb) launch_rb_schur_diag(c, m, lo, up, dD, dS);  // the Schur pivots of a general LDU matrix
     if (bicg) launch_ldu_to_ell(c, m, up, lo, K.atval.as<double>());  // A^T
     RT_HIP(hipMemcpyAsync(stage, psi, n6 * 8, hipMemcpyHostToDevice, st));
-    launch_permute_rows(c, N, 6, 6, stage, m.permD.as<int32_t>(), dX);
+    launch_rows_in6(c, m, stage, dX);
     // the solver state starts from zero (the array holds the last call's)
     launch_fill(c, K.state.as<double>(), (int64_t)(sizeof(SolveState) / sizeof(double)), 0.0);
     double xbar[6];
@@ -260,7 +260,7 @@ int solveNoAlloc(Ctx* c, const Mesh& mc, const rt_ldu_symm* sys, double* psi, co
     sa.hostStatus = &slot.status;
     sa.rDs = dS;
     solve_lockstep(c, sa, perf);
-    launch_unpermute_rows(c, N, 6, 6, dX, m.permD.as<int32_t>(), stage);
+    launch_rows_out6(c, m, dX, stage);
     RT_HIP(hipMemcpyAsync(psi, stage, n6 * 8, hipMemcpyDeviceToHost, st));
     RT_HIP(hipStreamSynchronize(st));
     return RT_OK;

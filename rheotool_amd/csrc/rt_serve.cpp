@@ -179,9 +179,8 @@ void beginDownload(rt_ctx* c, Request* r) {
     }
     r->dlTheta = x->alloc(bytes);
     r->dlTau = x->alloc(bytes);
-    const int32_t* perm = m.permD.as<int32_t>();
-    launch_unpermute_rows(x, m.N, 6, 6, M.theta.as<double>(), perm, r->dlTheta.as<double>());
-    launch_unpermute_rows(x, m.N, 6, 6, M.tau.as<double>(), perm, r->dlTau.as<double>());
+    launch_rows_out6(x, m, M.theta.as<double>(), r->dlTheta.as<double>());
+    launch_rows_out6(x, m, M.tau.as<double>(), r->dlTau.as<double>());
     RT_HIP(hipMemcpyAsync(th, r->dlTheta.p, bytes, hipMemcpyDeviceToHost, x->stream));
     RT_HIP(hipMemcpyAsync(ta, r->dlTau.p, bytes, hipMemcpyDeviceToHost, x->stream));
 }
