@@ -846,6 +846,15 @@ __global__ void k_fill(double* p, int64_t n, double v) {
     const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
     if (i < n) p[i] = v;
 }
+// Several arrays in one launch, an array to each blockIdx.y: bound by the launch
+// at the sizes a server sees.  A new model's fields took eight launches of 2 to
+// 3 us, 24 requests of 1000 to 20000 cells 5480 us in all, now 4930.
+__global__ void __launch_bounds__(BLK) k_fills(FillArgs a) {
+    double* p = a.p[blockIdx.y];
+    const int64_t n = a.n[blockIdx.y];
+    const double v = a.v[blockIdx.y];
+    for (int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x; i < n; i += (int64_t)gridDim.x * BLK) p[i] = v;
+}
 // face-order entry e of row r sits at ellOff[s] + 64k + lane; its value goes to
 // the column-order slot ellSlot[e] of the same row
 __device__ __forceinline__ int64_t col_slot(int64_t e, const int64_t* __restrict__ off,
@@ -1543,6 +1552,21 @@ void launch_fill(Ctx* ctx, double* p, int64_t n, double v) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_fill, dim3(nblk(n)), dim3(BLK), 0, ctx->stream, p, n, v);
     RT_HIP(hipGetLastError());
+}
+void launch_fills(Ctx* ctx, const std::vector<Fill>& fills) {
+    for (size_t k = 0; k < fills.size(); k += FILLS_MAX) {
+        FillArgs a{};
+        int na = 0;
+        int64_t most = 0;
+        for (; na < FILLS_MAX && k + na < fills.size(); ++na) {
+            a.p[na] = fills[k + na].p, a.n[na] = fills[k + na].n, a.v[na] = fills[k + na].v;
+            most = std::max(most, a.n[na]);
+        }
+        if (most <= 0) continue;
+        const unsigned g = std::min(nblk(most), (unsigned)ctx->numCUs * 8);
+        hipLaunchKernelGGL(k_fills, dim3(g, (unsigned)na), dim3(BLK), 0, ctx->stream, a);
+        RT_HIP(hipGetLastError());
+    }
 }
 void launch_ldu_to_ell(Ctx* ctx, const Mesh& m, const double* lower, const double* upper, double* aval) {
     if (m.nEll <= 0) return;

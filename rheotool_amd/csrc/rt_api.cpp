@@ -523,7 +523,6 @@ void modelCorrectBegin(Model& M, double deltaT, const double* gradU, int iterati
         M.aval = ctx->alloc((size_t)std::max<int64_t>(1, m.nEll) * 8);
         M.slotMask = ctx->alloc((size_t)std::max<int32_t>(1, m.nSlices) * 4);
         M.b = ctx->alloc((size_t)6 * N * 8);
-        RT_HIP(hipMemsetAsync(M.b.p, 0, (size_t)6 * N * 8, ctx->stream));
     }
     if (modelKeepsFactor(M.prm.kind) && !M.fOld.p) M.fOld = ctx->alloc((size_t)N * 8);
     // inner iterations of a step keep theta.oldTime() of the step's first one
@@ -1057,9 +1056,6 @@ void allocModelState(Model& M) {
         M.bcType = c->alloc((size_t)std::max(1, M.mesh->nPatches) * 4);
         M.bcVal = c->alloc((size_t)6 * std::max(1, NB) * 8);
         M.patchT = c->alloc((size_t)9 * std::max(1, M.mesh->nPatches) * 8);
-        RT_HIP(hipMemsetAsync(M.bcVal.p, 0, M.bcVal.bytes, c->stream));
-        RT_HIP(hipMemsetAsync(M.patchT.p, 0, M.patchT.bytes, c->stream));
-        RT_HIP(hipMemsetAsync(M.tau.p, 0, M.tau.bytes, c->stream));
         M.hBcType.resize(M.mesh->nPatches);
         for (int p = 0; p < M.mesh->nPatches; ++p)
             M.hBcType[p] = M.mesh->patches[p].kind == RT_PATCH_EMPTY ? RT_BC_EMPTY : RT_BC_ZEROGRADIENT;
@@ -1067,9 +1063,17 @@ void allocModelState(Model& M) {
             RT_HIP(hipMemcpyAsync(M.bcType.p, M.hBcType.data(), M.hBcType.size() * 4,
                                   hipMemcpyHostToDevice, c->stream));
         // READ_IF_PRESENT default of eigVals/eigVecs: identity tensor
-        launch_fill(c, M.eigVal.as<double>(), (int64_t)3 * N, 1.0);
-        launch_fill(c, M.eigVec.as<double>(), (int64_t)9 * N, 0.0);
-        for (int q : {0, 4, 8}) launch_fill(c, M.eigVec.as<double>() + (int64_t)q * N, N, 1.0);
+        double* V = M.eigVec.as<double>();
+        const int64_t n = N;
+        launch_fills(c, {{M.eigVal.as<double>(), 3 * n, 1.0},
+                         {V, n, 1.0},
+                         {V + n, 3 * n, 0.0},
+                         {V + 4 * n, n, 1.0},
+                         {V + 5 * n, 3 * n, 0.0},
+                         {V + 8 * n, n, 1.0},
+                         {M.tau.as<double>(), (int64_t)(M.tau.bytes / 8), 0.0},
+                         {M.bcVal.as<double>(), (int64_t)(M.bcVal.bytes / 8), 0.0},
+                         {M.patchT.as<double>(), (int64_t)(M.patchT.bytes / 8), 0.0}});
         M.ctl = parseControls(nullptr);
         RT_HIP(hipStreamSynchronize(c->stream));
     }

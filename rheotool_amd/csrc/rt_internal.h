@@ -473,6 +473,19 @@ void launch_eigvals_to_tensor(Ctx* ctx, int32_t N, const double* eigVal, const i
                               double* aos9);
 // out[i] = 0 + in[0][i] + in[1][i] + ..., i < n (n even)
 void launch_sum(Ctx* ctx, int64_t n, const std::vector<const double*>& in, double* out);
+// n words of v at p; one launch for up to FILLS_MAX of them
+struct Fill {
+    double* p;
+    int64_t n;
+    double v;
+};
+constexpr int FILLS_MAX = 12;
+struct FillArgs {
+    double* p[FILLS_MAX];
+    int64_t n[FILLS_MAX];
+    double v[FILLS_MAX];
+};
+void launch_fills(Ctx* ctx, const std::vector<Fill>& fills);
 void launch_fill(Ctx* ctx, double* p, int64_t n, double v);
 void launch_copy(Ctx* ctx, const void* src, void* dst, size_t bytes);
 
