@@ -156,6 +156,9 @@ int rt_mesh_valid_components(const rt_mesh* mesh, int32_t out[6]);
  *                          right Jacobi on the device; none)
  *   tolerance 1e-10; relTol 0; maxIter 1000; minIter 0;
  *   precision double;  (or "mixed": FP32 Krylov + FP64 iterative refinement)
+ *   residentPolls 200000;  (polls after which a workgroup of a small mesh's
+ *                          one-launch solve gives its wait up and the solve
+ *                          runs by launches; 0: always by launches)
  * Unknown solver / preconditioner keywords -> RT_E_UNKNOWN_TYPE listing the
  * valid ones (sparseSolver.C:48-56 style). */
 typedef struct {
