@@ -1567,12 +1567,20 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     KryArgs<T> a = m.a, b = m.b, sw = m.s;
     a.cs = b.cs = sw.cs = cs;
     a.host = b.host = sw.host = nullptr;
-    // the x/r pass has partial sums of its own: the t pass's may still be read
-    KryArgs<T> ax = a, af = a;
-    ax.partials = af.partials = a.partials + (int64_t)24 * a.G;
+    // Each pass with a reduction writes its plan's slot of the partial sums.  No
+    // barrier stands between a workgroup's reads of a reduction and the passes
+    // after it: Jacobi's t pass follows the v pass's finalizer at once, and its v
+    // pass (no p pass in an inner solve's first round) the sweep's.
+    constexpr ResPlan plan = BICG ? RES_PLAN_BICG : RES_PLAN_STAB;
+    auto slot = [&](ResSlot s) { return m.a.partials + (int64_t)RES_SLOT_BEGIN[s] * m.a.G; };
+    KryArgs<T> av = a, at = a, ax = a;  // the v (PBiCG: w), t and x/r passes
+    av.partials = slot(plan.slot[0]);
+    at.partials = slot(plan.slot[1]);
+    ax.partials = slot(plan.slot[plan.n - 1]);
+    sw.partials = a.partials = slot(RES_SWEEP_SLOT);
     // the finalizers sum the workgroups that have a tile: the others add zeros
-    KryArgs<T> an = a;
-    an.G = af.G = m.X;
+    KryArgs<T> fv = av, ft = at, fx = ax, fs = a;
+    fv.G = ft.G = fx.G = fs.G = m.X;
     ResBar bar{m.st, P, 1, P, nullptr, m.maxPolls, 0, (uint32_t)(m.P > 0), &bad};
     auto wait = [&] { return res_barrier(bar); };
     // one pass of the row kernels: workgroups 0 .. X-1 of G, RSUB at a time
@@ -1667,7 +1675,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
             pass(a.G, [&](const Blk& k) { k_residual_body<T, 1>(RB ? sw : a, k); });
             ok = wait();
             if (!ok) break;
-            k_fin_residual_body<T, 1, RBLK>(an, lds);
+            k_fin_residual_body<T, 1, RBLK>(fs, lds);
             __syncthreads();
             continue;
         }
@@ -1714,11 +1722,11 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
 #pragma unroll
                 for (int c = 0; c < 6; ++c) q[c] = rd.on[c] && rB >= 0 ? (T)0 + w0[c] * wv[c] : (T)0;
                 if (rB >= 0) st6(at_off(a.v, oB), wv);
-                write_partials<6>(q, a.partials, kRow);
+                write_partials<6>(q, av.partials, kRow);
             }
             ok = wait();
             if (!ok) break;
-            k_fin_v_body<T, RBLK>(an, lds);
+            k_fin_v_body<T, RBLK>(fv, lds);
             __syncthreads();
             T al[6];
 #pragma unroll
@@ -1747,11 +1755,11 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
                     q[6 + c] = o ? (T)0 + wt[c] * sv[c] : (T)0;
                     q[12 + c] = o ? (T)0 + wt[c] * wt[c] : (T)0;
                 }
-                write_partials<18>(q, a.partials, kRow);
+                write_partials<18>(q, at.partials, kRow);
             }
             ok = wait();
             if (!ok) break;
-            k_fin_t_body<T, RBLK>(an, lds);
+            k_fin_t_body<T, RBLK>(ft, lds);
             __syncthreads();
             {
                 double q[12], alphas[6], omegas[6];
@@ -1789,11 +1797,11 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
                     if constexpr (MIX) st6(at_off(a.e, oB), X);
                     else st6(at_off(a.x, oB), X);
                 }
-                write_partials<12>(q, af.partials, kRow);
+                write_partials<12>(q, ax.partials, kRow);
             }
             ok = wait();
             if (!ok) break;
-            k_fin_xr_body<T, RBLK>(af, lds);
+            k_fin_xr_body<T, RBLK>(fx, lds);
             __syncthreads();
         } else if constexpr (FORM == RF_BICG_ROW) {
             const Round rd = round_of(a);
@@ -1836,11 +1844,11 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
                 double q[6];
 #pragma unroll
                 for (int c = 0; c < 6; ++c) q[c] = rd.on[c] && rB >= 0 ? (T)0 + wA[c] * wv[c] : (T)0;
-                write_partials<6>(q, a.partials, kRow);
+                write_partials<6>(q, av.partials, kRow);
             }
             ok = wait();
             if (!ok) break;
-            k_fin_bicg_w_body<T, RBLK>(an, lds);
+            k_fin_bicg_w_body<T, RBLK>(fv, lds);
             __syncthreads();
             {
                 double q[12];
@@ -1861,25 +1869,25 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
                     if constexpr (MIX) st6(at_off(a.e, oB), X);
                     else st6(at_off(a.x, oB), X);
                 }
-                write_partials<12>(q, af.partials, kRow);
+                write_partials<12>(q, ax.partials, kRow);
             }
             ok = wait();
             if (!ok) break;
-            k_fin_bicg_xr_body<T, RBLK>(af, lds);
+            k_fin_bicg_xr_body<T, RBLK>(fx, lds);
             __syncthreads();
         } else if constexpr (BICG) {
             passAll(m.pg, [&](const Blk& k) { k_bicg_p_body<T>(a, k); });
             ok = wait();
             if (!ok) break;
-            pass(a.G, [&](const Blk& k) { k_bicg_w_body<T>(a, k); });
+            pass(a.G, [&](const Blk& k) { k_bicg_w_body<T>(av, k); });
             ok = wait();
             if (!ok) break;
-            k_fin_bicg_w_body<T, RBLK>(an, lds);
+            k_fin_bicg_w_body<T, RBLK>(fv, lds);
             __syncthreads();
             pass(a.G, [&](const Blk& k) { k_bicg_xr_body<T>(ax, k); });
             ok = wait();
             if (!ok) break;
-            k_fin_bicg_xr_body<T, RBLK>(af, lds);
+            k_fin_bicg_xr_body<T, RBLK>(fx, lds);
             __syncthreads();
         } else {
             if (round_of(a).inner > 0) {
@@ -1891,30 +1899,30 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
                 pass(m.Gw, [&](const Blk& k) { k_rb_w_body<T, 0>(a, k); });
                 ok = wait();
                 if (!ok) break;
-                pass(a.G, [&](const Blk& k) { k_rb_v_body<T>(a, k); });
+                pass(a.G, [&](const Blk& k) { k_rb_v_body<T>(av, k); });
             } else {
-                pass(a.G, [&](const Blk& k) { k_kry_v_body<T>(a, k); });
+                pass(a.G, [&](const Blk& k) { k_kry_v_body<T>(av, k); });
             }
             ok = wait();
             if (!ok) break;
-            k_fin_v_body<T, RBLK>(an, lds);
+            k_fin_v_body<T, RBLK>(fv, lds);
             __syncthreads();
             if constexpr (RB) {
                 pass(m.Gw, [&](const Blk& k) { k_rb_w_body<T, 1>(a, k); });
                 ok = wait();
                 if (!ok) break;
-                pass(a.G, [&](const Blk& k) { k_rb_t_body<T>(a, k); });
+                pass(a.G, [&](const Blk& k) { k_rb_t_body<T>(at, k); });
             } else {
-                pass(a.G, [&](const Blk& k) { k_kry_t_body<T>(a, k); });
+                pass(a.G, [&](const Blk& k) { k_kry_t_body<T>(at, k); });
             }
             ok = wait();
             if (!ok) break;
-            k_fin_t_body<T, RBLK>(an, lds);
+            k_fin_t_body<T, RBLK>(ft, lds);
             __syncthreads();
             pass(a.G, [&](const Blk& k) { k_kry_xr_body<T>(ax, k); });
             ok = wait();
             if (!ok) break;
-            k_fin_xr_body<T, RBLK>(af, lds);
+            k_fin_xr_body<T, RBLK>(fx, lds);
             __syncthreads();
         }
     }
@@ -2005,8 +2013,8 @@ void Krylov::ensure(Ctx* run, Mesh& m, bool mixed, bool bicg) {
         r = DBuf(); r0 = DBuf(); p = DBuf(); v = DBuf(); t = DBuf();
         rs = DBuf(); r0s = DBuf(); ps = DBuf(); vs = DBuf(); ts = DBuf(); es = DBuf();
         ahat32 = DBuf(); ahat64 = DBuf();
-        // the x/r pass of a resident solve has 12 more partial sums per workgroup
-        partials = ctx->alloc((size_t)grid * (N <= RES_MAX_ROWS ? 36 : 24) * sizeof(double));
+        // a resident solve's reductions have slots of their own
+        partials = ctx->alloc((size_t)grid * (N <= RES_MAX_ROWS ? RES_SUMS : 24) * sizeof(double));
         xSave = DBuf();
         if (N <= RES_MAX_ROWS && grid > RSUB) xSave = ctx->alloc(3 * vec * 8);
         state = ctx->alloc(sizeof(SolveState));
@@ -2486,7 +2494,7 @@ void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     Krylov& K = *sa.kry;
     R.resident = R.resLaunched = false;
     if (sa.ctl->residentPolls == 0 || ctx->profiling || K.N > RES_MAX_ROWS) return;
-    if (R.G % 8 == 0 || K.partials.bytes < (size_t)36 * K.grid * sizeof(double)) return;
+    if (R.G % 8 == 0 || K.partials.bytes < (size_t)RES_SUMS * K.grid * sizeof(double)) return;
     const Mesh& m = *sa.mesh;
     // row-kernel workgroups with a tile (their tiles in order: G is no multiple of 8)
     const int32_t row0 = R.rb ? m.nRed & ~(SLICE - 1) : 0;

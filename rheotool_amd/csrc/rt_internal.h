@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "rheo_gpu.h"
+#include "rt_resident.h"
 
 namespace rt {
 
@@ -272,7 +273,7 @@ struct Krylov {
     DBuf rD;               // double [N]    1/diag
     DBuf rDs;              // double [N]    red-black: 1/diag of the Schur complement
                            // (the ILU0 diagonal) where it differs from 1/diag
-    DBuf partials;         // double [grid][24] (36 on a mesh of at most RES_MAX_ROWS rows)
+    DBuf partials;         // double [grid][24] (RES_SUMS on a mesh of at most RES_MAX_ROWS rows)
     DBuf xSave;            // FP64 [3][N][6] the start of a resident solve of several workgroups
     DBuf state;            // SolveState
     std::unique_ptr<SolveRun, SolveRunDeleter> run;

@@ -28,7 +28,7 @@ namespace {
 
 constexpr size_t kScratchBytes = RT_NOALLOC_SCRATCH_BYTES;
 // behind the scratch bytes the meshes share: the reduction partials (at most
-// 2048 workgroups of 36 sums) and the solver state
+// 2048 workgroups of RES_SUMS sums) and the solver state
 constexpr size_t kTailBytes = size_t(1) << 20;
 constexpr int kMaxDevices = 64;
 
@@ -188,7 +188,7 @@ int solveNoAlloc(Ctx* c, const Mesh& mc, const rt_ldu_symm* sys, double* psi, co
     cv.take(1280);
     Carve tail{static_cast<char*>(slot.ptr) + kScratchBytes};
     const bool small = N <= RES_MAX_ROWS;
-    const size_t partBytes = (size_t)grid * (small ? 36 : 24) * sizeof(double);
+    const size_t partBytes = (size_t)grid * (small ? RES_SUMS : 24) * sizeof(double);
     K.partials = DBuf::viewOf(tail.take(partBytes), partBytes);
     K.state = DBuf::viewOf(tail.take(sizeof(SolveState)), sizeof(SolveState));
     K.xSave = DBuf();

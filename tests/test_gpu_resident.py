@@ -31,11 +31,14 @@ def step(ctx, dm, m, f, controls, steps=2):
     return rcs, perf, eq.theta(), eq.tau()
 
 
-# one row; one workgroup, full and not; the first sizes with two and three
-# workgroups of 512 rows' work, odd rows; the largest resident mesh and the first
-# that is not (65536 rows)
+# a workgroup takes 256 rows (red-black: 256 of each colour).  One row; one, two and
+# more workgroups, full and not; just more than one XCD's 32 CUs hold in FP64 (8192
+# rows; red-black 16384); the largest mesh the forms other than red-black take
+# resident (32768 rows) and one row less than a workgroup below; red-black's (65536)
+# and the first that is not
 @pytest.mark.parametrize("shape", [(1, 1, 1), (16, 16, 1), (32, 16, 1), (27, 19, 1), (33, 32, 1), (13, 11, 9),
-                                   (256, 256, 1), (257, 255, 1), (257, 256, 1)])
+                                   (91, 91, 1), (129, 128, 1), (181, 181, 1), (256, 128, 1), (256, 256, 1),
+                                   (257, 255, 1), (257, 256, 1)])
 @pytest.mark.parametrize("precision", ["double", "mixed"])
 def test_resident_solve_equals_launches(ctx, shape, precision):
     nx, ny, nz = shape
@@ -52,7 +55,7 @@ def test_resident_solve_equals_launches(ctx, shape, precision):
             assert np.array_equal(got[2], want[2]) and np.array_equal(got[3], want[3])
 
 
-@pytest.mark.parametrize("n", [500, 5000])
+@pytest.mark.parametrize("n", [500, 5000, 20000])
 @pytest.mark.parametrize("noalloc", [False, True])
 def test_resident_symm_solve_equals_launches(ctx, n, noalloc):
     """A general LDU system on a random face graph (rows wider than the staged
