@@ -1334,13 +1334,12 @@ __global__ void __launch_bounds__(FBLK) k_fin_mean6(int32_t N, int G, const doub
 // and the saved vectors then still hold the solve's start, and the host runs it
 // by launches.
 constexpr int RBLK = 256, RSUB = RBLK / BLK;
-constexpr int XCDS = 8;
+constexpr int XCDS = RES_XCDS;
 // workgroups a CU holds: FP32 solves are held to 256 registers a lane for two,
 // FP64 ones take up to 350 (held to 256 they spill, and a 128 x 128 channel's
 // step took 200 us instead of 179)
 template <class T>
 constexpr int RES_PER_CU = sizeof(T) == 4 ? 2 : 1;
-constexpr uint32_t RES_FAIL = 0x80000000u;
 
 template <class T>
 struct ResArgs {
@@ -1356,100 +1355,65 @@ struct ResArgs {
     double* xSave;
 };
 
-struct ResBar {
-    SolveState* st;
-    int P, nXcd, nHere;    // workgroups; XCDs they are on; workgroups on this one
-    uint32_t* here;        // this XCD's counters: arrivals, barriers passed, departures
-    uint32_t maxPolls, ph, one;  // ph: barriers so far; one: 1, unknown to the compiler
-    int* bad;
-};
-template <int SCOPE>
-__device__ __forceinline__ uint32_t at_add(uint32_t* p, uint32_t v) {
-    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, SCOPE);
-}
-// Polls *p (an atomic add of 0: L2 executes it, no L1 copy is read) until its low
-// bits reach target; returns with RES_FAIL set if a wait gave up, this or another
-template <int SCOPE>
-__device__ __forceinline__ uint32_t res_poll(uint32_t* p, uint32_t v, uint32_t target, const ResBar& B) {
-    for (uint32_t n = 0; v < target;) {
-        if (++n > B.maxPolls) return __hip_atomic_fetch_or(p, RES_FAIL, __ATOMIC_RELAXED, SCOPE) | RES_FAIL;
-        __builtin_amdgcn_s_sleep(1);
-        v = at_add<SCOPE>(p, B.one - 1u);
+// the operations of the barrier's words (rt_resident.h)
+struct ResAt {
+    template <ResScope S>
+    static constexpr int scope = S == RES_XCD ? __HIP_MEMORY_SCOPE_WORKGROUP : __HIP_MEMORY_SCOPE_AGENT;
+    template <ResScope S>
+    static __device__ __forceinline__ uint32_t add(uint32_t* p, uint32_t v) {
+        return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, scope<S>);
     }
-    return v;
-}
-// Before the first pass: counts the workgroups on each XCD and waits for all of
-// them, with a counter of its own and every workgroup fencing.
-__device__ __forceinline__ bool res_enter(ResBar& B) {
+    template <ResScope S>
+    static __device__ __forceinline__ uint32_t or_(uint32_t* p, uint32_t v) {
+        return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, scope<S>);
+    }
+    template <ResScope S>
+    static __device__ __forceinline__ uint32_t swap(uint32_t* p, uint32_t v) {
+        return __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, scope<S>);
+    }
+    static __device__ __forceinline__ uint32_t get(const uint32_t* p) {
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static __device__ __forceinline__ void set(uint32_t* p, uint32_t v) {
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static __device__ __forceinline__ void sleep() { __builtin_amdgcn_s_sleep(1); }
+    static __device__ __forceinline__ void release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
+    static __device__ __forceinline__ void acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
+};
+__device__ __forceinline__ bool res_enter(ResBar& B, int* bad) {
     if (B.P == 1) {
         __syncthreads();
         return true;
     }
-    constexpr int AG = __HIP_MEMORY_SCOPE_AGENT;
     const uint32_t x = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7u;  // hwreg XCC_ID, bits 0..3
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
-        at_add<AG>(&B.st->bar[8 + x], 1u);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const uint32_t v = res_poll<AG>(B.st->bar, at_add<AG>(B.st->bar, 1u) + 1u, (uint32_t)B.P, B);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        *B.bad = ((v | at_add<AG>(B.st->bar, B.one - 1u)) & RES_FAIL) != 0;
+        *bad = res_enter_wait<ResAt>(B, x);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();
-    B.nXcd = 0;
-    for (int i = 0; i < XCDS; ++i)
-        B.nXcd += __hip_atomic_load(&B.st->bar[8 + i], __ATOMIC_RELAXED, AG) != 0;
-    B.nHere = (int)__hip_atomic_load(&B.st->bar[8 + x], __ATOMIC_RELAXED, AG);
-    B.here = B.st->barL2[x];
-    return *B.bad == 0;
+    res_enter_place<ResAt>(B, x);
+    return *bad == 0;
 }
 // Every wave's stores have reached its L2 before the first wave arrives; no wave
 // goes on before that one has dropped the CU's L1 (the load after the fence
 // returns behind it).
-__device__ __forceinline__ bool res_barrier(ResBar& B) {
+__device__ __forceinline__ bool res_barrier(ResBar& B, int* bad) {
     if (B.P == 1) {
         __syncthreads();
         return true;
     }
-    constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP, AG = __HIP_MEMORY_SCOPE_AGENT;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     ++B.ph;
     if (threadIdx.x == 0) {
-        uint32_t v = at_add<WG>(&B.here[0], B.one) + 1u;
-        const uint32_t full = B.ph * (uint32_t)B.nHere;
-        if (B.nXcd == 1) {
-            v = res_poll<WG>(&B.here[0], v, full, B);
-        } else if (v == full) {
-            v = 0;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            uint32_t* g = &B.st->bar[2];
-            v = res_poll<AG>(g, at_add<AG>(g, 1u) + 1u, B.ph * (uint32_t)B.nXcd, B);
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            v |= at_add<AG>(g, B.one - 1u);
-            v = at_add<WG>(&B.here[1], (v & RES_FAIL) + B.one) | (v & RES_FAIL);
-        } else {
-            v = res_poll<WG>(&B.here[1], at_add<WG>(&B.here[1], B.one - 1u), B.ph, B);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        v |= at_add<WG>(&B.here[B.nXcd == 1 ? 0 : 1], B.one - 1u);
-        *B.bad = (v & RES_FAIL) != 0;
+        *bad = res_wait<ResAt>(B);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();
-    return *B.bad == 0;
-}
-// Past the last barrier: the last workgroup of an XCD, and the last of all, leave
-// their counters at zero for the next launch.
-__device__ __forceinline__ void res_leave(ResBar& B) {
-    if (B.P == 1 || threadIdx.x != 0) return;
-    constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP, AG = __HIP_MEMORY_SCOPE_AGENT;
-    if (at_add<WG>(&B.here[2], B.one) + 1u == (uint32_t)B.nHere)
-        for (int i = 0; i < 3; ++i) (void)__hip_atomic_exchange(&B.here[i], 0u, __ATOMIC_RELAXED, WG);
-    if (at_add<AG>(&B.st->bar[1], 1u) + 1u == (uint32_t)B.P)
-        for (int i = 0; i < 8 + XCDS; ++i) __hip_atomic_store(&B.st->bar[i], 0u, __ATOMIC_RELAXED, AG);
+    return *bad == 0;
 }
 
 // RF_RB_ROW, RF_BICG_ROW: every thread keeps one row (red-black: one of each
@@ -1581,8 +1545,8 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     // the finalizers sum the workgroups that have a tile: the others add zeros
     KryArgs<T> fv = av, ft = at, fx = ax, fs = a;
     fv.G = ft.G = fx.G = fs.G = m.X;
-    ResBar bar{m.st, P, 1, P, nullptr, m.maxPolls, 0, (uint32_t)(m.P > 0), &bad};
-    auto wait = [&] { return res_barrier(bar); };
+    ResBar bar{m.st->bar, m.st->barL2, P, 1, P, nullptr, m.maxPolls, 0, (uint32_t)(m.P > 0)};
+    auto wait = [&] { return res_barrier(bar, &bad); };
     // one pass of the row kernels: workgroups 0 .. X-1 of G, RSUB at a time
     auto passOf = [&](int X, int G, auto&& body) {
         for (int v0 = p * RSUB; v0 < X; v0 += P * RSUB) {
@@ -1617,7 +1581,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
             passAll(X0, [&](const Blk& k) { k_scale_body<T>(a, k); });
         }
     }
-    bool ok = res_enter(bar);
+    bool ok = res_enter(bar, &bad);
     // the kept rows: tile p RSUB + sub of the rows (red-black: of each colour)
     constexpr bool ROW = FORM == RF_RB_ROW || FORM == RF_BICG_ROW;
     const Blk kRow{p * RSUB + sub < m.X ? a.G : 0, p * RSUB + sub, tid, red[sub]};
@@ -1936,7 +1900,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
         (ok ? m.st->resDone : m.st->resFail) = m.epoch;
         if (m.host) (ok ? m.host->resDone : m.host->resFail) = m.epoch;
     }
-    if (ok) res_leave(bar);
+    if (ok && P > 1 && threadIdx.x == 0) res_depart<ResAt>(bar);
 }
 
 // workgroup b of the grid: b % XCDS is the XCD it is dealt to; xcd < 0: on all

@@ -241,11 +241,10 @@ struct SolveState {
     int32_t anyActive;
     double misc[8];  // misc[0]: ELL entries in live slots of the solve's matrix (set by the assembly)
     uint32_t resDone, resFail;  // the resident launch (its epoch) that finished, whose wait gave up
-    // barriers of a resident solve, zero between launches (top bit: a wait gave
-    // up).  bar: [0] entered, [1] left, [2] the XCDs' barrier, [8 + x] workgroups on
-    // XCD x; barL2[x]: XCD x's own, a cache line each (arrivals, barriers, departures)
+    // barriers of a resident solve (ResBar), zero between launches; barL2: a cache
+    // line for each XCD
     alignas(128) uint32_t bar[32];
-    alignas(128) uint32_t barL2[8][32];
+    alignas(128) uint32_t barL2[RES_XCDS][32];
 };
 
 struct SolveRun;  // host side of a resumable solve (kernels_krylov.hip)

@@ -109,7 +109,100 @@ static void partial_sums(uint64_t seed) {
     s.run(seed, rng() % 2 ? (int)(rng() % P) : -1);
 }
 
+// The barrier: workgroups on one to three XCDs meet a few times, over the same
+// words launch after launch, some with so few polls that waits give up.
+struct At {
+    static Sched* s;
+    template <ResScope>
+    static uint32_t add(uint32_t* p, uint32_t v) {
+        s->yield();
+        const uint32_t o = *p;
+        *p += v;
+        return o;
+    }
+    template <ResScope>
+    static uint32_t or_(uint32_t* p, uint32_t v) {
+        s->yield();
+        const uint32_t o = *p;
+        *p |= v;
+        return o;
+    }
+    template <ResScope>
+    static uint32_t swap(uint32_t* p, uint32_t v) {
+        s->yield();
+        const uint32_t o = *p;
+        *p = v;
+        return o;
+    }
+    static uint32_t get(const uint32_t* p) {
+        s->yield();
+        return *p;
+    }
+    static void set(uint32_t* p, uint32_t v) {
+        s->yield();
+        *p = v;
+    }
+    static void sleep() { s->yield(); }
+    static void release() {}
+    static void acquire() {}
+};
+Sched* At::s = nullptr;
+
+static int gaveUp = 0, finished = 0, finalAll = 0;
+static void barrier(uint64_t seed) {
+    std::mt19937_64 rng(seed);
+    uint32_t bar[32] = {0}, barL2[RES_XCDS][32] = {{0}};
+    for (int launch = 0; launch < 3; ++launch) {
+        const int P = 2 + (int)(rng() % 6), nx = 1 + (int)(rng() % 3), K = 1 + (int)(rng() % 4);
+        const uint32_t polls = rng() % 2 ? 1000000u : 1u + (uint32_t)(rng() % 60);
+        std::vector<int> arrived(K + 1, 0);
+        int failed = 0, passed = 0;
+        Sched s;
+        At::s = &s;
+        for (int p = 0; p < P; ++p)
+            s.spawn([&, p] {
+                const uint32_t x = (uint32_t)(p % nx);
+                ResBar B{bar, barL2, P, 1, P, nullptr, polls, 0, 1};
+                ++arrived[0];
+                if (res_enter_wait<At>(B, x)) {
+                    ++failed;
+                    return;
+                }
+                res_enter_place<At>(B, x);
+                for (int k = 0;; ++k) {
+                    CHECK(arrived[k] == P, "workgroup %d passed barrier %d with %d of %d there", p, k, arrived[k], P);
+                    if (k == K) break;
+                    s.yield();
+                    ++arrived[k + 1];
+                    ++B.ph;
+                    if (res_wait<At>(B)) {
+                        ++failed;
+                        return;
+                    }
+                }
+                ++passed;
+                res_depart<At>(B);
+            });
+        s.run(seed * 7 + launch, rng() % 2 ? (int)(rng() % P) : -1);
+        bool clean = true;
+        for (uint32_t w : bar) clean = clean && w == 0;
+        for (auto& l : barL2)
+            for (uint32_t w : l) clean = clean && w == 0;
+        CHECK(clean || failed, "counters left set with no workgroup to say so");
+        if (failed) {  // as the host does
+            for (uint32_t& w : bar) w = 0;
+            for (auto& l : barL2)
+                for (uint32_t& w : l) w = 0;
+        }
+        CHECK(polls < 1000000u || !failed, "a wait gave up on workgroups that all run");
+        (failed == 0 ? finished : passed ? finalAll : gaveUp)++;
+    }
+}
+
 int main() {
     for (uint64_t seed = 1; seed <= 500; ++seed) partial_sums(seed);
+    for (uint64_t seed = 1; seed <= 5000; ++seed) barrier(seed);
+    std::printf("launches finished %d, gave up %d, gave up behind the last barrier %d\n", finished, gaveUp, finalAll);
+    CHECK(finished > 1000 && gaveUp > 1000 && finalAll > 10, "the schedules miss an outcome");
     std::printf("OK\n");
 }
