@@ -68,6 +68,11 @@ const char* rt_last_error(const rt_ctx* ctx);
 /* Device bytes currently allocated by the context. */
 size_t rt_ctx_bytes_in_use(const rt_ctx* ctx);
 
+/* How the context's linear solves ran: counts[0] finished in one resident
+ * launch (small meshes), counts[1] resident launches that gave their wait up
+ * (each then ran by launches), counts[2] finished by launches. */
+int rt_ctx_solve_counts(const rt_ctx* ctx, int64_t counts[3]);
+
 /* Kernel timing: when enabled, every launch is bracketed by HIP events on the
  * context's stream.  rt_ctx_kernel_stats fills up to `cap` records (name,
  * launches, total ms) and returns the number of distinct kernels. */
@@ -426,6 +431,8 @@ int rt_server_finished(rt_server* server, int64_t* tickets, int max);
 int rt_server_set_batching(rt_server* server, int enable);
 /* Batched Krylov rounds launched so far (each covers every request then in its batch). */
 int64_t rt_server_batched_rounds(const rt_server* server);
+/* rt_ctx_solve_counts over the requests' solves. */
+int rt_server_solve_counts(const rt_server* server, int64_t counts[3]);
 
 /* Page-locked host memory (hipHostMalloc on the context's device) for a
  * serving caller's request and result arrays.  Transfers from and to it run

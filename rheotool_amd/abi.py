@@ -95,6 +95,7 @@ def lib():
             "rt_ctx_destroy": (None, [vp]),
             "rt_last_error": (C.c_char_p, [vp]),
             "rt_ctx_bytes_in_use": (C.c_size_t, [vp]),
+            "rt_ctx_solve_counts": (i32, [vp, vp]),
             "rt_ctx_set_profiling": (i32, [vp, i32]),
             "rt_ctx_kernel_stats": (i32, [vp, vp, i32]),
             "rt_ctx_reset_stats": (None, [vp]),
@@ -133,6 +134,7 @@ def lib():
             "rt_server_set_batching": (i32, [vp, i32]),
             "rt_request_bytes_estimate": (C.c_size_t, [vp, i32, i32]),
             "rt_server_batched_rounds": (C.c_int64, [vp]),
+            "rt_server_solve_counts": (i32, [vp, vp]),
             "rt_host_alloc": (i32, [vp, C.c_size_t, vp]),
             "rt_host_free": (None, [vp]),
         }
@@ -196,6 +198,13 @@ class Context:
     @property
     def bytes_in_use(self):
         return lib().rt_ctx_bytes_in_use(self.h)
+
+    @property
+    def solve_counts(self):
+        """(resident, gave up, by launches): how the linear solves ran (rt_ctx_solve_counts)."""
+        n = (C.c_int64 * 3)()
+        self.check(lib().rt_ctx_solve_counts(self.h, n), "solve_counts")
+        return tuple(n)
 
     def set_profiling(self, on=True):
         self.check(lib().rt_ctx_set_profiling(self.h, int(on)), "set_profiling")
@@ -521,6 +530,13 @@ class Server:
     def batched_rounds(self) -> int:
         """Batched Krylov rounds launched so far (rt_server_batched_rounds)."""
         return int(lib().rt_server_batched_rounds(self.h))
+
+    @property
+    def solve_counts(self):
+        """Context.solve_counts over the requests' solves (rt_server_solve_counts)."""
+        n = (C.c_int64 * 3)()
+        self.ctx.check(lib().rt_server_solve_counts(self.h, n), "solve_counts")
+        return tuple(n)
 
     def submit(self, mesh: "Mesh", fields, dict_text, deltaT, controls=None, gradU=None, out=None,
                eigen=True) -> int:

@@ -2619,6 +2619,7 @@ bool resident_done(Ctx* ctx, SolveRun& R) {
         launch_fill(ctx, reinterpret_cast<double*>(R.st->barL2), sizeof(R.st->barL2) / 8, 0.0);
     }
     if (R.hostState->resDone == R.epoch) return true;
+    ++R.ctx->solveCounts[1];
     const size_t n6 = (size_t)6 * (size_t)R.N;
     const size_t w = R.mixed ? sizeof(float) : sizeof(double);
     const size_t nv = (n6 * w + 15) / 16 * 16;  // whole 16-byte words; the buffers are padded to 256
@@ -3059,6 +3060,7 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
 
 void solve_finish(Krylov& K, rt_solver_perf perf[6]) {
     SolveRun& R = *K.run;
+    ++R.ctx->solveCounts[R.resident ? 0 : 2];
     for (int c = 0; c < 6; ++c) {
         rt_solver_perf& pf = perf[c];
         pf = rt_solver_perf{0, 0, 0, 0, 0, 0};

@@ -811,6 +811,12 @@ const char* rt_last_error(const rt_ctx* ctx) { return ctx ? ctx->impl.lastError.
 
 size_t rt_ctx_bytes_in_use(const rt_ctx* ctx) { return ctx ? ctx->impl.inUse : 0; }
 
+int rt_ctx_solve_counts(const rt_ctx* ctx, int64_t counts[3]) {
+    if (!ctx || !counts) return RT_E_BAD_ARG;
+    for (int i = 0; i < 3; ++i) counts[i] = ctx->impl.solveCounts[i];
+    return RT_OK;
+}
+
 int rt_ctx_set_profiling(rt_ctx* ctx, int enable) {
     if (!ctx) return RT_E_BAD_ARG;
     return guarded(&ctx->impl, [&] {

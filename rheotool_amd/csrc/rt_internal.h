@@ -70,6 +70,7 @@ struct Ctx {
     int device = 0;
     int numCUs = 256;
     uint32_t resEpoch = 0;  // resident launches so far
+    int64_t solveCounts[3] = {0, 0, 0};  // finished resident, gave up, finished by launches
     int xcd = 0;  // where its resident solves run: contexts take turns
     hipStream_t stream = nullptr;
     size_t budget = 0, inUse = 0;

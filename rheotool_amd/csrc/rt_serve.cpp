@@ -299,6 +299,15 @@ int64_t rt_server_batched_rounds(const rt_server* S) {
     return n;
 }
 
+int rt_server_solve_counts(const rt_server* S, int64_t counts[3]) {
+    if (!S || !counts) return RT_E_BAD_ARG;
+    for (int i = 0; i < 3; ++i) {
+        counts[i] = 0;
+        for (const rt_ctx* c : S->slots) counts[i] += c->impl.solveCounts[i];
+    }
+    return RT_OK;
+}
+
 int rt_server_submit(rt_server* S, const rt_request* q, int64_t* ticket) {
     if (!S || !q || !ticket) return RT_E_BAD_ARG;
     rt_ctx* P = S->parent;

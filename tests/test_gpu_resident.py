@@ -13,22 +13,26 @@ pytestmark = pytest.mark.gpu
 FORMS = [("PBiCGStab", "DILU"), ("PBiCGStab", "diagonal"), ("PBiCGStab", "none"), ("PBiCG", "DILU")]
 
 
-@pytest.fixture(scope="module")
-def ctx():
-    c = abi.Context(0)
-    yield c
-    c.close()
+def step(m, f, controls, steps=2):
+    """The steps in a context of their own: results, records, fields, solve counts."""
+    with abi.Context(0) as ctx:
+        eq = ctx.constitutiveEq("", ctx.mesh(m), abi.model_dict("GiesekusLog", lam=2.0, alpha=0.2))
+        eq.set_solver(controls)
+        eq.set_state(f.theta, f.eigVals, f.eigVecs)
+        eq.set_flow(f.U, f.Ub, f.phi)
+        rcs = [eq.correct(0.2 / max(m.nCells ** 0.5, 1.0)) for _ in range(steps)]
+        perf = [(q.initialResidual, q.finalResidual, q.nIterations, q.nRefinements, q.converged, q.solved)
+                for q in eq.solver_perf()]
+        return rcs, perf, eq.theta(), eq.tau(), ctx.solve_counts
 
 
-def step(ctx, dm, m, f, controls, steps=2):
-    eq = ctx.constitutiveEq("", dm, abi.model_dict("GiesekusLog", lam=2.0, alpha=0.2))
-    eq.set_solver(controls)
-    eq.set_state(f.theta, f.eigVals, f.eigVecs)
-    eq.set_flow(f.U, f.Ub, f.phi)
-    rcs = [eq.correct(0.2 / max(m.nCells ** 0.5, 1.0)) for _ in range(steps)]
-    perf = [(q.initialResidual, q.finalResidual, q.nIterations, q.nRefinements, q.converged, q.solved)
-            for q in eq.solver_perf()]
-    return rcs, perf, eq.theta(), eq.tau()
+def workgroups(n, solver, precond):
+    """Workgroups of the solve of an n-cell two-colourable mesh whose rows have at
+    most six entries; 0: by launches."""
+    rb = solver == "PBiCGStab" and precond == "DILU"
+    P = -(-(n - n // 2 if rb else n) // 256)
+    kept = rb or solver == "PBiCG"
+    return P if P <= 128 and n <= (65536 if kept else 32768) else 0
 
 
 # a workgroup takes 256 rows (red-black: 256 of each colour).  One row; one, two and
@@ -40,29 +44,36 @@ def step(ctx, dm, m, f, controls, steps=2):
                                    (91, 91, 1), (129, 128, 1), (181, 181, 1), (256, 128, 1), (256, 256, 1),
                                    (257, 255, 1), (257, 256, 1)])
 @pytest.mark.parametrize("precision", ["double", "mixed"])
-def test_resident_solve_equals_launches(ctx, shape, precision):
+def test_resident_solve_equals_launches(shape, precision):
     nx, ny, nz = shape
     m = cases.cartesian(nx, ny, nz, twoD=nz == 1 and nx > 1, channel=True)
     f = cases.make_fields(m, cases.FIELDS_CHANNEL, seed=nx + ny)
-    dm = ctx.mesh(m)
     for solver, precond in FORMS:
         base = abi.solver_dict(1e-10, solver=solver, precond=precond, precision=precision)
         print(f"[case] resident {shape} {solver} {precond} {precision}", flush=True)
-        want = step(ctx, dm, m, f, base + " residentPolls 0;")
-        for controls in (base, base + " residentPolls 1;", base):
-            got = step(ctx, dm, m, f, controls)
+        want = step(m, f, base + " residentPolls 0;")
+        assert want[4] == (0, 0, 2)
+        P = workgroups(m.nCells, solver, precond)
+        for controls, gives_up in ((base, False), (base + " residentPolls 1;", True)):
+            got = step(m, f, controls)
             assert got[0] == want[0] and got[1] == want[1]
             assert np.array_equal(got[2], want[2]) and np.array_equal(got[3], want[3])
+            if P == 0:
+                assert got[4] == (0, 0, 2)
+            elif not gives_up or P == 1:
+                assert got[4] == (2, 0, 0)
+            else:
+                assert got[4][0] + got[4][2] == 2
+                assert got[4][1] >= 1 or P < 8  # a few workgroups may all arrive within a poll
 
 
 @pytest.mark.parametrize("n", [500, 5000, 20000])
 @pytest.mark.parametrize("noalloc", [False, True])
-def test_resident_symm_solve_equals_launches(ctx, n, noalloc):
-    """A general LDU system on a random face graph (rows wider than the staged
+def test_resident_symm_solve_equals_launches(n, noalloc):
+    """A general LDU system on a random face graph (rows wider than the kept
     width, no two-colouring) and on a box (Schur pivots)."""
     rng = np.random.default_rng(n)
     for m in (cases.random_graph(n, kNear=5, sigma=0.5, seed=3), cases.cartesian(n // 100, 10, 10)):
-        dm = ctx.mesh(m)
         lo, up = -rng.uniform(0.1, 1.0, m.nInternal), -rng.uniform(0.1, 1.0, m.nInternal)
         d = np.full(m.nCells, 0.5)
         np.add.at(d, m.owner[:m.nInternal], -lo)
@@ -70,29 +81,70 @@ def test_resident_symm_solve_equals_launches(ctx, n, noalloc):
         src, psi = rng.normal(size=(m.nCells, 6)), rng.normal(size=(m.nCells, 6))
         for solver, precond in FORMS:
             base = abi.solver_dict(1e-10, solver=solver, precond=precond)
-            want = ctx.symm_solve(dm, d, lo, up, src, psi, base + " residentPolls 0;", noalloc=noalloc)
-            for controls in (base, base + " residentPolls 1;"):
-                got = ctx.symm_solve(dm, d, lo, up, src, psi, controls, noalloc=noalloc)
-                assert np.array_equal(got[0], want[0])
-                assert [q.nIterations for q in got[1]] == [q.nIterations for q in want[1]]
+            print(f"[case] resident system {m.nCells} {solver} {precond} noalloc={noalloc}", flush=True)
+            out = []
+            for controls in (base + " residentPolls 0;", base, base + " residentPolls 1;"):
+                with abi.Context(0) as ctx:
+                    got = ctx.symm_solve(ctx.mesh(m), d, lo, up, src, psi, controls, noalloc=noalloc)
+                    out.append((got[0], [q.nIterations for q in got[1]], ctx.solve_counts))
+            assert [o[2][:2] for o in out[:2]] == [(0, 0), (1, 0)]
+            assert out[2][2][1] == 1 or n < 2048
+            for o in out[1:]:
+                assert np.array_equal(o[0], out[0][0]) and o[1] == out[0][1]
 
 
-def test_resident_server_batch_gives_up_and_finishes(ctx):
+# members on one XCD; on more than one (above 64 workgroups in FP32, 32 in FP64), beside small ones
+@pytest.mark.parametrize("precision,sides", [("mixed", (40, 60, 80)), ("mixed", (220, 30, 190, 16)),
+                                             ("double", (150, 30, 180, 140, 16))])
+def test_resident_server_batch_gives_up_and_finishes(precision, sides):
     """A batch of resident solves whose waits give up finishes by launches,
     with the same bits."""
-    reqs = []
-    for i, n in enumerate((40, 60, 80)):
-        m = cases.cartesian(n, n, 1, twoD=True, channel=True)
-        reqs.append((ctx.mesh(m), cases.make_fields(m, cases.FIELDS_CHANNEL, seed=i), 0.1 / n))
-    out = {}
-    for polls in ("0", "1", "200000"):
-        srv = abi.Server(ctx, max_inflight=4)
-        base = abi.solver_dict(1e-10, precision="mixed") + f" residentPolls {polls};"
-        ts = [srv.submit(dm, f, abi.model_dict("Oldroyd-BLog"), dt, base) for dm, f, dt in reqs]
-        while srv.progress():
-            pass
-        out[polls] = [srv.poll(t) for t in ts]
-        srv.close()
-    for polls in ("1", "200000"):
-        for a, b in zip(out[polls], out["0"]):
-            assert np.array_equal(a["theta"], b["theta"]) and np.array_equal(a["tau"], b["tau"])
+    with abi.Context(0) as ctx:
+        reqs = []
+        for i, n in enumerate(sides):
+            m = cases.cartesian(n, n, 1, twoD=True, channel=True)
+            reqs.append((ctx.mesh(m), cases.make_fields(m, cases.FIELDS_CHANNEL, seed=i), 0.1 / n))
+        out, counts = {}, {}
+        for polls in ("0", "1", "200000"):
+            print(f"[case] server {sides} {precision} residentPolls {polls}", flush=True)
+            srv = abi.Server(ctx, max_inflight=8)
+            base = abi.solver_dict(1e-10, precision=precision) + f" residentPolls {polls};"
+            ts = [srv.submit(dm, f, abi.model_dict("Oldroyd-BLog"), dt, base) for dm, f, dt in reqs]
+            while srv.progress():
+                pass
+            out[polls] = [srv.poll(t) for t in ts]
+            counts[polls] = srv.solve_counts
+            srv.close()
+        assert counts["0"] == (0, 0, len(sides)) and counts["200000"] == (len(sides), 0, 0)
+        assert counts["1"][1] >= 1 and counts["1"][0] + counts["1"][2] == len(sides)
+        for polls in ("1", "200000"):
+            for a, b in zip(out[polls], out["0"]):
+                assert np.array_equal(a["theta"], b["theta"]) and np.array_equal(a["tau"], b["tau"])
+
+
+@pytest.mark.parametrize("precision,precond,side", [("mixed", "DILU", 220), ("double", "DILU", 150),
+                                                    ("double", "diagonal", 120)])
+def test_resident_modes_equal_launches(precision, precond, side):
+    """The modes of a multiMode step as one group of resident solves, each more
+    than an XCD holds."""
+    m = cases.cartesian(side, side, 1, twoD=True, channel=True)
+    f = cases.make_fields(m, cases.FIELDS_CHANNEL, seed=5)
+    modes = [abi.model_dict("GiesekusLog", lam=lam, alpha=0.2, etaP=0.2) for lam in (0.5, 1.0, 2.0)]
+    body = "\n".join("M%d {%s}" % (i, t.split("{", 1)[1].rsplit("}", 1)[0]) for i, t in enumerate(modes))
+    text = "parameters\n{\n    type multiMode;\n    models\n    (\n" + body + "\n    );\n}\n"
+    out = []
+    for polls, counts in (("0", (0, 0, 6)), ("200000", (6, 0, 0)), ("1", None)):
+        print(f"[case] modes {side} {precision} {precond} residentPolls {polls}", flush=True)
+        with abi.Context(0) as ctx:
+            eq = ctx.constitutiveEq("", ctx.mesh(m), text)
+            eq.set_solver(abi.solver_dict(1e-10, precision=precision, precond=precond) + f" residentPolls {polls};")
+            for u in eq.modes():
+                u.set_state(f.theta, f.eigVals, f.eigVecs)
+            eq.set_flow(f.U, f.Ub, f.phi)
+            for _ in range(2):
+                eq.correct(0.1 / side)
+            got = [eq.tau()] + [u.theta() for u in eq.modes()]
+            n = ctx.solve_counts
+        out.append(got)
+        assert n == counts if counts else n[1] >= 1 and n[0] + n[2] == 6
+        assert all(np.array_equal(a, b) for a, b in zip(got, out[0]))
