@@ -1903,6 +1903,14 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     if (ok && P > 1 && threadIdx.x == 0) res_depart<ResAt>(bar);
 }
 
+// map: per workgroup of the grid its member and index in it, -1 for none
+template <class T, int FORM>
+__global__ void __launch_bounds__(RBLK, RES_PER_CU<T>) k_solve_group(const ResArgs<T>* __restrict__ tab, const int2* __restrict__ map) {
+    const int2 w = map[blockIdx.x];
+    if (w.x < 0) return;
+    solve_resident<T, FORM>(tab[w.x], w.y);
+}
+
 // workgroup b of the grid: b % XCDS is the XCD it is dealt to; xcd < 0: on all
 template <class T, int FORM>
 __global__ void __launch_bounds__(RBLK, RES_PER_CU<T>) k_solve_one(ResArgs<T> m, int xcd) {
@@ -2045,6 +2053,7 @@ struct SolveRun {
     uint32_t maxPolls = 0, epoch = 0;
     double* xSave = nullptr;
     SolveState* st = nullptr;
+    ResHold hold;  // the resident launch's CUs
     ~SolveRun() {
         if (hostState && ownsHost) ctx->givePinnedBlock(hostState);
         if (ev) (void)hipEventDestroy(ev);
@@ -2439,25 +2448,30 @@ auto with_form(int form, F&& f) {
     }
 }
 
+// whether a CU holds the workgroups its share of the budget stands for
 template <class T>
 bool resident_fits(int form) {
     return with_form<T>(form, [](auto F) {
-        static int perCU = -1;  // the same on every gfx950 device
-        if (perCU < 0) {
-            int nb = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_solve_one<T, decltype(F)::value>, RBLK, 0) != hipSuccess)
-                nb = 0;
-            perCU = nb;
-        }
-        return perCU >= RES_PER_CU<T>;
+        static const bool fits = [] {  // the same on every gfx950 device
+            int one = 0, grp = 0;
+            return hipOccupancyMaxActiveBlocksPerMultiprocessor(&one, k_solve_one<T, decltype(F)::value>, RBLK, 0) == hipSuccess &&
+                   hipOccupancyMaxActiveBlocksPerMultiprocessor(&grp, k_solve_group<T, decltype(F)::value>, RBLK, 0) == hipSuccess &&
+                   std::min(one, grp) >= RES_PER_CU<T>;
+        }();
+        return fits;
     });
 }
+
+constexpr int RES_DEVICES = 64;
+ResBudget resBudgets[RES_DEVICES];
+constexpr int HALF_CUS = 2;  // the budget's units on a CU
+int half_cus(const Ctx* ctx) { return HALF_CUS * ctx->numCUs / XCDS; }
 
 template <class T>
 void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     Krylov& K = *sa.kry;
     R.resident = R.resLaunched = false;
-    if (sa.ctl->residentPolls == 0 || ctx->profiling || K.N > RES_MAX_ROWS) return;
+    if (sa.ctl->residentPolls == 0 || ctx->profiling || K.N > RES_MAX_ROWS || ctx->device >= RES_DEVICES) return;
     if (R.G % 8 == 0 || K.partials.bytes < (size_t)RES_SUMS * K.grid * sizeof(double)) return;
     const Mesh& m = *sa.mesh;
     // row-kernel workgroups with a tile (their tiles in order: G is no multiple of 8)
@@ -2500,17 +2514,23 @@ ResArgs<T> resident_args(SolveRun& R) {
     return m;
 }
 
+// false: the device has no room for its workgroups beside the resident launches
+// under way (a single workgroup waits for none)
 template <class T>
-void launch_resident(Ctx* ctx, SolveRun& R) {
+bool launch_resident(Ctx* ctx, SolveRun& R) {
+    int xcd = ctx->xcd;
+    if (R.P > 1) {
+        xcd = resBudgets[ctx->device].take(R.P, HALF_CUS / RES_PER_CU<T>, half_cus(ctx), ctx->xcd, R.hold);
+        if (xcd == RES_FULL) return false;
+    }
     const ResArgs<T> m = resident_args<T>(R);
-    // on one XCD if they fit there
-    const int xcd = R.P <= RES_PER_CU<T> * ctx->numCUs / XCDS ? ctx->xcd : -1;
     const int grid = xcd < 0 ? R.P : R.P == 1 ? xcd + 1 : XCDS * R.P;
     with_form<T>(R.form, [&](auto F) {
         hipLaunchKernelGGL((k_solve_one<T, decltype(F)::value>), dim3(grid), dim3(RBLK), 0, ctx->stream, m, xcd);
     });
     RT_HIP(hipGetLastError());
     R.resLaunched = true;
+    return true;
 }
 
 // rounds a non-blocking advance queues per host round trip
@@ -2574,6 +2594,7 @@ void solve_begin(Ctx* ctx, const SolveArgs& sa) {
     }
     R.done = false;
     R.rounds = 0;
+    R.hold.release();
     if (mixed) {
         fill_args<float>(ctx, sa, R);
         choose_resident<float>(ctx, sa, R);
@@ -2636,9 +2657,9 @@ bool resident_done(Ctx* ctx, SolveRun& R) {
 bool solve_queue_resident(Ctx* ctx, Krylov& K, SolveGate& gate) {
     SolveRun& R = *K.run;
     if (!R.resident || R.resLaunched || R.done) return false;
-    if (R.mixed) launch_resident<float>(ctx, R);
-    else launch_resident<double>(ctx, R);
+    R.resident = R.mixed ? launch_resident<float>(ctx, R) : launch_resident<double>(ctx, R);
     queue_pull(ctx, K, R);
+    if (!R.resident) return false;
     gate = SolveGate{&R.st->resDone, R.epoch};
     return true;
 }
@@ -2670,6 +2691,7 @@ bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
             RT_HIP(e);
         }
         R.pending = false;
+        R.hold.release();
         if (R.neFromDevice) {
             R.ne = R.hostState->misc[0];
             R.neFromDevice = false;
@@ -2759,14 +2781,6 @@ __global__ void __launch_bounds__(BLK) k_group(const KryArgs<T>* __restrict__ ta
     Body(a, Blk{starts[i + 1] - starts[i], (int)blockIdx.x - starts[i], (int)threadIdx.x, red});
 }
 
-// map: per workgroup of the grid its member and index in it, -1 for none
-template <class T, int FORM>
-__global__ void __launch_bounds__(RBLK, RES_PER_CU<T>) k_solve_group(const ResArgs<T>* __restrict__ tab, const int2* __restrict__ map) {
-    const int2 w = map[blockIdx.x];
-    if (w.x < 0) return;
-    solve_resident<T, FORM>(tab[w.x], w.y);
-}
-
 template <class T, void (*Body)(const KryArgs<T>&, double*)>
 __global__ void __launch_bounds__(FBLK) k_group_fin(const KryArgs<T>* __restrict__ tab) {
     __shared__ double lds[FIN_LDS];
@@ -2841,50 +2855,39 @@ void group_tables(SolveGroup& g, size_t bytes) {
     if (g.tables.bytes < bytes) g.tables = g.ctx->alloc(bytes);
 }
 
-// A group of resident solves: every member's whole solve, in launches that
-// place at most RES_PER_CU workgroups per CU.  A member goes to the XCD with the fewest
-// workgroups so far (the largest members first would pack tighter; a queue's
-// order keeps its latency).
+// the member leaves the group and goes on by launches, behind the group's queued work
+void group_evict(SolveGroup& g, size_t i, std::vector<SolveGroup::Member>& evicted) {
+    SolveRun& R = *g.members[i].K->run;
+    R.resident = false;
+    queue_pull(g.ctx, *g.members[i].K, R);
+    evicted.push_back(g.members[i]);
+    g.members.erase(g.members.begin() + i);
+    g.dirty = true;
+}
+
+// A group of resident solves: every member's whole solve, in launches that the
+// budget has the CUs for.
 template <class T>
-void group_launch_resident(SolveGroup& g) {
-    const int n = (int)g.members.size();
-    struct Launch {
-        std::vector<int2> map;
-        int load[XCDS] = {0};
-        int form = 0;
-    };
-    std::vector<Launch> launches;
-    const int cap = RES_PER_CU<T> * g.ctx->numCUs / XCDS;
-    for (int i = 0; i < n; ++i) {
-        const int P = g.members[i].K->run->P, form = g.members[i].K->run->form;
-        const bool spread = P > cap;  // more than an XCD's CUs: over all of them
-        const int need = spread ? (P + XCDS - 1) / XCDS : P;
-        int x = 0;
-        if (!launches.empty()) {
-            const int* ld = launches.back().load;
-            x = (int)((spread ? std::max_element(ld, ld + XCDS) : std::min_element(ld, ld + XCDS)) - ld);
-        }
-        if (launches.empty() || launches.back().form != form || launches.back().load[x] + need > cap) {
-            launches.emplace_back();
-            launches.back().form = form;
-            x = 0;
-        }
-        Launch& L = launches.back();
-        for (int p = 0; p < P; ++p) {
-            if (spread) x = p % XCDS;
-            const size_t b = (size_t)XCDS * L.load[x]++ + x;
-            if (L.map.size() <= b) L.map.resize(b + 1, int2{-1, 0});
-            L.map[b] = int2{i, p};
-        }
-    }
+void group_launch_resident(SolveGroup& g, std::vector<SolveGroup::Member>& evicted) {
+    std::vector<ResMember> ms;
+    for (const auto& mb : g.members) ms.push_back({mb.K->run->P, mb.K->run->form});
+    std::vector<int> left;
+    const std::vector<ResLaunch> launches =
+        resBudgets[g.ctx->device].group(ms, HALF_CUS / RES_PER_CU<T>, half_cus(g.ctx), g.hold, left);
+    std::vector<SolveGroup::Member> all = g.members;  // the launches' maps index these
+    for (size_t k = left.size(); k-- > 0;) group_evict(g, left[k], evicted);
+    if (g.members.empty()) return;
+    const int n = (int)all.size();
     size_t blocks = 0;
     for (auto& L : launches) blocks += L.map.size();
     const size_t szA = sizeof(ResArgs<T>) * n, bytes = szA + sizeof(int2) * blocks;
     group_tables(g, bytes);
     auto* tab = static_cast<ResArgs<T>*>(g.hostTables);
     auto* map = reinterpret_cast<int2*>(static_cast<unsigned char*>(g.hostTables) + szA);
-    for (int i = 0; i < n; ++i) tab[i] = resident_args<T>(*g.members[i].K->run);
-    for (auto& L : launches) map = std::copy(L.map.begin(), L.map.end(), map);
+    for (int i = 0; i < n; ++i)
+        if (all[i].K->run->resident) tab[i] = resident_args<T>(*all[i].K->run);
+    for (auto& L : launches)
+        for (const auto& w : L.map) *map++ = int2{w[0], w[1]};
     RT_HIP(hipMemcpyAsync(g.tables.p, g.hostTables, bytes, hipMemcpyHostToDevice, g.ctx->stream));
     const auto* dt = static_cast<const ResArgs<T>*>(g.tables.p);
     const auto* dm = reinterpret_cast<const int2*>(static_cast<const unsigned char*>(g.tables.p) + szA);
@@ -2988,6 +2991,7 @@ void group_remove(SolveGroup& g, Krylov& K) {
     for (size_t i = 0; i < g.members.size(); ++i)
         if (g.members[i].K == &K) {
             RT_HIP(hipStreamSynchronize(g.ctx->stream));
+            g.hold.release();
             if (K.run) K.run->pending = false;
             g.members.erase(g.members.begin() + i);
             g.dirty = true;
@@ -2995,7 +2999,7 @@ void group_remove(SolveGroup& g, Krylov& K) {
         }
 }
 
-void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
+void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<SolveGroup::Member>& evicted) {
     bool allBack = true;
     for (auto& mb : g.members) {
         SolveRun& R = *mb.K->run;
@@ -3014,6 +3018,7 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
     }
     if (!allBack) return;
     g.launched = false;
+    g.hold.release();
     // members whose solve has finished leave; their streams go on after the
     // group's queued work (which reads them) has drained
     hipEvent_t drained = nullptr;
@@ -3025,9 +3030,8 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
         if (R.resident) {
             fin = R.resLaunched;
             if (fin && !resident_done(g.ctx, R)) {
-                // its resident launch gave up: by launches, to the end
-                while (!solve_advance(g.ctx, *g.members[i].K, true)) {
-                }
+                group_evict(g, i, evicted);
+                continue;
             }
         } else {
             fin = (nAct == 0 && nRef == 0) || R.rounds >= 100000;
@@ -3049,8 +3053,8 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished) {
     if (drained) RT_HIP(hipEventDestroy(drained));  // released once the waits are satisfied
     if (g.members.empty()) return;
     if (g.resident) {
-        if (g.mixed) group_launch_resident<float>(g);
-        else group_launch_resident<double>(g);
+        if (g.mixed) group_launch_resident<float>(g, evicted);
+        else group_launch_resident<double>(g, evicted);
     } else if (g.mixed) {
         group_launch<float>(g);
     } else {

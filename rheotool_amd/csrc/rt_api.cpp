@@ -1297,29 +1297,36 @@ int rt_model_correct_iter(rt_model* model, double deltaT, const double* gradU, i
                     while (!modelCorrectAdvance(mode->impl, true)) {
                     }
             } else {
-                SolveGroup G;
-                G.ctx = M.ctx;
-                G.mixed = mixed0;
-                G.rb = rb0;
+                SolveGroup G, L;  // L: the modes that leave a resident group for launches
+                G.ctx = L.ctx = M.ctx;
+                G.mixed = L.mixed = mixed0;
+                G.rb = L.rb = rb0;
                 G.resident = res0;
                 for (rt_model* mode : M.modes) group_join(G, mode->impl.kry, M.ctx->stream);
                 std::vector<Krylov*> done;
+                std::vector<SolveGroup::Member> evicted;
                 if (res0) {
-                    // the whole step is queued: the solves in one launch, each
-                    // mode's eigen/tau (run if its solve finishes) and the sum
-                    group_advance(G, done);
-                    for (rt_model* mode : M.modes) modelEigTau(mode->impl, solve_gate(mode->impl.kry));
-                    sumModes(M);
-                    summed = true;
+                    group_advance(G, done, evicted);
+                    if (evicted.empty()) {
+                        // the whole step is queued: the solves in one launch, each
+                        // mode's eigen/tau (run if its solve finishes) and the sum
+                        for (rt_model* mode : M.modes) modelEigTau(mode->impl, solve_gate(mode->impl.kry));
+                        sumModes(M);
+                        summed = true;
+                    }
                 }
-                while (!G.members.empty()) {
+                const bool queued = summed;
+                while (!G.members.empty() || !L.members.empty() || !evicted.empty()) {
+                    for (const auto& mb : evicted) group_join(L, *mb.K, mb.home);
+                    evicted.clear();
                     RT_HIP(hipStreamSynchronize(M.ctx->stream));  // the queued rounds' states are back
                     done.clear();
-                    group_advance(G, done);
+                    group_advance(G, done, evicted);
+                    group_advance(L, done, evicted);
                     for (Krylov* K : done)
                         for (rt_model* mode : M.modes) {
                             if (&mode->impl.kry != K) continue;
-                            if (solve_resident(*K)) {
+                            if (queued && solve_resident(*K)) {
                                 solve_finish(*K, mode->impl.perf);
                             } else {
                                 modelCorrectFinish(mode->impl);

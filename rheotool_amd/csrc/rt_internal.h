@@ -543,8 +543,9 @@ void solve_begin(Ctx* ctx, const SolveArgs& a);
 // the host's copy of the records, made before the assembly that fills it (NULL:
 // a caller's pageable block)
 SolveState* solve_prepare(Ctx* ctx, Krylov& K, SolveState* hostStatus = nullptr);
-// a begun solve that runs as one resident launch: queues it, true; work queued
-// behind it with its gate runs only if it finishes
+// a begun solve that runs as one resident launch: queues it if the device has the
+// CUs for it, true (else the solve goes on by launches); work queued behind it
+// with its gate runs only if it finishes
 bool solve_queue_resident(Ctx* ctx, Krylov& K, SolveGate& gate);
 SolveGate solve_gate(const Krylov& K);  // of a resident solve queued by its group
 bool solve_resident(const Krylov& K);   // a finished solve: its resident launch did it
@@ -562,6 +563,7 @@ int grid_for(const Ctx* ctx, int32_t N);
 struct SolveGroup {
     Ctx* ctx = nullptr;  // the group's stream and table memory
     bool mixed = false, rb = false, resident = false;
+    ResHold hold;  // a resident launch's CUs
     struct Member {
         Krylov* K;
         hipStream_t home;  // the stream the solve was begun on (and continues on)
@@ -582,8 +584,11 @@ void group_join(SolveGroup& g, Krylov& K, hipStream_t home);
 // Polls the members' states without blocking.  Members whose solve has
 // finished leave the group (their `home` stream first waits for the group's
 // queued work, which may still read them) and are appended to `finished`.
-// When every member's state is back, launches the next grouped rounds.
-void group_advance(SolveGroup& g, std::vector<Krylov*>& finished);
+// When every member's state is back, launches the next grouped rounds.  Members
+// whose resident launch gave up, or finds no room on the device, leave as well and
+// are appended to `evicted`: they are no longer resident, and join a group that
+// runs them by launches (one that shares this group's stream) or are advanced alone.
+void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<SolveGroup::Member>& evicted);
 // takes a member out (a failed request): waits for the group's queued work
 void group_remove(SolveGroup& g, Krylov& K);
 // looks up the device address of the no-allocation scratch array on the

@@ -2,7 +2,11 @@
 // its barriers.  Plain C++: the host tests run these rules against every
 // interleaving the kernels allow.
 #pragma once
+#include <algorithm>
+#include <array>
 #include <cstdint>
+#include <mutex>
+#include <vector>
 
 #ifdef __HIP__
 #define RES_FN __device__ __forceinline__
@@ -131,6 +135,129 @@ RES_FN void res_depart(const ResBar& B) {
         for (int i = 0; i < 3; ++i) At::template swap<RES_XCD>(&B.here[i], 0u);
     if (At::template add<RES_CHIP>(&B.bar[1], 1u) + 1u == (uint32_t)B.P)
         for (int i = 0; i < 8 + RES_XCDS; ++i) At::set(&B.bar[i], 0u);
+}
+
+// ------------------------------------------------------------------ host side
+// A barrier needs its workgroups on the chip together.  Two launches that each
+// got part of their workgroups placed wait for each other until their polls run
+// out, so the resident launches of a process take their CUs from one budget per
+// device: per XCD, in half CUs (an FP32 solve's workgroup takes half a CU's
+// registers, an FP64 one's a whole CU's).  What is held together always fits:
+// FP32 workgroups can share every CU that no FP64 one is on, and once they end,
+// which they do, the FP64 ones have a CU each.  Other kernels end by themselves.
+// Another process's launches are not counted: there the bounded wait remains.
+class ResBudget;
+struct ResHold {  // what a launch holds, given back once it has ended
+    ResBudget* from = nullptr;
+    int n[RES_XCDS] = {0};
+    ResHold() = default;
+    ResHold(const ResHold&) = delete;
+    ResHold& operator=(const ResHold&) = delete;
+    ~ResHold() { release(); }
+    inline void release();
+};
+
+// one launch of a group: workgroup b of the grid (on XCD b % RES_XCDS) is
+// {member, its workgroup}, {-1, 0} for none
+struct ResLaunch {
+    int form = 0;
+    int load[RES_XCDS] = {0};
+    std::vector<std::array<int32_t, 2>> map;
+};
+struct ResMember {
+    int P, form;
+};
+constexpr int RES_SPREAD = -1, RES_FULL = -2;
+
+class ResBudget {
+    std::mutex mu;
+    int held[RES_XCDS] = {0};
+    static int share(int P, int x) { return (P - x + RES_XCDS - 1) / RES_XCDS; }  // of P dealt over all XCDs
+
+   public:
+    // A launch of P workgroups of `unit` half CUs each; cap: half CUs of an XCD.
+    // The XCD (of those with room the one with most, from `first` on) that takes
+    // them all, RES_SPREAD: dealt over all, or RES_FULL
+    int take(int P, int unit, int cap, int first, ResHold& h) {
+        std::lock_guard<std::mutex> lk(mu);
+        int best = RES_FULL;
+        for (int i = 0; i < RES_XCDS; ++i) {
+            const int x = (first + i) % RES_XCDS;
+            if (held[x] + P * unit <= cap && (best < 0 || held[x] < held[best])) best = x;
+        }
+        if (best >= 0) {
+            h.n[best] = P * unit;
+        } else {
+            for (int x = 0; x < RES_XCDS; ++x)
+                if (held[x] + share(P, x) * unit > cap) return RES_FULL;
+            for (int x = 0; x < RES_XCDS; ++x) h.n[x] = share(P, x) * unit;
+            best = RES_SPREAD;
+        }
+        for (int x = 0; x < RES_XCDS; ++x) held[x] += h.n[x];
+        h.from = this;
+        return best;
+    }
+    // The launches, one after another on a stream, of a group of solves: a member
+    // goes to the XCD with the most room left, one that no XCD can take over all
+    // of them (the largest members first would pack tighter; a queue's order keeps
+    // its latency).  Holds the most any launch places on an XCD; left: the members
+    // no launch can take beside what others hold.
+    std::vector<ResLaunch> group(const std::vector<ResMember>& ms, int unit, int cap, ResHold& h, std::vector<int>& left) {
+        std::lock_guard<std::mutex> lk(mu);
+        int room[RES_XCDS];  // workgroups
+        for (int x = 0; x < RES_XCDS; ++x) room[x] = std::max(0, cap - held[x]) / unit;
+        std::vector<ResLaunch> out;
+        const ResLaunch none;
+        auto freest = [&](const ResLaunch& L) {
+            int b = 0;
+            for (int x = 1; x < RES_XCDS; ++x)
+                if (room[x] - L.load[x] > room[b] - L.load[b]) b = x;
+            return b;
+        };
+        auto spreads = [&](const ResLaunch& L, int P) {
+            for (int x = 0; x < RES_XCDS; ++x)
+                if (L.load[x] + share(P, x) > room[x]) return false;
+            return true;
+        };
+        for (int i = 0; i < (int)ms.size(); ++i) {
+            const int P = ms[i].P;
+            const bool one = room[freest(none)] >= P;
+            if (!one && !spreads(none, P)) {
+                left.push_back(i);
+                continue;
+            }
+            const bool open = !out.empty() && out.back().form == ms[i].form;
+            if (!open || !(one ? room[freest(out.back())] - out.back().load[freest(out.back())] >= P : spreads(out.back(), P))) {
+                out.emplace_back();
+                out.back().form = ms[i].form;
+            }
+            ResLaunch& L = out.back();
+            const int on = one ? freest(L) : RES_SPREAD;
+            for (int p = 0; p < P; ++p) {
+                const int x = one ? on : p % RES_XCDS;
+                const size_t b = (size_t)RES_XCDS * L.load[x]++ + x;
+                if (L.map.size() <= b) L.map.resize(b + 1, {-1, 0});
+                L.map[b] = {i, p};
+            }
+        }
+        for (int x = 0; x < RES_XCDS; ++x) {
+            h.n[x] = 0;
+            for (const ResLaunch& L : out) h.n[x] = std::max(h.n[x], L.load[x] * unit);
+            held[x] += h.n[x];
+        }
+        h.from = this;
+        return out;
+    }
+    void giveBack(const int (&n)[RES_XCDS]) {
+        std::lock_guard<std::mutex> lk(mu);
+        for (int x = 0; x < RES_XCDS; ++x) held[x] -= n[x];
+    }
+};
+inline void ResHold::release() {
+    if (!from) return;
+    from->giveBack(n);
+    from = nullptr;
+    for (int& v : n) v = 0;
 }
 
 }  // namespace rt

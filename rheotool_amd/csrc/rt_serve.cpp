@@ -108,6 +108,16 @@ void fail(rt_server* S, Request* r, int rc, const std::string& msg) {
     releaseRequest(S, r);
 }
 
+// group g: 4 for resident solves, 2 for mixed precision, 1 for red-black
+void joinGroup(rt_server* S, Request* r, int g, hipStream_t home) {
+    SolveGroup& G = S->groups[g];
+    G.resident = g & 4;
+    G.mixed = g & 2;
+    G.rb = g & 1;
+    group_join(G, r->model->impl.kry, home);
+    r->group = g;
+}
+
 // creates the device objects of a request in a free slot and launches its first work
 void admit(rt_server* S, Request* r, int slot) {
     rt_ctx* c = S->slots[slot];
@@ -144,13 +154,7 @@ void admit(rt_server* S, Request* r, int slot) {
         r->state = Request::RUNNING;
         bool mixed = false, rb = false, resident = false;
         if (S->batching && solve_groupable(M.kry, &mixed, &rb, &resident)) {
-            const int g = (resident ? 4 : 0) + (mixed ? 2 : 0) + (rb ? 1 : 0);
-            SolveGroup& G = S->groups[g];
-            G.mixed = mixed;
-            G.rb = rb;
-            G.resident = resident;
-            group_join(G, M.kry, c->impl.stream);
-            r->group = g;
+            joinGroup(S, r, (resident ? 4 : 0) + (mixed ? 2 : 0) + (rb ? 1 : 0), c->impl.stream);
             S->byKrylov[&M.kry] = r;
         }
     } catch (const Error& e) {
@@ -369,16 +373,26 @@ int rt_server_progress(rt_server* S) {
     }
     // batched Krylov rounds; requests whose solve finished go on with eigen/tau
     std::vector<Krylov*> done;
+    std::vector<SolveGroup::Member> evicted;
     for (auto& g : S->groups) {
         if (g.members.empty()) continue;
         done.clear();
+        evicted.clear();
         try {
             RT_HIP(hipSetDevice(S->gctx->impl.device));
-            group_advance(g, done);
+            group_advance(g, done, evicted);
+            // resident solves that go on by launches (at the next call: their group precedes this one)
+            while (!evicted.empty()) {
+                Request* r = S->byKrylov[evicted.back().K];
+                joinGroup(S, r, r->group & ~4, evicted.back().home);
+                evicted.pop_back();
+            }
         } catch (const Error& e) {
             // the batch's launch failed: every member fails with it
+            (void)hipStreamSynchronize(S->gctx->impl.stream);
             std::vector<Request*> members;
             for (auto& mb : g.members) members.push_back(S->byKrylov[mb.K]);
+            for (auto& mb : evicted) members.push_back(S->byKrylov[mb.K]);
             for (Request* r : members) fail(S, r, e.code, e.msg);
             continue;
         }

@@ -199,7 +199,108 @@ static void barrier(uint64_t seed) {
     }
 }
 
+// The budget: launches and groups come and go in random order.  No XCD is ever
+// promised more than it has, every member of a group has all its workgroups in one
+// launch on the XCDs counted, and what is held together ends: workgroups placed on
+// any CU with room, in any order, do not leave two launches waiting for each other.
+static void budget(uint64_t seed) {
+    std::mt19937_64 rng(seed);
+    const int cus = 2 + (int)(rng() % 6), cap = 2 * cus;
+    struct Job {  // one launch under way: workgroups per XCD, in `unit` half CUs
+        std::unique_ptr<ResHold> hold;
+        int unit;
+        std::vector<std::array<int, RES_XCDS>> launches;  // one after another
+        int placed[RES_XCDS] = {0};
+        std::vector<std::pair<int, int>> on;  // (XCD, CU) of its placed workgroups
+    };
+    ResBudget B;
+    std::vector<Job> jobs;
+    for (int i = 0; i < 6; ++i) {
+        Job j;
+        j.hold.reset(new ResHold);
+        j.unit = 1 + (int)(rng() % 2);
+        if (rng() % 2) {
+            const int P = 2 + (int)(rng() % (RES_XCDS * cus));
+            const int x = B.take(P, j.unit, cap, (int)(rng() % RES_XCDS), *j.hold);
+            if (x == RES_FULL) continue;
+            std::array<int, RES_XCDS> n{};
+            for (int p = 0; p < P; ++p) ++n[x == RES_SPREAD ? p % RES_XCDS : x];
+            j.launches.push_back(n);
+        } else {
+            std::vector<ResMember> ms;
+            for (int k = 0; k < 1 + (int)(rng() % 9); ++k)
+                ms.push_back({1 + (int)(rng() % (rng() % 3 ? 2 * cus : RES_XCDS * cus)), (int)(rng() % 2)});
+            std::vector<int> left;
+            const std::vector<ResLaunch> ls = B.group(ms, j.unit, cap, *j.hold, left);
+            std::vector<int> seen(ms.size(), 0), at(ms.size(), -1);
+            for (int i : left) seen[i] = ms[i].P;
+            for (size_t l = 0; l < ls.size(); ++l) {
+                std::array<int, RES_XCDS> n{};
+                for (size_t b = 0; b < ls[l].map.size(); ++b) {
+                    const int m = ls[l].map[b][0];
+                    if (m < 0) continue;
+                    CHECK(ms[m].form == ls[l].form && (at[m] == -1 || at[m] == (int)l), "member %d in two launches", m);
+                    at[m] = (int)l;
+                    CHECK(ls[l].map[b][1] < ms[m].P, "member %d has a workgroup too many", m);
+                    ++seen[m];
+                    ++n[b % RES_XCDS];
+                }
+                j.launches.push_back(n);
+            }
+            for (size_t m = 0; m < ms.size(); ++m) CHECK(seen[m] == ms[m].P, "member %d: %d of %d workgroups", (int)m, seen[m], ms[m].P);
+        }
+        for (const auto& n : j.launches)
+            for (int x = 0; x < RES_XCDS; ++x) CHECK(n[x] * j.unit <= j.hold->n[x], "XCD %d: more than is held", x);
+        jobs.push_back(std::move(j));
+    }
+    for (int x = 0; x < RES_XCDS; ++x) {
+        int sum = 0;
+        for (const Job& j : jobs) sum += j.hold->n[x];
+        CHECK(sum <= cap, "XCD %d: %d of %d half CUs promised", x, sum, cap);
+    }
+    // placement: used[x][c] half CUs; a launch ends once all its workgroups are placed
+    std::vector<std::vector<int>> used(RES_XCDS, std::vector<int>(cus, 0));
+    while (!jobs.empty()) {
+        std::vector<std::array<int, 3>> moves;  // job, XCD, CU
+        for (int k = 0; k < (int)jobs.size(); ++k) {
+            Job& j = jobs[k];
+            if (j.launches.empty()) {
+                moves.push_back({k, -1, -1});
+                continue;
+            }
+            bool all = true;
+            for (int x = 0; x < RES_XCDS; ++x)
+                if (j.placed[x] < j.launches[0][x]) {
+                    all = false;
+                    for (int c = 0; c < cus; ++c)
+                        if (used[x][c] + j.unit <= 2) moves.push_back({k, x, c});
+                }
+            if (all) moves.push_back({k, -1, -1});
+        }
+        CHECK(!moves.empty(), "launches wait for each other");
+        const auto mv = moves[rng() % moves.size()];
+        Job& j = jobs[mv[0]];
+        if (mv[1] >= 0) {
+            used[mv[1]][mv[2]] += j.unit;
+            ++j.placed[mv[1]];
+            j.on.push_back({mv[1], mv[2]});
+            continue;
+        }
+        for (auto& o : j.on) used[o.first][o.second] -= j.unit;
+        j.on.clear();
+        std::fill(j.placed, j.placed + RES_XCDS, 0);
+        if (!j.launches.empty()) j.launches.erase(j.launches.begin());
+        if (j.launches.empty()) {
+            j.hold->release();
+            jobs.erase(jobs.begin() + mv[0]);
+        }
+    }
+    ResHold h;
+    CHECK(B.take(RES_XCDS * cus, 2, cap, 3, h) == RES_SPREAD, "not everything was given back");
+}
+
 int main() {
+    for (uint64_t seed = 1; seed <= 2000; ++seed) budget(seed);
     for (uint64_t seed = 1; seed <= 500; ++seed) partial_sums(seed);
     for (uint64_t seed = 1; seed <= 5000; ++seed) barrier(seed);
     std::printf("launches finished %d, gave up %d, gave up behind the last barrier %d\n", finished, gaveUp, finalAll);

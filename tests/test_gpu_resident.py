@@ -3,6 +3,8 @@ launches: the fields and the solver records are the same bits, whatever the
 number of workgroups, the preconditioner form and the precision, also when a
 workgroup gives up its wait (residentPolls 1) and the solve is run again by
 launches from the saved theta.  residentPolls 0 never uses the resident launch."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -148,3 +150,44 @@ def test_resident_modes_equal_launches(precision, precond, side):
         out.append(got)
         assert n == counts if counts else n[1] >= 1 and n[0] + n[2] == 6
         assert all(np.array_equal(a, b) for a, b in zip(got, out[0]))
+
+
+def test_resident_solves_of_several_threads_do_not_wait_for_each_other():
+    """Threads whose resident solves take up to half the chip each, and a server's
+    batch beside them: those there is no room for run by launches, none gives up."""
+    sides, steps = (240, 225, 250, 240, 200, 240), 60
+    ms = [cases.cartesian(n, n, 1, twoD=True, channel=True) for n in sides]
+    fs = [cases.make_fields(m, cases.FIELDS_CHANNEL, seed=i) for i, m in enumerate(ms)]
+    controls = [abi.solver_dict(1e-10, precision="mixed" if i == 4 else "double") for i in range(len(sides))]
+    want = [step(m, f, c, steps) for m, f, c in zip(ms, fs, controls)]
+    got, served = {}, {}
+
+    def serve():
+        with abi.Context(0) as ctx:
+            reqs = [cases.cartesian(n, n, 1, twoD=True, channel=True) for n in (150, 100, 210, 60)]
+            flds = [cases.make_fields(m, cases.FIELDS_CHANNEL, seed=9) for m in reqs]
+            dms = [ctx.mesh(m) for m in reqs]
+            srv = abi.Server(ctx, max_inflight=8)
+            for _ in range(steps // 2):
+                for dm, f in zip(dms, flds):
+                    srv.submit(dm, f, abi.model_dict("Oldroyd-BLog"), 1e-3, abi.solver_dict(1e-10, precision="mixed"))
+                while srv.progress():
+                    pass
+            served["counts"] = srv.solve_counts
+            srv.close()
+
+    def run(i):
+        got[i] = step(ms[i], fs[i], controls[i], steps)
+
+    ts = [threading.Thread(target=run, args=(i,)) for i in range(len(sides))] + [threading.Thread(target=serve)]
+    print("[case] resident solves of seven threads", flush=True)
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    counts = [got[i][4] for i in range(len(sides))] + [served["counts"]]
+    print(counts)
+    assert all(c[1] == 0 for c in counts) and sum(counts[-1]) == 4 * (steps // 2)
+    for i in range(len(sides)):
+        assert want[i][4] == (steps, 0, 0)
+        assert got[i][:2] == want[i][:2] and all(np.array_equal(a, b) for a, b in zip(got[i][2:4], want[i][2:4]))
