@@ -2488,7 +2488,7 @@ void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     // 385 / 349 at 36864, 466 / 475 at 65536
     if (R.form < RF_RB_ROW && m.N > RES_MAX_ROWS / 2) return;
     if (R.P > 1 && !K.xSave.p) return;
-    if (!resident_fits<T>(R.form)) return;
+    if (!resident_fits<T>(R.form) || (R.P > 1 && ctx->backoff->skip())) return;
     R.maxPolls = sa.ctl->residentPolls;
     R.xSave = R.P > 1 ? K.xSave.as<double>() : nullptr;
     R.st = K.state.as<SolveState>();
@@ -2697,9 +2697,13 @@ bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
             R.neFromDevice = false;
         }
     }
-    if (R.resident && resident_done(ctx, R)) {
-        R.done = true;
-        return true;
+    if (R.resident) {
+        if (resident_done(ctx, R)) {
+            ctx->backoff->finished();
+            R.done = true;
+            return true;
+        }
+        ctx->backoff->gaveUp();
     }
     double nAct = 0, nRef = 0;
     bool start = true;  // every component of the round begins an inner solve (p = r = r0)
@@ -3022,6 +3026,7 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<So
     // members whose solve has finished leave; their streams go on after the
     // group's queued work (which reads them) has drained
     hipEvent_t drained = nullptr;
+    bool gaveUp = false;
     for (size_t i = 0; i < g.members.size();) {
         SolveRun& R = *g.members[i].K->run;
         double nAct = 0, nRef = 0;
@@ -3030,9 +3035,11 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<So
         if (R.resident) {
             fin = R.resLaunched;
             if (fin && !resident_done(g.ctx, R)) {
+                gaveUp = true;
                 group_evict(g, i, evicted);
                 continue;
             }
+            if (fin) g.ctx->backoff->finished();
         } else {
             fin = (nAct == 0 && nRef == 0) || R.rounds >= 100000;
         }
@@ -3050,6 +3057,7 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<So
             ++i;
         }
     }
+    if (gaveUp) g.ctx->backoff->gaveUp();
     if (drained) RT_HIP(hipEventDestroy(drained));  // released once the waits are satisfied
     if (g.members.empty()) return;
     if (g.resident) {

@@ -253,6 +253,24 @@ class ResBudget {
         for (int x = 0; x < RES_XCDS; ++x) held[x] -= n[x];
     }
 };
+// A wait that gave up cost the time of all its polls (about 0.1 s) and a step by
+// launches.  What kept the workgroups apart, another process's work, is likely to
+// be there at the next step too, so the context's next solves run by launches: 64
+// after the first, twice as many after each further one, until as many resident
+// solves as that have finished again.
+struct ResBackoff {
+    uint32_t pause = 0, span = 0, good = 0;
+    bool skip() { return pause > 0 && pause-- > 0; }  // of a solve that would run resident
+    void gaveUp() {
+        span = std::min(std::max(2 * span, 64u), 65536u);
+        pause = span;
+        good = 0;
+    }
+    void finished() {
+        if (span > 0 && ++good >= span) span = 0;
+    }
+};
+
 inline void ResHold::release() {
     if (!from) return;
     from->giveBack(n);

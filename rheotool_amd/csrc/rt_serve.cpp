@@ -252,6 +252,7 @@ int rt_server_create(rt_ctx* ctx, size_t hbm_budget, int max_inflight, rt_server
             ctx->impl.lastError = "rt_server_create: slot context creation failed";
             return rc;
         }
+        c->impl.backoff = &S->gctx->impl.ownBackoff;
         S->slots.push_back(c);
         S->slotReq.push_back(nullptr);
     }

@@ -191,3 +191,22 @@ def test_resident_solves_of_several_threads_do_not_wait_for_each_other():
     for i in range(len(sides)):
         assert want[i][4] == (steps, 0, 0)
         assert got[i][:2] == want[i][:2] and all(np.array_equal(a, b) for a, b in zip(got[i][2:4], want[i][2:4]))
+
+
+def test_after_a_wait_gave_up_the_next_solves_run_by_launches():
+    m = cases.cartesian(128, 128, 1, twoD=True, channel=True)
+    f = cases.make_fields(m, cases.FIELDS_CHANNEL, seed=1)
+    with abi.Context(0) as ctx:
+        eq = ctx.constitutiveEq("", ctx.mesh(m), abi.model_dict("GiesekusLog", lam=2.0, alpha=0.2))
+        eq.set_state(f.theta, f.eigVals, f.eigVecs)
+        eq.set_flow(f.U, f.Ub, f.phi)
+        solves = []
+        for polls, steps in (("1", 1), ("200000", 64), ("1", 1), ("200000", 128), ("200000", 128), ("1", 1), ("200000", 65)):
+            eq.set_solver(abi.solver_dict(1e-10) + f" residentPolls {polls};")
+            for _ in range(steps):
+                eq.correct(1e-4)
+            solves.append(ctx.solve_counts)
+        print(solves)
+        # (resident, gave up, by launches): 64 solves by launches after the first,
+        # 128 after the second; 64 again once 128 resident solves have finished
+        assert solves == [(0, 1, 1), (0, 1, 65), (0, 2, 66), (0, 2, 194), (128, 2, 194), (128, 3, 195), (129, 3, 259)]
