@@ -1987,8 +1987,6 @@ void Krylov::ensure(Ctx* run, Mesh& m, bool mixed, bool bicg) {
         ahat32 = DBuf(); ahat64 = DBuf();
         // a resident solve's reductions have slots of their own
         partials = ctx->alloc((size_t)grid * (N <= RES_MAX_ROWS ? RES_SUMS : 24) * sizeof(double));
-        xSave = DBuf();
-        if (N <= RES_MAX_ROWS && grid > RSUB) xSave = ctx->alloc(3 * vec * 8);
         state = ctx->alloc(sizeof(SolveState));
         // on the solve's stream: on the mesh's, behind other work, the zeros could
         // land on records the assembly had written
@@ -2051,7 +2049,7 @@ struct SolveRun {
     bool resident = false, resLaunched = false;
     int P = 1, X = 1, form = 0;
     uint32_t maxPolls = 0, epoch = 0;
-    double* xSave = nullptr;
+    DBuf xSave;  // the start of a resident solve of several workgroups (ResArgs::xSave)
     SolveState* st = nullptr;
     ResHold hold;  // the resident launch's CUs
     ~SolveRun() {
@@ -2487,10 +2485,9 @@ void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     // at 16384; the passes over memory of the other forms 338 / 266 at 16384,
     // 385 / 349 at 36864, 466 / 475 at 65536
     if (R.form < RF_RB_ROW && m.N > RES_MAX_ROWS / 2) return;
-    if (R.P > 1 && !K.xSave.p) return;
+    if (R.P > 1 && K.noAlloc && !K.xSave.p) return;
     if (!resident_fits<T>(R.form) || (R.P > 1 && ctx->backoff->skip())) return;
     R.maxPolls = sa.ctl->residentPolls;
-    R.xSave = R.P > 1 ? K.xSave.as<double>() : nullptr;
     R.st = K.state.as<SolveState>();
     R.resident = true;
 }
@@ -2510,15 +2507,37 @@ ResArgs<T> resident_args(SolveRun& R) {
     m.epoch = R.epoch = ++R.ctx->resEpoch;
     m.st = R.st;
     m.host = R.ownsHost ? R.hostState : nullptr;
-    m.xSave = R.xSave;
+    m.xSave = R.xSave.as<double>();
     return m;
 }
 
-// false: the device has no room for its workgroups beside the resident launches
-// under way (a single workgroup waits for none)
+// Memory for the solve's start, taken at the launch, behind everything the step
+// allocates, and given back when the solve has finished: a budget that holds the
+// step holds it without this, and then the solve runs by launches (false).
+bool take_save(Krylov& K, SolveRun& R) {
+    if (R.P == 1) return true;
+    const size_t bytes = sizeof(double) * NCMP * K.N * (1 + !R.rb + R.bicg);
+    if (K.noAlloc) {
+        R.xSave = DBuf::viewOf(K.xSave.p, K.xSave.bytes);
+        return true;
+    }
+    try {
+        // the mesh's context, where the solve's vectors are from; if that has a
+        // budget, a server's other requests may still need it
+        R.xSave = (K.ctx->budget ? R.ctx : K.ctx)->alloc(bytes);
+    } catch (const Error& e) {
+        if (e.code != RT_E_OOM) throw;
+        return false;
+    }
+    return true;
+}
+
+// false: no memory for its start, or the device has no room for its workgroups
+// beside the resident launches under way (a single workgroup waits for none)
 template <class T>
-bool launch_resident(Ctx* ctx, SolveRun& R) {
+bool launch_resident(Ctx* ctx, Krylov& K, SolveRun& R) {
     int xcd = ctx->xcd;
+    if (!take_save(K, R)) return false;
     if (R.P > 1) {
         xcd = resBudgets[ctx->device].take(R.P, HALF_CUS / RES_PER_CU<T>, half_cus(ctx), ctx->xcd, R.hold);
         if (xcd == RES_FULL) return false;
@@ -2595,6 +2614,7 @@ void solve_begin(Ctx* ctx, const SolveArgs& sa) {
     R.done = false;
     R.rounds = 0;
     R.hold.release();
+    R.xSave.release();
     if (mixed) {
         fill_args<float>(ctx, sa, R);
         choose_resident<float>(ctx, sa, R);
@@ -2644,9 +2664,10 @@ bool resident_done(Ctx* ctx, SolveRun& R) {
     const size_t n6 = (size_t)6 * (size_t)R.N;
     const size_t w = R.mixed ? sizeof(float) : sizeof(double);
     const size_t nv = (n6 * w + 15) / 16 * 16;  // whole 16-byte words; the buffers are padded to 256
-    launch_copy(ctx, R.xSave, R.mixed ? R.af.x : R.ad.x, n6 * sizeof(double));
-    if (!R.rb) launch_copy(ctx, R.xSave + n6, R.mixed ? (void*)R.af.r0 : (void*)R.ad.r0, nv);
-    if (R.bicg) launch_copy(ctx, R.xSave + 2 * n6, R.mixed ? (void*)R.af.r : (void*)R.ad.r, nv);
+    const double* save = R.xSave.as<double>();
+    launch_copy(ctx, save, R.mixed ? R.af.x : R.ad.x, n6 * sizeof(double));
+    if (!R.rb) launch_copy(ctx, save + n6, R.mixed ? (void*)R.af.r0 : (void*)R.ad.r0, nv);
+    if (R.bicg) launch_copy(ctx, save + 2 * n6, R.mixed ? (void*)R.af.r : (void*)R.ad.r, nv);
     R.resident = R.resLaunched = false;
     R.needScale = R.nEll > 0;
     return false;
@@ -2657,7 +2678,7 @@ bool resident_done(Ctx* ctx, SolveRun& R) {
 bool solve_queue_resident(Ctx* ctx, Krylov& K, SolveGate& gate) {
     SolveRun& R = *K.run;
     if (!R.resident || R.resLaunched || R.done) return false;
-    R.resident = R.mixed ? launch_resident<float>(ctx, R) : launch_resident<double>(ctx, R);
+    R.resident = R.mixed ? launch_resident<float>(ctx, K, R) : launch_resident<double>(ctx, K, R);
     queue_pull(ctx, K, R);
     if (!R.resident) return false;
     gate = SolveGate{&R.st->resDone, R.epoch};
@@ -2874,8 +2895,10 @@ void group_evict(SolveGroup& g, size_t i, std::vector<SolveGroup::Member>& evict
 template <class T>
 void group_launch_resident(SolveGroup& g, std::vector<SolveGroup::Member>& evicted) {
     std::vector<ResMember> ms;
-    for (const auto& mb : g.members) ms.push_back({mb.K->run->P, mb.K->run->form});
     std::vector<int> left;
+    for (size_t i = g.members.size(); i-- > 0;)
+        if (!take_save(*g.members[i].K, *g.members[i].K->run)) group_evict(g, i, evicted);
+    for (const auto& mb : g.members) ms.push_back({mb.K->run->P, mb.K->run->form});
     const std::vector<ResLaunch> launches =
         resBudgets[g.ctx->device].group(ms, HALF_CUS / RES_PER_CU<T>, half_cus(g.ctx), g.hold, left);
     std::vector<SolveGroup::Member> all = g.members;  // the launches' maps index these
@@ -3073,6 +3096,7 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<So
 void solve_finish(Krylov& K, rt_solver_perf perf[6]) {
     SolveRun& R = *K.run;
     ++R.ctx->solveCounts[R.resident ? 0 : 2];
+    R.xSave.release();  // the launches that use it have ended
     for (int c = 0; c < 6; ++c) {
         rt_solver_perf& pf = perf[c];
         pf = rt_solver_perf{0, 0, 0, 0, 0, 0};

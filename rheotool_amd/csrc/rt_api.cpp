@@ -658,7 +658,6 @@ size_t modelBytesEstimate(int32_t N, int32_t F, int32_t NB, int64_t nEll, bool m
     // Krylov: r r0 p v t (and the mixed solve's correction e) x 6 components,
     // rD, ahat, partials, state
     by += 6 * n * (mixed ? 6 * 4 : 5 * 8) + 8 * n + ne * (mixed ? 4 : 8) + 2048 * 24 * 8 + 4096;
-    if (N <= RES_MAX_ROWS) by += 3 * 6 * 8 * n + 2048 * 12 * 8;  // resident solve: its saved start, more partials
     // staging for AoS transfers (9 comps)
     by += 9 * 8 * n;
     if (gradU) by += 9 * 8 * n;      // the prescribed gradient
@@ -667,6 +666,9 @@ size_t modelBytesEstimate(int32_t N, int32_t F, int32_t NB, int64_t nEll, bool m
     // out blocks up to 1.5 times a request; 1.25 covers the usual mix
     return (size_t)(by * 1.25) + (1u << 20);
 }
+
+// what its solve takes on top while it runs resident, where there is room for it
+size_t residentBytesEstimate(int32_t N) { return N <= RES_MAX_ROWS ? (size_t)(3 * 6 * 8 * 1.25 * N) : 0; }
 
 }  // namespace rt
 

@@ -275,7 +275,7 @@ struct Krylov {
     DBuf rDs;              // double [N]    red-black: 1/diag of the Schur complement
                            // (the ILU0 diagonal) where it differs from 1/diag
     DBuf partials;         // double [grid][24] (RES_SUMS on a mesh of at most RES_MAX_ROWS rows)
-    DBuf xSave;            // FP64 [3][N][6] the start of a resident solve of several workgroups
+    DBuf xSave;            // no-allocation path: FP64 [3][N][6] for the start of a resident solve
     DBuf state;            // SolveState
     std::unique_ptr<SolveRun, SolveRunDeleter> run;
     // set when the buffers above are views into the no-allocation scratch
@@ -611,6 +611,7 @@ void modelCorrect(Model& M, double deltaT, const double* gradU, int iteration = 
 // device bytes a model of this size allocates (for admission control)
 size_t modelBytesEstimate(int32_t N, int32_t F, int32_t NB, int64_t nEll, bool mixed, bool gradU = false,
                           bool download = false);
+size_t residentBytesEstimate(int32_t N);
 
 }  // namespace rt
 

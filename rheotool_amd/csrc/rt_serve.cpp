@@ -141,6 +141,14 @@ void admit(rt_server* S, Request* r, int slot) {
     }
     try {
         RT_HIP(hipSetDevice(c->impl.device));
+        // a resident solve's own memory, where the budget has room for it beside the request
+        const size_t res = residentBytesEstimate(r->nCells);
+        if (S->budget && S->inflightBytes + res > S->budget) {
+            r->model->impl.ctl.residentPolls = 0;
+        } else {
+            r->estBytes += res;
+            S->inflightBytes += res;
+        }
         // the request's arrays stay unchanged until its ticket finishes, so
         // the uploads are queued without waiting for them
         Model& M = r->model->impl;

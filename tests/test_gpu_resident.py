@@ -210,3 +210,53 @@ def test_after_a_wait_gave_up_the_next_solves_run_by_launches():
         # (resident, gave up, by launches): 64 solves by launches after the first,
         # 128 after the second; 64 again once 128 resident solves have finished
         assert solves == [(0, 1, 1), (0, 1, 65), (0, 2, 66), (0, 2, 194), (128, 2, 194), (128, 3, 195), (129, 3, 259)]
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+def test_a_budget_that_holds_the_launches_holds_the_step(precision):
+    """The memory a resident solve saves its start in is taken if there is room:
+    a context whose budget is just what the same steps take by launches runs them
+    by launches, also with two modes, and one with more runs them resident."""
+    m = cases.cartesian(120, 110, 1, twoD=True, channel=True)
+    f = cases.make_fields(m, cases.FIELDS_CHANNEL, seed=2)
+    one = abi.model_dict("GiesekusLog", lam=2.0, alpha=0.2)
+    body = "\n".join("M%d {%s}" % (i, one.split("{", 1)[1].rsplit("}", 1)[0]) for i in range(2))
+    for text, solves in ((one, 2), ("parameters\n{\n    type multiMode;\n    models\n    (\n" + body + "\n    );\n}\n", 4)):
+        def run(budget, polls):
+            with abi.Context(0, hbm_budget=budget) as ctx:
+                eq = ctx.constitutiveEq("", ctx.mesh(m), text)
+                eq.set_solver(abi.solver_dict(1e-10, precision=precision) + polls)
+                for u in eq.modes() or [eq]:
+                    u.set_state(f.theta, f.eigVals, f.eigVecs)
+                eq.set_flow(f.U, f.Ub, f.phi)
+                for _ in range(2):
+                    eq.correct(1e-3)
+                used = ctx.bytes_in_use
+                return eq.tau(), ctx.solve_counts, used
+        want, counts, used = run(0, " residentPolls 0;")
+        assert counts == (0, 0, solves)
+        used_at_most = used + (16 << 10)  # a group's argument tables, held during a step
+        for budget, polls, counts in ((used_at_most, " residentPolls 0;", (0, 0, solves)),
+                                      (used_at_most, "", (0, 0, solves)), (2 * used, "", (solves, 0, 0))):
+            print(f"[case] budget {budget} {precision} {solves}{polls}", flush=True)
+            got = run(budget, polls)
+            assert got[1] == counts and got[2] == used and np.array_equal(got[0], want)
+
+
+def test_a_servers_budget_admits_what_it_admitted_without_resident_solves():
+    m = cases.cartesian(120, 110, 1, twoD=True, channel=True)
+    f = cases.make_fields(m, cases.FIELDS_CHANNEL, seed=2)
+    with abi.Context(0) as ctx:
+        dm = ctx.mesh(m)
+        est = abi.lib().rt_request_bytes_estimate(dm.h, 1, 0)
+        out = []
+        for budget, counts in ((est, (0, 0, 3)), (2 * est, (3, 0, 0))):
+            print(f"[case] server budget {budget}", flush=True)
+            srv = abi.Server(ctx, hbm_budget=budget, max_inflight=1)
+            ts = [srv.submit(dm, f, abi.model_dict("Oldroyd-BLog"), 1e-3) for _ in range(3)]
+            while srv.progress():
+                pass
+            out += [srv.poll(t)["theta"] for t in ts]
+            assert srv.solve_counts == counts
+            srv.close()
+        assert all(np.array_equal(a, out[0]) for a in out)
