@@ -879,9 +879,11 @@ __global__ void k_ldu_to_ell(int64_t nEll, int32_t nSlices, const int64_t* __res
     const int32_t f = fid[e];
     aval[col_slot(e, off, slot, nSlices)] = f == RT_FID_PAD ? 0.0 : (f >= 0 ? upper[f] : lower[-f - 1]);
 }
-__global__ void k_face_to_entry(int64_t nEll, const int32_t* __restrict__ fid,
-                                const double* __restrict__ phi, double* __restrict__ ePhi) {
+__global__ void k_face_to_entry(int64_t nEll, int32_t F, int32_t NB, const int32_t* __restrict__ fid,
+                                const double* __restrict__ phi, double* __restrict__ ePhi,
+                                double* __restrict__ phiB) {
     const int64_t e = (int64_t)blockIdx.x * BLK + threadIdx.x;
+    if (e < NB) phiB[e] = phi[F + e];
     if (e >= nEll) return;
     const int32_t f = fid[e];
     ePhi[e] = f == RT_FID_PAD ? 0.0 : phi[f >= 0 ? f : -f - 1];
@@ -1575,10 +1577,11 @@ void launch_ldu_to_ell(Ctx* ctx, const Mesh& m, const double* lower, const doubl
                        upper, aval);
     RT_HIP(hipGetLastError());
 }
-void launch_face_to_entry(Ctx* ctx, const Mesh& m, const double* phi, double* ePhi) {
-    if (m.nEll <= 0) return;
-    hipLaunchKernelGGL(k_face_to_entry, dim3(nblk(m.nEll)), dim3(BLK), 0, ctx->stream, m.nEll,
-                       m.ellFid.as<int32_t>(), phi, ePhi);
+void launch_face_to_entry(Ctx* ctx, const Mesh& m, const double* phi, double* ePhi, double* phiB) {
+    const int64_t n = std::max<int64_t>(m.nEll, m.NB);
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_face_to_entry, dim3(nblk(n)), dim3(BLK), 0, ctx->stream, m.nEll,
+                       m.F, m.NB, m.ellFid.as<int32_t>(), phi, ePhi, phiB);
     RT_HIP(hipGetLastError());
 }
 // `in` and `out` lie on 16-byte boundaries, as every buffer of the runtime does

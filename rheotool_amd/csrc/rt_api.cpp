@@ -459,8 +459,8 @@ void modelUploadFlow(Model& M, const double* U, const double* Ub, const double* 
         uploadAos(c, st, Ub, (int64_t)3 * m.NB);
         launch_aos_to_soa(c, m.NB, 3, st.as<double>(), nullptr, M.Ub.as<double>());
     }
-    RT_HIP(hipMemcpyAsync(M.phi.p, phi, ((size_t)m.F + m.NB) * 8, hipMemcpyHostToDevice, c->stream));
-    launch_face_to_entry(c, m, M.phi.as<double>(), M.ePhi.as<double>());
+    uploadAos(c, st, phi, (int64_t)m.F + m.NB);
+    launch_face_to_entry(c, m, st.as<double>(), M.ePhi.as<double>(), M.phiB.as<double>());
     if (wait) RT_HIP(hipStreamSynchronize(c->stream));
     M.hasFlow = true;
 }
@@ -504,7 +504,7 @@ AssembleArgs meshArgs(Model& M) {
     a.patchT = M.patchT.as<double>();
     a.NB = m.NB;
     a.bSf = m.bSf.as<double>();
-    a.phiB = M.phi.as<double>() + m.F;
+    a.phiB = M.phiB.as<double>();
     a.V = m.V.as<double>();
     a.U = M.U.as<double>();
     a.Ub = M.Ub.as<double>();
@@ -652,14 +652,14 @@ void modelCorrect(Model& M, double deltaT, const double* gradU, int iteration) {
 size_t modelBytesEstimate(int32_t N, int32_t F, int32_t NB, int64_t nEll, bool mixed, bool gradU, bool download) {
     const double n = N, f = F, nb = NB, ne = (double)nEll;
     double by = 0;
-    // model state + flow + matrix: theta tau eigVal eigVec U b diag fOld, Ub, phi, bc, ePhi, aval
-    by += 8 * n * (6 + 6 + 3 + 9 + 4 + 6 + 1 + 1) + 8 * (3 * nb + f + nb) + 6 * 8 * nb + 8 * ne + 8 * ne +
+    // model state + flow + matrix: theta tau eigVal eigVec U b diag fOld, Ub, phiB, bc, ePhi, aval
+    by += 8 * n * (6 + 6 + 3 + 9 + 4 + 6 + 1 + 1) + 8 * (3 * nb + nb) + 6 * 8 * nb + 8 * ne + 8 * ne +
           4 * n / 64;
     // Krylov: r r0 p v t (and the mixed solve's correction e) x 6 components,
     // rD, ahat, partials, state
     by += 6 * n * (mixed ? 6 * 4 : 5 * 8) + 8 * n + ne * (mixed ? 4 : 8) + 2048 * 24 * 8 + 4096;
-    // staging for AoS transfers (9 comps)
-    by += 9 * 8 * n;
+    // staging for AoS transfers (9 comps, or the face fluxes)
+    by += 8 * std::max(9 * n, f + nb);
     if (gradU) by += 9 * 8 * n;      // the prescribed gradient
     if (download) by += 2 * 6 * 8 * n;  // theta and tau in the caller's order on their way home
     // size classes round each buffer up by at most 1/8, and the cache hands
@@ -1062,7 +1062,7 @@ void allocModelState(Model& M) {
         M.eigVec = c->alloc((size_t)9 * N * 8);
         M.U = c->alloc((size_t)4 * N * 8);
         M.Ub = c->alloc((size_t)3 * std::max(1, NB) * 8);
-        M.phi = c->alloc(((size_t)M.mesh->F + NB) * 8);
+        M.phiB = c->alloc((size_t)std::max(1, NB) * 8);
         M.ePhi = c->alloc((size_t)std::max<int64_t>(1, M.mesh->nEll) * 8);
         M.bcType = c->alloc((size_t)std::max(1, M.mesh->nPatches) * 4);
         M.bcVal = c->alloc((size_t)6 * std::max(1, NB) * 8);

@@ -342,7 +342,7 @@ struct Model {
     DBuf eigVec;            // [9][N]
     DBuf U;                 // [N][4] interleaved (4th slot unused)
     DBuf Ub;                // [3][NB]
-    DBuf phi;               // [F+NB] caller's face order
+    DBuf phiB;              // [NB] boundary fluxes (the interior ones are in ePhi)
     DBuf ePhi;              // [nEll] face flux per ELL entry (face order)
     DBuf gradU;             // [9][N] when supplied
     DBuf diag, aval, b, fOld;  // matrix (column order) / sources [N][6] of the step
@@ -468,7 +468,8 @@ void launch_rows_in3(Ctx* ctx, const Mesh& m, const double* in, double* out);
 void launch_rows_out6(Ctx* ctx, const Mesh& m, const double* in, double* out);
 void launch_rows_out3(Ctx* ctx, const Mesh& m, const double* in, double* out);
 // per-entry face flux: ePhi[e] = phi[face of entry e]
-void launch_face_to_entry(Ctx* ctx, const Mesh& m, const double* phi, double* ePhi);
+// and phiB[b] = phi[F + b]
+void launch_face_to_entry(Ctx* ctx, const Mesh& m, const double* phi, double* ePhi, double* phiB);
 void launch_eigvals_from_tensor(Ctx* ctx, int32_t N, const double* aos9, const int32_t* perm,
                                 double* eigVal);
 void launch_eigvals_to_tensor(Ctx* ctx, int32_t N, const double* eigVal, const int32_t* perm,

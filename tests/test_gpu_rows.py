@@ -38,3 +38,22 @@ def test_fields_in_and_out(ctx, shape, renumber):
     assert np.array_equal(eq.tau(), tau)
     assert close(eq.tau_total(), O.tau_total(m, f.U, f.Ub, tau, 0.3))
     assert close(eq.div_tau(), O.div_tau(m, tau, None, 1.0))
+
+
+@pytest.mark.parametrize("shape,precision,was", [((40, 36, 30), "double", 47418112), ((40, 36, 30), "mixed", 42081280),
+                                                 ((96, 96, 96), "double", 1015474432), ((120, 110, 1), "mixed", 14131200)])
+def test_a_step_fits_the_device_memory_it_fitted(shape, precision, was):
+    """A mesh, a model and its step take what they took before the meshes kept
+    the face loops' column words and the cells' rows (`was`, bytes measured then;
+    half a per cent for the size classes), so that a context's budget holds them
+    as before."""
+    print(f"[case] memory {shape} {precision}", flush=True)
+    m = cases.cartesian(*shape, twoD=shape[2] == 1, channel=True)
+    f = cases.make_fields(m, cases.FIELDS_CHANNEL, seed=2)
+    with abi.Context(0) as c:
+        eq = c.constitutiveEq("", c.mesh(m), abi.model_dict("GiesekusLog", lam=2.0, alpha=0.2))
+        eq.set_solver(abi.solver_dict(1e-10, precision=precision))
+        eq.set_state(f.theta, f.eigVals, f.eigVecs)
+        eq.set_flow(f.U, f.Ub, f.phi)
+        eq.correct(1e-3)
+        assert c.bytes_in_use <= 1.005 * was
