@@ -20,6 +20,8 @@
 // solve of the FP64-refined "mixed" solve).  x (theta), b, the matrix used
 // for the true residual and the grid-level reductions are FP64; per-thread
 // partial sums use T.
+#include <unistd.h>
+
 #include <cstring>
 
 #include "rt_device.h"
@@ -2639,6 +2641,13 @@ void solve_begin(Ctx* ctx, const SolveArgs& sa) {
 
 namespace {
 
+void back_off(Ctx* ctx) {
+    ctx->backoff->gaveUp();
+    // the contexts of processes that share a device all start on the same XCDs:
+    // each leaves in steps of its own
+    ctx->xcd = (ctx->xcd + 1 + (int)(getpid() % (XCDS - 1))) % XCDS;
+}
+
 // components of the state last pulled that are still iterating or waiting for a sweep
 void open_components(const SolveRun& R, double& nAct, double& nRef) {
     nAct = nRef = 0;
@@ -2724,7 +2733,7 @@ bool solve_advance(Ctx* ctx, Krylov& K, bool block) {
             R.done = true;
             return true;
         }
-        ctx->backoff->gaveUp();
+        back_off(ctx);
     }
     double nAct = 0, nRef = 0;
     bool start = true;  // every component of the round begins an inner solve (p = r = r0)
@@ -3080,7 +3089,7 @@ void group_advance(SolveGroup& g, std::vector<Krylov*>& finished, std::vector<So
             ++i;
         }
     }
-    if (gaveUp) g.ctx->backoff->gaveUp();
+    if (gaveUp) back_off(g.ctx);
     if (drained) RT_HIP(hipEventDestroy(drained));  // released once the waits are satisfied
     if (g.members.empty()) return;
     if (g.resident) {

@@ -3,8 +3,6 @@
 // Context (device, stream, HBM budget, kernel timing), mesh and model
 // handles, the constitutiveEq run-time selection from dictionary text, the
 // correct() sequence and the sparseSolver<symmTensor>::solve surface.
-#include <unistd.h>
-
 #include <algorithm>
 #include <atomic>
 #include <cctype>
@@ -792,8 +790,7 @@ int rt_ctx_create(int device, size_t hbm_budget, rt_ctx** out) {
             throw Error{RT_E_NO_DEVICE, std::string("device ") + std::to_string(device) + " is " +
                                             prop.gcnArchName + "; this library is built for gfx950"};
         x.numCUs = prop.multiProcessorCount;
-        // processes that share a device start at different XCDs
-        static std::atomic<unsigned> made{(unsigned)getpid()};
+        static std::atomic<unsigned> made{0};
         x.xcd = (int)(made.fetch_add(1) % RES_XCDS);
         x.budget = hbm_budget;
         RT_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));

@@ -71,7 +71,8 @@ struct Ctx {
     int numCUs = 256;
     uint32_t resEpoch = 0;  // resident launches so far
     int64_t solveCounts[3] = {0, 0, 0};  // finished resident, gave up, finished by launches
-    int xcd = 0;  // where its resident solves look for room first: contexts take turns
+    int xcd = 0;  // where its resident solves look for room first: contexts take turns,
+                  // and move on after a wait gave up
     ResBackoff ownBackoff, *backoff = &ownBackoff;  // a server's slots share one
     hipStream_t stream = nullptr;
     size_t budget = 0, inUse = 0;
