@@ -1491,8 +1491,8 @@ static int launch_assemble_kind(Ctx* ctx, const AssembleArgs& a, int cap) {
 void launch_assemble(Ctx* ctx, const AssembleArgs& a, int grid) {
     // algorithmic bytes per cell: theta 48, eigen state 96, U 32, V 8, b 48, diag 8, 1/diag 8,
     // the residual (6 x w, unless the solve writes it), theta.oldTime() 48 more in inner
-    // iterations, the old tau 48 for Saramito; per ELL entry: face id 4, slot 1, column 4,
-    // phi 8, value 8 (+ Sf 24 and w 8 for the gradient)
+    // iterations, the old tau 48 for Saramito; per ELL entry: column 4, slot 1, phi 8,
+    // value 8 (+ Sf 24 and w 8 for the gradient)
     const double w = a.mixed ? 4 : 8;
     const double by = (double)a.N * (48 + 96 + 32 + 8 + 48 + 8 + 8 + (a.r ? 6 * w : 0) + (a.thetaOld ? 48 : 0) +
                                      (a.tauOld ? 48 : 0) + (a.aux ? 8 : 0)) +

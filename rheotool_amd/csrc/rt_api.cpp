@@ -486,8 +486,6 @@ AssembleArgs meshArgs(Model& M) {
     a.N = m.N;
     a.ellOff = m.ellOff.as<int64_t>();
     a.ellWidth = m.ellWidth.as<int32_t>();
-    a.ellCol = m.ellCol.as<int32_t>();
-    a.ellFid = m.ellFid.as<int32_t>();
     a.ellSlot = m.ellSlot.as<uint8_t>();
     a.eCol = m.eCol.as<int32_t>();
     a.eSf = m.eSf.as<double>();

@@ -381,8 +381,6 @@ struct AssembleArgs {
     int32_t N;
     const int64_t* ellOff;
     const int32_t* ellWidth;
-    const int32_t* ellCol;
-    const int32_t* ellFid;
     const uint8_t* ellSlot;
     const int32_t* eCol;
     const double* eSf;    // [3][nEll]
