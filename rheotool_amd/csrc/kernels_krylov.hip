@@ -219,7 +219,7 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& 
     // (the first colour's residual is zero once it has been eliminated)
     const int32_t rowB = a.rowBegin & ~(SLICE - 1);  // wavefronts on whole slices
     const int64_t nRows = (int64_t)a.N - rowB;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = a.rowBegin > 0 ? tile_of_g(it, nRows, 0, k_.G, k_.b) : tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -335,7 +335,7 @@ __device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, const Blk& k_)
     }
     const T* pOld = q.inner == 1 ? a.r0 : a.p;
     const int64_t N = a.N;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
         T rr[6], pp[6], vv[6];
         ld6(a.r + NCMP * i, rr);
         ld6(pOld + NCMP * i, pp);
@@ -359,7 +359,7 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_)
     if (!rd.any) return;
     const T* pv = rd.inner == 0 ? a.r0 : a.p;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -429,7 +429,7 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
     T q[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -525,7 +525,7 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
     for (int i = 0; i < 12; ++i) q[i] = 0;
     // red-black: the second colour's rows, as the v and t passes take them
     const int32_t first = a.ctl.rb ? a.nRed : 0, row0 = first & ~(SLICE - 1);
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, (int64_t)a.N - row0, a.ctl.rb ? 0 : a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -610,7 +610,7 @@ __device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, const Blk& k_) 
         any |= on[c];
     }
     if (!any || inner_running(a)) return;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < a.N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
         double xv[6];
         T ev[6];
         ld6(a.x + NCMP * i, xv);
@@ -722,7 +722,7 @@ __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) 
 #pragma unroll
     for (int c = 0; c < 6; ++c) alpha[c] = (T)uni(a.cs[c].alpha);
     const int64_t n = a.nRed;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -755,7 +755,7 @@ __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) 
     T q[6] = {0, 0, 0, 0, 0, 0};
     const int32_t r0b = a.nRed & ~(SLICE - 1);  // wavefronts on whole slices
     const int64_t n = (int64_t)a.N - r0b;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -805,7 +805,7 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) 
     for (int i = 0; i < 18; ++i) q[i] = 0;
     const int32_t r0b = a.nRed & ~(SLICE - 1);  // wavefronts on whole slices
     const int64_t n = (int64_t)a.N - r0b;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -857,7 +857,7 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, const Blk
     }
     if (!any || inner_running(a)) return;
     const int64_t n = a.nRed;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -934,7 +934,7 @@ __device__ __forceinline__ void k_bicg_init_body(const KryArgs<T>& a, const Blk&
     }
     if (!any) return;
     double q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1008,7 +1008,7 @@ __device__ __forceinline__ void k_bicg_p_body(const KryArgs<T>& a, const Blk& k_
         any |= on[c];
     }
     if (!any) return;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < a.N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
         const T rm = a.rM ? (T)a.rM[i] : (T)1;
         T rA[6], rT[6], pA[6], pT[6];
         ld6(a.r + NCMP * i, rA);
@@ -1044,7 +1044,7 @@ __device__ __forceinline__ void k_bicg_w_body(const KryArgs<T>& a, const Blk& k_
     }
     if (!any) return;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1134,7 +1134,7 @@ __device__ __forceinline__ void k_bicg_xr_body(const KryArgs<T>& a, const Blk& k
     T q[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
-    for (int64_t it = 0; k_.b < k_.G; ++it) {
+    for (int64_t it = 0;; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1256,7 +1256,7 @@ __global__ void k_rdiag(int32_t N, const double* __restrict__ diag, double* __re
 template <class T>
 __device__ __forceinline__ void k_scale_body(const KryArgs<T>& a, const Blk& k_) {
     T* ahat = const_cast<T*>(a.ahat);
-    for (int64_t r = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && r < a.N; r += (int64_t)k_.G * BLK) {
+    for (int64_t r = (int64_t)k_.b * BLK + k_.tid; r < a.N; r += (int64_t)k_.G * BLK) {
         const int s = (int)(r >> 6), lane = (int)(r & 63);
         const int64_t base = a.ellOff[s] + lane;
         const int w = a.ellWidth[s];
@@ -1311,8 +1311,8 @@ __global__ void __launch_bounds__(FBLK) k_fin_mean6(int32_t N, int G, const doub
 // is a few microseconds of dependent loads and a launch costs as much again; a
 // 128 x 128 channel's step spent two thirds of its time in the solve's 38
 // launches and five host round trips.  Here P workgroups of RBLK threads stay
-// for the solve: each runs the row kernels' bodies for its share of their
-// workgroups (the same tiles, the same partial sums), a barrier between the
+// for the solve, one for each of the row kernels' workgroups that has a tile: it
+// runs their bodies (the same tile, the same partial sums), a barrier between the
 // passes replaces the launch, and every workgroup finalizes each reduction by
 // itself on its own copy of the component records, so all take the same
 // branches without asking the host.  The fields are the bits the launches give.
@@ -1335,7 +1335,7 @@ __global__ void __launch_bounds__(FBLK) k_fin_mean6(int32_t N, int G, const doub
 // leaves, which the others see in their own waits.  The records on the device
 // and the saved vectors then still hold the solve's start, and the host runs it
 // by launches.
-constexpr int RBLK = 256, RSUB = RBLK / BLK;
+constexpr int RBLK = BLK;
 constexpr int XCDS = RES_XCDS;
 // workgroups a CU holds: FP32 solves are held to 256 registers a lane for two,
 // FP64 ones take up to 350 (held to 256 they spill, and a 128 x 128 channel's
@@ -1346,8 +1346,9 @@ constexpr int RES_PER_CU = sizeof(T) == 4 ? 2 : 1;
 template <class T>
 struct ResArgs {
     KryArgs<T> a, b, s;   // all rows; red-black: the second colour's rows, its sweep residual
-    int32_t P, pg, Gw;    // workgroups; row-kernel workgroups of the pointwise and first-colour passes
-    int32_t X;            // row-kernel workgroups with a tile: the first X of a.G
+    // workgroups: the first P of the row kernels' a.G, those that have a tile;
+    // row-kernel workgroups of the pointwise and first-colour passes
+    int32_t P, pg, Gw;
     int32_t doScale;
     uint32_t maxPolls, epoch;  // epoch: this launch, what resDone or resFail is set to
     SolveState* st;
@@ -1524,9 +1525,9 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     constexpr bool MIX = std::is_same<T, float>::value;
     __shared__ CompState cs[6];
     __shared__ double lds[FIN_LDS];
-    __shared__ double red[RSUB][RED_MAX * (BLK / 64)];
+    __shared__ double red[RED_MAX * (BLK / 64)];
     __shared__ int bad;
-    const int sub = threadIdx.x / BLK, tid = threadIdx.x % BLK, P = m.P;
+    const int P = m.P, tid = threadIdx.x;
     for (int i = threadIdx.x; i < (int)(sizeof(cs) / 8); i += RBLK)
         reinterpret_cast<double*>(cs)[i] = reinterpret_cast<const double*>(m.a.cs)[i];
     __syncthreads();
@@ -1546,19 +1547,13 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     sw.partials = a.partials = slot(RES_SWEEP_SLOT);
     // the finalizers sum the workgroups that have a tile: the others add zeros
     KryArgs<T> fv = av, ft = at, fx = ax, fs = a;
-    fv.G = ft.G = fx.G = fs.G = m.X;
+    fv.G = ft.G = fx.G = fs.G = P;
     ResBar bar{m.st->bar, m.st->barL2, P, 1, P, nullptr, m.maxPolls, 0, (uint32_t)(m.P > 0)};
     auto wait = [&] { return res_barrier(bar, &bad); };
-    // one pass of the row kernels: workgroups 0 .. X-1 of G, RSUB at a time
-    auto passOf = [&](int X, int G, auto&& body) {
-        for (int v0 = p * RSUB; v0 < X; v0 += P * RSUB) {
-            body(Blk{v0 + sub < X ? G : 0, v0 + sub, tid, red[sub]});
-            if (X > P * RSUB) __syncthreads();  // the partial-sum slots are used again
-        }
+    // workgroup p of a pass of G row-kernel workgroups
+    auto pass = [&](int G, auto&& body) {
+        if (p < G) body(Blk{G, p, tid, red});
     };
-    auto pass = [&](int G, auto&& body) { passOf(min(G, m.X), G, body); };
-    auto passAll = [&](int G, auto&& body) { passOf(G, G, body); };
-    const int X0 = P * RSUB;
     if (m.xSave) {
         const int64_t n6 = (int64_t)NCMP * a.N;
         for (int64_t i = (int64_t)p * RBLK + threadIdx.x; i < n6; i += (int64_t)P * RBLK) {
@@ -1580,13 +1575,13 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
                     }
                 }
         } else {
-            passAll(X0, [&](const Blk& k) { k_scale_body<T>(a, k); });
+            pass(P, [&](const Blk& k) { k_scale_body<T>(a, k); });
         }
     }
     bool ok = res_enter(bar, &bad);
-    // the kept rows: tile p RSUB + sub of the rows (red-black: of each colour)
+    // the kept rows: tile p of the rows (red-black: of each colour)
     constexpr bool ROW = FORM == RF_RB_ROW || FORM == RF_BICG_ROW;
-    const Blk kRow{p * RSUB + sub < m.X ? a.G : 0, p * RSUB + sub, tid, red[sub]};
+    const Blk kRow{a.G, p, tid, red};
     int32_t rR = -1, rB = -1;
     RowEnts<T> eR, eB;  // red-black: the first and the second colour's row; PBiCG: A^T's and A's
     T w0[6], wr[6], wp[6], wv[6], dgB = (T)1;
@@ -1595,7 +1590,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
     double rdB = 1.0;
     uint32_t oR = 0, oB = 0;
     if constexpr (ROW) {
-        const int64_t i = (int64_t)(p * RSUB + sub) * BLK + tid;
+        const int64_t i = (int64_t)p * BLK + tid;
         if constexpr (RB) {
             const int64_t rb = (a.nRed & ~(SLICE - 1)) + i;
             if (i < a.nRed) rR = (int32_t)i;
@@ -1628,7 +1623,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
         if (!act && !ref) break;
         if (!act) {
             if (fold) {
-                passAll(m.pg, [&](const Blk& k) { k_fold_body<T>(RB ? b : a, k); });
+                pass(m.pg, [&](const Blk& k) { k_fold_body<T>(RB ? b : a, k); });
                 ok = wait();
             }
             if constexpr (RB) {
@@ -1842,7 +1837,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
             k_fin_bicg_xr_body<T, RBLK>(fx, lds);
             __syncthreads();
         } else if constexpr (BICG) {
-            passAll(m.pg, [&](const Blk& k) { k_bicg_p_body<T>(a, k); });
+            pass(m.pg, [&](const Blk& k) { k_bicg_p_body<T>(a, k); });
             ok = wait();
             if (!ok) break;
             pass(a.G, [&](const Blk& k) { k_bicg_w_body<T>(av, k); });
@@ -1857,7 +1852,7 @@ __device__ __forceinline__ void solve_resident(const ResArgs<T>& m, int p) {
             __syncthreads();
         } else {
             if (round_of(a).inner > 0) {
-                passAll(m.pg, [&](const Blk& k) { k_kry_p_body<T>(RB ? b : a, k); });
+                pass(m.pg, [&](const Blk& k) { k_kry_p_body<T>(RB ? b : a, k); });
                 ok = wait();
                 if (!ok) break;
             }
@@ -2049,7 +2044,7 @@ struct SolveRun {
     int rounds = 0;
     // the whole solve in one launch of P workgroups (k_solve_one / k_solve_group)
     bool resident = false, resLaunched = false;
-    int P = 1, X = 1, form = 0;
+    int P = 1, form = 0;
     uint32_t maxPolls = 0, epoch = 0;
     DBuf xSave;  // the start of a resident solve of several workgroups (ResArgs::xSave)
     SolveState* st = nullptr;
@@ -2472,20 +2467,23 @@ void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     Krylov& K = *sa.kry;
     R.resident = R.resLaunched = false;
     if (sa.ctl->residentPolls == 0 || ctx->profiling || K.N > RES_MAX_ROWS || ctx->device >= RES_DEVICES) return;
-    if (R.G % 8 == 0 || K.partials.bytes < (size_t)RES_SUMS * K.grid * sizeof(double)) return;
+    if (R.G % 8 == 0 || R.Gw % 8 == 0 || K.partials.bytes < (size_t)RES_SUMS * K.grid * sizeof(double)) return;
     const Mesh& m = *sa.mesh;
-    // row-kernel workgroups with a tile (their tiles in order: G is no multiple of 8)
+    // row-kernel workgroups with a tile: the first ones (tile t is workgroup t's where
+    // the grid is no multiple of 8)
     const int32_t row0 = R.rb ? m.nRed & ~(SLICE - 1) : 0;
-    R.X = std::max((int)kblk(m.N - row0), R.rb ? (int)kblk(m.nRed) : 1);
-    if (R.X > R.G) return;
-    R.P = (R.X + RSUB - 1) / RSUB;
+    R.P = std::max((int)kblk(m.N - row0), R.rb ? (int)kblk(m.nRed) : 1);
+    if (R.P > R.G) return;
     const bool row = m.maxWidth <= ROW_W;
     R.form = R.bicg ? (row ? RF_BICG_ROW : RF_BICG) : R.rb ? (row ? RF_RB_ROW : RF_REDBLACK) : RF_JACOBI;
     if (R.P > ctx->numCUs / 2) return;
-    // Measured (us a step, by launches / resident): rows kept, red-black FP64 233 /
-    // 146 at 4096 cells, 285 / 207 at 16384, 356 / 299 at 65536, PBiCG 511 / 326
-    // at 16384; the passes over memory of the other forms 338 / 266 at 16384,
-    // 385 / 349 at 36864, 466 / 475 at 65536
+    // Half the CUs at a row a thread (red-black: one of each colour): 65536 rows
+    // red-black, 32768 in the other forms.  Measured (us a step, by launches /
+    // resident): rows kept, red-black FP64 233 / 146 at 4096 cells, 285 / 207 at
+    // 16384, 356 / 299 at 65536, PBiCG 511 / 326 at 16384; the passes over memory of
+    // Jacobi 338 / 266 at 16384 and, with no limit on the CUs, 385 / 349 at 36864 and
+    // 466 / 475 at 65536.  (Red-black rows wider than six take the passes over memory
+    // too.)
     if (R.form < RF_RB_ROW && m.N > RES_MAX_ROWS / 2) return;
     if (R.P > 1 && K.noAlloc && !K.xSave.p) return;
     if (!resident_fits<T>(R.form) || (R.P > 1 && ctx->backoff->skip())) return;
@@ -2503,7 +2501,6 @@ ResArgs<T> resident_args(SolveRun& R) {
     m.P = R.P;
     m.pg = point_grid(R);
     m.Gw = R.Gw;
-    m.X = R.X;
     m.doScale = R.needScale ? 1 : 0;
     m.maxPolls = R.maxPolls;
     m.epoch = R.epoch = ++R.ctx->resEpoch;

@@ -62,8 +62,8 @@ __device__ __forceinline__ int64_t tile_of(int64_t i, int64_t N, int64_t nRed = 
 
 // A row kernel's workgroup: index b of G workgroups of BLK threads, this
 // thread's index in it, and its LDS slots for partial sums ([RED_MAX][BLK/64]).
-// Bodies take it as an argument so that a launch of several solves, or a
-// workgroup made of several of these, runs them with the same arithmetic.
+// Bodies take it as an argument so that a launch of several solves, and a
+// resident solve, run them with the same arithmetic.
 constexpr int RED_MAX = 19;
 struct Blk {
     int G, b, tid;
@@ -138,7 +138,7 @@ __device__ __forceinline__ void write_partials(const double (&v)[NQ], double* pa
     const double s = wave_scatter<NQ, 32>(v, k.tid & 63, lo, n);
     if (n > 0) k.red[lo * W + (k.tid >> 6)] = s;
     __syncthreads();
-    if (k.tid < NQ && k.b < k.G) {
+    if (k.tid < NQ) {
         double t = 0;
         for (int w = 0; w < W; ++w) t += k.red[k.tid * W + w];
         partials[(int64_t)k.b * NQ + k.tid] = t;
