@@ -219,7 +219,7 @@ __device__ __forceinline__ void k_residual_body(const KryArgs<T>& a, const Blk& 
     // (the first colour's residual is zero once it has been eliminated)
     const int32_t rowB = a.rowBegin & ~(SLICE - 1);  // wavefronts on whole slices
     const int64_t nRows = (int64_t)a.N - rowB;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = a.rowBegin > 0 ? tile_of_g(it, nRows, 0, k_.G, k_.b) : tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -335,7 +335,7 @@ __device__ __forceinline__ void k_kry_p_body(const KryArgs<T>& a, const Blk& k_)
     }
     const T* pOld = q.inner == 1 ? a.r0 : a.p;
     const int64_t N = a.N;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < N; i += (int64_t)k_.G * BLK) {
         T rr[6], pp[6], vv[6];
         ld6(a.r + NCMP * i, rr);
         ld6(pOld + NCMP * i, pp);
@@ -359,7 +359,7 @@ __device__ __forceinline__ void k_kry_v_body(const KryArgs<T>& a, const Blk& k_)
     if (!rd.any) return;
     const T* pv = rd.inner == 0 ? a.r0 : a.p;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -429,7 +429,7 @@ __device__ __forceinline__ void k_kry_t_body(const KryArgs<T>& a, const Blk& k_)
     T q[18];
 #pragma unroll
     for (int i = 0; i < 18; ++i) q[i] = 0;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -525,7 +525,7 @@ __device__ __forceinline__ void k_kry_xr_body(const KryArgs<T>& a, const Blk& k_
     for (int i = 0; i < 12; ++i) q[i] = 0;
     // red-black: the second colour's rows, as the v and t passes take them
     const int32_t first = a.ctl.rb ? a.nRed : 0, row0 = first & ~(SLICE - 1);
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, (int64_t)a.N - row0, a.ctl.rb ? 0 : a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -610,7 +610,7 @@ __device__ __forceinline__ void k_fold_body(const KryArgs<T>& a, const Blk& k_) 
         any |= on[c];
     }
     if (!any || inner_running(a)) return;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < a.N; i += (int64_t)k_.G * BLK) {
         double xv[6];
         T ev[6];
         ld6(a.x + NCMP * i, xv);
@@ -722,7 +722,7 @@ __device__ __forceinline__ void k_rb_w_body(const KryArgs<T>& a, const Blk& k_) 
 #pragma unroll
     for (int c = 0; c < 6; ++c) alpha[c] = (T)uni(a.cs[c].alpha);
     const int64_t n = a.nRed;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -755,7 +755,7 @@ __device__ __forceinline__ void k_rb_v_body(const KryArgs<T>& a, const Blk& k_) 
     T q[6] = {0, 0, 0, 0, 0, 0};
     const int32_t r0b = a.nRed & ~(SLICE - 1);  // wavefronts on whole slices
     const int64_t n = (int64_t)a.N - r0b;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -805,7 +805,7 @@ __device__ __forceinline__ void k_rb_t_body(const KryArgs<T>& a, const Blk& k_) 
     for (int i = 0; i < 18; ++i) q[i] = 0;
     const int32_t r0b = a.nRed & ~(SLICE - 1);  // wavefronts on whole slices
     const int64_t n = (int64_t)a.N - r0b;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -857,7 +857,7 @@ __device__ __forceinline__ void k_rb_backsub_body(const KryArgs<T>& a, const Blk
     }
     if (!any || inner_running(a)) return;
     const int64_t n = a.nRed;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, n, 0, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -934,7 +934,7 @@ __device__ __forceinline__ void k_bicg_init_body(const KryArgs<T>& a, const Blk&
     }
     if (!any) return;
     double q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1008,7 +1008,7 @@ __device__ __forceinline__ void k_bicg_p_body(const KryArgs<T>& a, const Blk& k_
         any |= on[c];
     }
     if (!any) return;
-    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; i < a.N; i += (int64_t)k_.G * BLK) {
+    for (int64_t i = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && i < a.N; i += (int64_t)k_.G * BLK) {
         const T rm = a.rM ? (T)a.rM[i] : (T)1;
         T rA[6], rT[6], pA[6], pT[6];
         ld6(a.r + NCMP * i, rA);
@@ -1044,7 +1044,7 @@ __device__ __forceinline__ void k_bicg_w_body(const KryArgs<T>& a, const Blk& k_
     }
     if (!any) return;
     T q[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1134,7 +1134,7 @@ __device__ __forceinline__ void k_bicg_xr_body(const KryArgs<T>& a, const Blk& k
     T q[12];
 #pragma unroll
     for (int i = 0; i < 12; ++i) q[i] = 0;
-    for (int64_t it = 0;; ++it) {
+    for (int64_t it = 0; k_.b < k_.G; ++it) {
         const int64_t tl = tile_of_g(it, a.N, a.nRed, k_.G, k_.b);
         if (tl < 0) {
             if (tl == -1) break;
@@ -1256,7 +1256,7 @@ __global__ void k_rdiag(int32_t N, const double* __restrict__ diag, double* __re
 template <class T>
 __device__ __forceinline__ void k_scale_body(const KryArgs<T>& a, const Blk& k_) {
     T* ahat = const_cast<T*>(a.ahat);
-    for (int64_t r = (int64_t)k_.b * BLK + k_.tid; r < a.N; r += (int64_t)k_.G * BLK) {
+    for (int64_t r = (int64_t)k_.b * BLK + k_.tid; k_.b < k_.G && r < a.N; r += (int64_t)k_.G * BLK) {
         const int s = (int)(r >> 6), lane = (int)(r & 63);
         const int64_t base = a.ellOff[s] + lane;
         const int w = a.ellWidth[s];
