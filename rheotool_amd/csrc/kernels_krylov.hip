@@ -1329,10 +1329,10 @@ __global__ void __launch_bounds__(FBLK) k_fin_mean6(int32_t N, int G, const doub
 // one row a thread is bound by instruction issue and latency (512 threads took
 // 2.6 us for the x/r pass, 256 take 1.2 us).
 //
-// The barrier needs the workgroups resident together: no more are launched than
-// fit, but other streams and processes may hold the CUs, so the wait is bounded:
-// a workgroup that polls maxPolls times sets the top bit of the counters and
-// leaves, which the others see in their own waits.  The records on the device
+// The barrier needs the workgroups resident together: the launches take their CUs
+// from a budget (ResBudget), but other processes may hold them, so the wait is
+// bounded: a workgroup that polls maxPolls times marks the counter and leaves,
+// which the others see in their own waits.  The records on the device
 // and the saved vectors then still hold the solve's start, and the host runs it
 // by launches.
 constexpr int RBLK = BLK;
@@ -2481,7 +2481,7 @@ void choose_resident(Ctx* ctx, const SolveArgs& sa, SolveRun& R) {
     // red-black, 32768 in the other forms.  Measured (us a step, by launches /
     // resident): rows kept, red-black FP64 233 / 146 at 4096 cells, 285 / 207 at
     // 16384, 356 / 299 at 65536, PBiCG 511 / 326 at 16384; the passes over memory of
-    // Jacobi 338 / 266 at 16384 and, with no limit on the CUs, 385 / 349 at 36864 and
+    // Jacobi 338 / 266 at 16384 and, before the limit on the CUs, 385 / 349 at 36864 and
     // 466 / 475 at 65536.  (Red-black rows wider than six take the passes over memory
     // too.)
     if (R.form < RF_RB_ROW && m.N > RES_MAX_ROWS / 2) return;
