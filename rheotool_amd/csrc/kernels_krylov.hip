@@ -2538,7 +2538,7 @@ bool launch_resident(Ctx* ctx, Krylov& K, SolveRun& R) {
     int xcd = ctx->xcd;
     if (!take_save(K, R)) return false;
     if (R.P > 1) {
-        xcd = resBudgets[ctx->device].take(R.P, HALF_CUS / RES_PER_CU<T>, half_cus(ctx), ctx->xcd, R.hold);
+        xcd = resBudgets[ctx->device].take(R.P, HALF_CUS / RES_PER_CU<T>, half_cus(ctx), ctx->xcd, ctx->lane, R.hold);
         if (xcd == RES_FULL) return false;
     }
     const ResArgs<T> m = resident_args<T>(R);
@@ -2906,7 +2906,7 @@ void group_launch_resident(SolveGroup& g, std::vector<SolveGroup::Member>& evict
         if (!take_save(*g.members[i].K, *g.members[i].K->run)) group_evict(g, i, evicted);
     for (const auto& mb : g.members) ms.push_back({mb.K->run->P, mb.K->run->form});
     const std::vector<ResLaunch> launches =
-        resBudgets[g.ctx->device].group(ms, HALF_CUS / RES_PER_CU<T>, half_cus(g.ctx), g.hold, left);
+        resBudgets[g.ctx->device].group(ms, HALF_CUS / RES_PER_CU<T>, half_cus(g.ctx), g.ctx->lane, g.hold, left);
     std::vector<SolveGroup::Member> all = g.members;  // the launches' maps index these
     for (size_t k = left.size(); k-- > 0;) group_evict(g, left[k], evicted);
     if (g.members.empty()) return;

@@ -73,6 +73,7 @@ struct Ctx {
     int64_t solveCounts[3] = {0, 0, 0};  // finished resident, gave up, finished by launches
     int xcd = 0;  // where its resident solves look for room first: contexts take turns,
                   // and move on after a wait gave up
+    std::shared_ptr<ResLane> lane = std::make_shared<ResLane>();  // its stream's resident launches
     ResBackoff ownBackoff, *backoff = &ownBackoff;  // a server's slots share one
     hipStream_t stream = nullptr;
     size_t budget = 0, inUse = 0;

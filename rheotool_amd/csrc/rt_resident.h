@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <array>
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -146,9 +147,18 @@ RES_FN void res_depart(const ResBar& B) {
 // FP32 workgroups can share every CU that no FP64 one is on, and once they end,
 // which they do, the FP64 ones have a CU each.  Other kernels end by themselves.
 // Another process's launches are not counted: there the bounded wait remains.
+// Launches of one stream run one after another, so a stream (ResLane) takes the
+// most that any of its launches under way holds.
 class ResBudget;
+struct ResHold;
+struct ResLane {
+    int n[RES_XCDS] = {0};    // the most of its holds
+    ResHold* first = nullptr;  // its holds
+};
 struct ResHold {  // what a launch holds, given back once it has ended
     ResBudget* from = nullptr;
+    std::shared_ptr<ResLane> lane;
+    ResHold* next = nullptr;
     int n[RES_XCDS] = {0};
     ResHold() = default;
     ResHold(const ResHold&) = delete;
@@ -171,30 +181,45 @@ constexpr int RES_SPREAD = -1, RES_FULL = -2;
 
 class ResBudget {
     std::mutex mu;
-    int held[RES_XCDS] = {0};
+    int held[RES_XCDS] = {0};  // of all lanes
     static int share(int P, int x) { return (P - x + RES_XCDS - 1) / RES_XCDS; }  // of P dealt over all XCDs
+    int others(const ResLane& l, int x) const { return held[x] - l.n[x]; }
+    void settle(ResLane& l) {
+        for (int x = 0; x < RES_XCDS; ++x) {
+            int most = 0;
+            for (const ResHold* h = l.first; h; h = h->next) most = std::max(most, h->n[x]);
+            held[x] += most - l.n[x];
+            l.n[x] = most;
+        }
+    }
+    void give(const std::shared_ptr<ResLane>& l, ResHold& h) {
+        h.from = this;
+        h.lane = l;
+        h.next = l->first;
+        l->first = &h;
+        settle(*l);
+    }
 
    public:
     // A launch of P workgroups of `unit` half CUs each; cap: half CUs of an XCD.
     // The XCD (of those with room the one with most, from `first` on) that takes
     // them all, RES_SPREAD: dealt over all, or RES_FULL
-    int take(int P, int unit, int cap, int first, ResHold& h) {
+    int take(int P, int unit, int cap, int first, const std::shared_ptr<ResLane>& lane, ResHold& h) {
         std::lock_guard<std::mutex> lk(mu);
         int best = RES_FULL;
         for (int i = 0; i < RES_XCDS; ++i) {
             const int x = (first + i) % RES_XCDS;
-            if (held[x] + P * unit <= cap && (best < 0 || held[x] < held[best])) best = x;
+            if (others(*lane, x) + P * unit <= cap && (best < 0 || others(*lane, x) < others(*lane, best))) best = x;
         }
         if (best >= 0) {
             h.n[best] = P * unit;
         } else {
             for (int x = 0; x < RES_XCDS; ++x)
-                if (held[x] + share(P, x) * unit > cap) return RES_FULL;
+                if (others(*lane, x) + share(P, x) * unit > cap) return RES_FULL;
             for (int x = 0; x < RES_XCDS; ++x) h.n[x] = share(P, x) * unit;
             best = RES_SPREAD;
         }
-        for (int x = 0; x < RES_XCDS; ++x) held[x] += h.n[x];
-        h.from = this;
+        give(lane, h);
         return best;
     }
     // The launches, one after another on a stream, of a group of solves: a member
@@ -202,10 +227,11 @@ class ResBudget {
     // of them (the largest members first would pack tighter; a queue's order keeps
     // its latency).  Holds the most any launch places on an XCD; left: the members
     // no launch can take beside what others hold.
-    std::vector<ResLaunch> group(const std::vector<ResMember>& ms, int unit, int cap, ResHold& h, std::vector<int>& left) {
+    std::vector<ResLaunch> group(const std::vector<ResMember>& ms, int unit, int cap,
+                                 const std::shared_ptr<ResLane>& lane, ResHold& h, std::vector<int>& left) {
         std::lock_guard<std::mutex> lk(mu);
         int room[RES_XCDS];  // workgroups
-        for (int x = 0; x < RES_XCDS; ++x) room[x] = std::max(0, cap - held[x]) / unit;
+        for (int x = 0; x < RES_XCDS; ++x) room[x] = std::max(0, cap - others(*lane, x)) / unit;
         std::vector<ResLaunch> out;
         const ResLaunch none;
         auto freest = [&](const ResLaunch& L) {
@@ -243,14 +269,16 @@ class ResBudget {
         for (int x = 0; x < RES_XCDS; ++x) {
             h.n[x] = 0;
             for (const ResLaunch& L : out) h.n[x] = std::max(h.n[x], L.load[x] * unit);
-            held[x] += h.n[x];
         }
-        h.from = this;
+        give(lane, h);
         return out;
     }
-    void giveBack(const int (&n)[RES_XCDS]) {
+    void takeBack(ResHold& h) {
         std::lock_guard<std::mutex> lk(mu);
-        for (int x = 0; x < RES_XCDS; ++x) held[x] -= n[x];
+        ResHold** p = &h.lane->first;
+        while (*p != &h) p = &(*p)->next;
+        *p = h.next;
+        settle(*h.lane);
     }
 };
 // A wait that gave up cost the time of all its polls (about 0.1 s) and a step by
@@ -273,8 +301,10 @@ struct ResBackoff {
 
 inline void ResHold::release() {
     if (!from) return;
-    from->giveBack(n);
+    from->takeBack(*this);
     from = nullptr;
+    lane.reset();
+    next = nullptr;
     for (int& v : n) v = 0;
 }
 

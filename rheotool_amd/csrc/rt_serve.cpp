@@ -278,7 +278,10 @@ void rt_server_destroy(rt_server* S) {
             releaseRequest(S, kv.second.get());
         }
     for (auto* c : S->slots) rt_ctx_destroy(c);
-    for (auto& g : S->groups) g.tables.release();
+    for (auto& g : S->groups) {
+        g.tables.release();
+        g.hold.release();
+    }
     rt_ctx_destroy(S->gctx);
     Ctx* parent = &S->parent->impl;
     delete S;

@@ -212,16 +212,20 @@ static void budget(uint64_t seed) {
         std::vector<std::array<int, RES_XCDS>> launches;  // one after another
         int placed[RES_XCDS] = {0};
         std::vector<std::pair<int, int>> on;  // (XCD, CU) of its placed workgroups
+        int lane = 0;                         // jobs of a lane run in their order
     };
     ResBudget B;
+    std::vector<std::shared_ptr<ResLane>> lanes(3);
+    for (auto& l : lanes) l.reset(new ResLane);
     std::vector<Job> jobs;
     for (int i = 0; i < 6; ++i) {
         Job j;
         j.hold.reset(new ResHold);
         j.unit = 1 + (int)(rng() % 2);
+        j.lane = (int)(rng() % lanes.size());
         if (rng() % 2) {
             const int P = 2 + (int)(rng() % (RES_XCDS * cus));
-            const int x = B.take(P, j.unit, cap, (int)(rng() % RES_XCDS), *j.hold);
+            const int x = B.take(P, j.unit, cap, (int)(rng() % RES_XCDS), lanes[j.lane], *j.hold);
             if (x == RES_FULL) continue;
             std::array<int, RES_XCDS> n{};
             for (int p = 0; p < P; ++p) ++n[x == RES_SPREAD ? p % RES_XCDS : x];
@@ -231,8 +235,11 @@ static void budget(uint64_t seed) {
             for (int k = 0; k < 1 + (int)(rng() % 9); ++k)
                 ms.push_back({1 + (int)(rng() % (rng() % 3 ? 2 * cus : RES_XCDS * cus)), (int)(rng() % 2)});
             std::vector<int> left;
-            const std::vector<ResLaunch> ls = B.group(ms, j.unit, cap, *j.hold, left);
+            const std::vector<ResLaunch> ls = B.group(ms, j.unit, cap, lanes[j.lane], *j.hold, left);
             std::vector<int> seen(ms.size(), 0), at(ms.size(), -1);
+            bool alone = true;  // no other lane holds anything
+            for (const Job& o : jobs) alone = alone && o.lane == j.lane;
+            CHECK(!alone || left.empty(), "a lane alone on the device leaves a member out");
             for (int i : left) seen[i] = ms[i].P;
             for (size_t l = 0; l < ls.size(); ++l) {
                 std::array<int, RES_XCDS> n{};
@@ -255,7 +262,13 @@ static void budget(uint64_t seed) {
     }
     for (int x = 0; x < RES_XCDS; ++x) {
         int sum = 0;
-        for (const Job& j : jobs) sum += j.hold->n[x];
+        for (int l = 0; l < (int)lanes.size(); ++l) {
+            int most = 0;
+            for (const Job& j : jobs)
+                if (j.lane == l) most = std::max(most, j.hold->n[x]);
+            CHECK(lanes[l]->n[x] == most, "lane %d takes %d, its launches %d", l, lanes[l]->n[x], most);
+            sum += most;
+        }
         CHECK(sum <= cap, "XCD %d: %d of %d half CUs promised", x, sum, cap);
     }
     // placement: used[x][c] half CUs; a launch ends once all its workgroups are placed
@@ -264,6 +277,9 @@ static void budget(uint64_t seed) {
         std::vector<std::array<int, 3>> moves;  // job, XCD, CU
         for (int k = 0; k < (int)jobs.size(); ++k) {
             Job& j = jobs[k];
+            bool waits = false;  // for an earlier launch of its stream
+            for (int e = 0; e < k; ++e) waits = waits || jobs[e].lane == j.lane;
+            if (waits) continue;
             if (j.launches.empty()) {
                 moves.push_back({k, -1, -1});
                 continue;
@@ -296,7 +312,7 @@ static void budget(uint64_t seed) {
         }
     }
     ResHold h;
-    CHECK(B.take(RES_XCDS * cus, 2, cap, 3, h) == RES_SPREAD, "not everything was given back");
+    CHECK(B.take(RES_XCDS * cus, 2, cap, 3, lanes[0], h) == RES_SPREAD, "not everything was given back");
 }
 
 int main() {

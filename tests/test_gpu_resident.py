@@ -260,3 +260,25 @@ def test_a_servers_budget_admits_what_it_admitted_without_resident_solves():
             assert srv.solve_counts == counts
             srv.close()
         assert all(np.array_equal(a, out[0]) for a in out)
+
+
+def test_a_servers_groups_share_their_streams_cus():
+    """The forms of a burst run in groups of their own, one after another on the
+    server's stream: none is kept from running resident by another."""
+    with abi.Context(0) as ctx:
+        ms = [cases.cartesian(n, n, 1, twoD=True, channel=True) for n in (170, 120, 150, 60)]
+        dms = [ctx.mesh(m) for m in ms]
+        fs = [cases.make_fields(m, cases.FIELDS_CHANNEL, seed=4) for m in ms]
+        text = abi.model_dict("Oldroyd-BLog")
+        controls = [abi.solver_dict(1e-10, precision=p, precond=c) for p in ("mixed", "double") for c in ("DILU", "diagonal")]
+        print("[case] server, four forms", flush=True)
+        out = {}
+        for polls in ("", " residentPolls 0;"):
+            srv = abi.Server(ctx, max_inflight=16)
+            ts = [srv.submit(dm, f, text, 1e-3, c + polls) for c in controls for dm, f in zip(dms, fs)]
+            while srv.progress():
+                pass
+            out[polls] = [srv.poll(t)["theta"] for t in ts]
+            assert srv.solve_counts == ((16, 0, 0) if not polls else (0, 0, 16))
+            srv.close()
+        assert all(np.array_equal(a, b) for a, b in zip(*out.values()))
