@@ -281,6 +281,7 @@ class ResBudget {
         settle(*h.lane);
     }
 };
+
 // A wait that gave up cost the time of all its polls (about 0.1 s) and a step by
 // launches.  What kept the workgroups apart, another process's work, is likely to
 // be there at the next step too, so the context's next solves run by launches: 64
